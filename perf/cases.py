@@ -80,7 +80,7 @@ def draw(rng):
     if kind == "prologue":
         H = rng.choice([1, 2, 4, 6, 8, 10, 12])
         return dict(kind=kind, dtype=rng.choices(["bf16", "fp32"], [3, 1])[0], B=_log(rng, 1, 16), T=_log(rng, 4, 2048), H=H,
-                    Hkv=H // rng.choice([r for r in (1, 2) if H % r == 0]), D=rng.choice([16, 32, 64, 64, 96, 128, 128]),
+                    Hkv=H // rng.choice([r for r in (1, 2) if H % r == 0]), D=rng.choice([16, 32, 64, 64, 128, 128]),
                     positions=rng.choice(["none", "packed"]))
     if kind == "loss":
         V = rng.choice([8192, 32768, _log(rng, 50, 50257), 50257, 50304])
