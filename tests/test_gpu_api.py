@@ -155,6 +155,35 @@ def test_autograd_matches_explicit_backward(gpu):
         assert torch.equal(x.grad, g)
 
 
+@pytest.mark.parametrize("mode,dtypes,D", [
+    ("fast", (torch.bfloat16, torch.bfloat16, torch.bfloat16), 128),
+    ("fast", (torch.bfloat16, torch.bfloat16, torch.bfloat16), 80),
+    ("fast", (torch.bfloat16, torch.float32, torch.bfloat16), 64),
+    ("fast", (torch.float16, torch.float16, torch.float16), 64),
+    ("exact", (torch.bfloat16, torch.bfloat16, torch.bfloat16), 64),
+])
+def test_autograd_gradient_dtypes(gpu, mode, dtypes, D):
+    """The gradients in each leaf's dtype equal the float32 gradients of an
+    explicit backward into zeroed buffers, rounded once, bit for bit; rows and
+    keys that see nothing (a window left of every key) get zeros."""
+    B, T, H, Hkv, window = 2, 200, 4, 2, (40, -3)
+    A = MFMAFast() if mode == "fast" else MFMAExact()
+    Q, K, V, dO = _inputs(5 + D, B, T, H, Hkv, D)
+    leaves = [torch.from_numpy(x).to(gpu).to(dt).requires_grad_(True) for x, dt in zip((Q, K, V), dtypes)]
+    junk = torch.full((64 << 20,), float("nan"), device=gpu)  # what the freed blocks of the next allocations hold
+    del junk
+    O = Kn.AttentionFunction.apply(*leaves, window, A, None)
+    dOd = torch.from_numpy(dO).to(gpu).to(O.dtype)
+    grads = torch.autograd.grad(O, leaves, dOd)
+    st = Kn.attention_state(A, *(x.detach() for x in leaves), window)
+    ref = [torch.zeros(x.shape, dtype=torch.float32, device=gpu) for x in (st.Q, st.K, st.V)]
+    Kn.delta_attention_(A, *ref, dOd, st.Q, st.K, st.V, st.O, st.l, st.m, window)
+    torch.cuda.synchronize()
+    for g, r, dt in zip(grads, ref, dtypes):
+        assert g.dtype == dt and torch.equal(g, r.to(dt))
+    assert not grads[0][:, :3].any() and not grads[1][:, T - 3:].any() and not grads[2][:, T - 3:].any()
+
+
 def test_attention_fp16_inputs(gpu):
     """float16 inputs select the matrix-core path as in the reference
     (ext/FemtoChatCUDAExt.jl:214-223); this library's matrix-core format is
