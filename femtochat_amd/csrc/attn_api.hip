@@ -585,25 +585,37 @@ fc_status fc_cross_entropy_count(const fc_xent_desc* desc, const void* targets, 
   return ok();
 }
 
-fc_status fc_cross_entropy_bwd(const fc_xent_desc* desc, float* dlogits, const float* logits, const void* targets,
-                               const float* dy, const float* count, const float* lse, void* stream) {
+// The two gradient entry points; full: every column written, zeros for ignored targets.
+static fc_status xent_bwd(const char* who, bool full, const fc_xent_desc* desc, float* dlogits, const float* logits,
+                          const void* targets, const float* dy, const float* count, const float* lse, void* stream) {
   fc::XentArgs a;
-  const fc_status st = xent_args(desc, targets, "fc_cross_entropy_bwd", &a);
+  const fc_status st = xent_args(desc, targets, who, &a);
   if (st != FC_OK) return st;
   if (dlogits == nullptr || logits == nullptr || dy == nullptr)
-    return fail(FC_ERR_INVALID_ARGUMENT, "fc_cross_entropy_bwd: dlogits, logits and dy are required");
+    return fail(FC_ERR_INVALID_ARGUMENT, "%s: dlogits, logits and dy are required", who);
   if (desc->reduction == FC_REDUCE_MEAN && count == nullptr)
-    return fail(FC_ERR_INVALID_ARGUMENT, "fc_cross_entropy_bwd: the mean gradient needs the valid-target count");
+    return fail(FC_ERR_INVALID_ARGUMENT, "%s: the mean gradient needs the valid-target count", who);
   if (!aligned4(dlogits) || !aligned4(logits) || !aligned4(dy) || !aligned4(count) || !aligned4(lse))
-    return fail(FC_ERR_INVALID_ARGUMENT, "fc_cross_entropy_bwd: float buffers must be 4-byte aligned");
+    return fail(FC_ERR_INVALID_ARGUMENT, "%s: float buffers must be 4-byte aligned", who);
   a.dlogits = dlogits;
   a.logits = logits;
   a.dy = dy;
   a.count = const_cast<float*>(count);
   a.lse_in = lse;
+  if (full) a.overwrite = a.zero_ignored = 1;
   const hipError_t e = fc::launch_xent_bwd(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(FC_ERR_HIP, "cross-entropy gradient launch failed: %s", hipGetErrorString(e));
   return ok();
+}
+
+fc_status fc_cross_entropy_bwd(const fc_xent_desc* desc, float* dlogits, const float* logits, const void* targets,
+                               const float* dy, const float* count, const float* lse, void* stream) {
+  return xent_bwd("fc_cross_entropy_bwd", false, desc, dlogits, logits, targets, dy, count, lse, stream);
+}
+
+fc_status fc_cross_entropy_bwd_full(const fc_xent_desc* desc, float* dlogits, const float* logits, const void* targets,
+                                    const float* dy, const float* count, const float* lse, void* stream) {
+  return xent_bwd("fc_cross_entropy_bwd_full", true, desc, dlogits, logits, targets, dy, count, lse, stream);
 }
 
 fc_status fc_cross_entropy_fused(const fc_xent_desc* desc, const float* logits, const void* targets, float* losses,

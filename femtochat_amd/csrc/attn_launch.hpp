@@ -102,6 +102,7 @@ inline FastDiv fast_div(uint32_t d) {
   while ((uint64_t(1) << l) < d) ++l;
   return FastDiv{uint32_t((((uint64_t(1) << l) - d) << 32) / d + 1), l};
 }
+__device__ inline uint32_t divide(uint32_t n, FastDiv f) { return (__umulhi(n, f.m) + n) >> f.l; }
 
 struct RopeNormArgs {
   const void* X;
@@ -139,6 +140,7 @@ struct XentArgs {
   int index_base, index_type;  // index_type 0: int32, 1: int64
   int reduction;               // 0 none, 1 sum, 2 mean
   int overwrite;               // backward writes instead of adding
+  int zero_ignored;            // overwriting backward: zeros into the columns of ignored targets
 };
 hipError_t launch_xent_fwd(const XentArgs& a, hipStream_t s);
 hipError_t launch_xent_count(const XentArgs& a, hipStream_t s);

@@ -16,7 +16,8 @@
 // a single pass keeps a running (max, sum of exp) per thread, eight 16-byte
 // loads in flight per round, combined across the workgroup at the end.  The
 // gradient reuses the forward's log-sum-exp when the caller passes it (one
-// read of the logits instead of two).
+// read of the logits instead of two) and is then elementwise over the whole
+// array.
 #include "attn_launch.hpp"
 #include "attn_device.hpp"
 
@@ -28,6 +29,7 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kFwdBatch = 8;  // 16-byte loads in flight per thread in a forward round (4, 8, 16 within 1%)
+constexpr int kWaveV = 2048; // longest column that the forward gives to one wave
 constexpr int kBwdBatch = 8;  // chunks per backward round (4, 8 measured within 3%)
 
 template <typename I>
@@ -70,56 +72,79 @@ __device__ inline Lse block_combine(Lse v) {
   return r;
 }
 
-// One thread's pass over its part of a column: values j = tid*4 + 1024 k
-// (vectorised) or j = tid + 256 k (scalar).  Each round loads up to eight
-// 16-byte chunks, then folds their maximum into m with one rescale of s.
+// One thread's pass over its part of a column: up to three values in front of
+// the first 16-byte boundary and after the last one go to the first threads,
+// the aligned chunks between them to thread tid, tid + 256, ...  Each round
+// loads up to eight chunks, then folds their maximum into m with one rescale
+// of s.  A column whose vocabulary is not a multiple of 4 starts off a
+// boundary in three rows of four; read value by value it took 3.8 times as
+// long (1024 x 50257: see kFwdBatch's note for the aligned rate).
 // kStream: the column is read only once (the forward), so the loads are
 // nontemporal (25% faster at 8192 x 32768); the gradient, which reads the
 // column again, keeps it in the caches.
-template <bool kVec, bool kStream = false>
-__device__ inline Lse column_pass(const float* col, int V) {
+// kThreads threads (tid) share the column, kBatch chunks each per round.
+template <bool kStream, int kThreads = 256, int kBatch = kFwdBatch>
+__device__ inline Lse column_pass(const float* col, int V, int tid) {
+  const int head = min((int)((16 - (reinterpret_cast<uintptr_t>(col) & 15)) & 15) / 4, V);
+  const int chunks = (V - head) / 4, tail = V - head - 4 * chunks;
+  const float* body = col + head;
   Lse acc{-INFINITY, 0.0f};
-  if (kVec) {
-    const int chunks = V / 4;
-    for (int base = threadIdx.x; base < chunks; base += 256 * kFwdBatch) {
-      f32x4 v[kFwdBatch];
-      float bm = -INFINITY;
+  // x = -inf adds nothing (and must not set a reference of -inf).
+  auto one = [](float x) { return Lse{x, x == -INFINITY ? 0.0f : 1.0f}; };
+  if (tid < head) acc = combine(acc, one(col[tid]));
+  if (tid < tail) acc = combine(acc, one(body[4 * chunks + tid]));
+  for (int base = tid; base < chunks; base += kThreads * kBatch) {
+    f32x4 v[kBatch];
+    float bm = -INFINITY;
 #pragma unroll
-      for (int k = 0; k < kFwdBatch; ++k) {
-        const int c = base + 256 * k;
-        const f32x4* p = reinterpret_cast<const f32x4*>(col + 4 * c);
-        v[k] = c < chunks ? (kStream ? __builtin_nontemporal_load(p) : *p) : f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-      }
-#pragma unroll
-      for (int k = 0; k < kFwdBatch; ++k) bm = fmaxf(bm, fmaxf(fmaxf(v[k][0], v[k][1]), fmaxf(v[k][2], v[k][3])));
-      const float m = fmaxf(acc.m, bm);
-      float s = acc.s == 0.0f ? 0.0f : acc.s * exp2f((acc.m - m) * kLog2e);
-#pragma unroll
-      for (int k = 0; k < kFwdBatch; ++k)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s += exp2f((v[k][i] - m) * kLog2e);  // exp2(-inf) = 0 for padding
-      acc = Lse{m, s};
+    for (int k = 0; k < kBatch; ++k) {
+      const int c = base + kThreads * k;
+      const f32x4* p = reinterpret_cast<const f32x4*>(body + 4 * c);
+      v[k] = c < chunks ? (kStream ? __builtin_nontemporal_load(p) : *p) : f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
-  } else {
-    for (int j = threadIdx.x; j < V; j += 256) acc = combine(acc, Lse{col[j], 1.0f});
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) bm = fmaxf(bm, fmaxf(fmaxf(v[k][0], v[k][1]), fmaxf(v[k][2], v[k][3])));
+    const float m = fmaxf(acc.m, bm);
+    const float ref = m == -INFINITY ? 0.0f : m;  // every value so far is -inf: all exponentials are 0
+    float s = acc.s == 0.0f ? 0.0f : acc.s * exp2f((acc.m - ref) * kLog2e);
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s += exp2f((v[k][i] - ref) * kLog2e);  // exp2(-inf) = 0 for padding
+    acc = Lse{m, s};
   }
   return acc;
 }
 
-template <bool kVec>
+__device__ inline void store_loss(const XentArgs& a, int64_t token, const float* col, Lse r) {
+  const float lse = r.m + logf(r.s);
+  const int64_t raw = index_at(a.targets, token, a.index_type);
+  const int64_t t = raw - a.index_base;
+  float loss = 0.0f;
+  if (raw != a.ignore_index) loss = (t >= 0 && t < a.V) ? lse - col[t] : __builtin_nanf("");
+  a.losses[token] = loss;
+  if (a.lse != nullptr) a.lse[token] = lse;
+}
+
 __global__ __launch_bounds__(256) void xent_fwd_kernel(XentArgs a) {
   const int64_t token = blockIdx.x;
   const float* col = a.logits + token * (int64_t)a.V;
-  const Lse r = block_combine(column_pass<kVec, true>(col, a.V));
-  if (threadIdx.x == 0) {
-    const float lse = r.m + logf(r.s);
-    const int64_t raw = index_at(a.targets, token, a.index_type);
-    const int64_t t = raw - a.index_base;
-    float loss = 0.0f;
-    if (raw != a.ignore_index) loss = (t >= 0 && t < a.V) ? lse - col[t] : __builtin_nanf("");
-    a.losses[token] = loss;
-    if (a.lse != nullptr) a.lse[token] = lse;
-  }
+  const Lse r = block_combine(column_pass<true>(col, a.V, threadIdx.x));
+  if (threadIdx.x == 0) store_loss(a, token, col, r);
+}
+
+// Short columns: a wave each, four to a workgroup, no barrier (8192 x 1000: 10
+// us, 28 with a workgroup each; 8192 x 53: 10 and 12).
+template <int kBatch>
+__global__ __launch_bounds__(256) void xent_fwd_wave_kernel(XentArgs a) {
+  const int64_t token = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
+  if (token >= a.N) return;
+  const int lane = threadIdx.x & 63;
+  const float* col = a.logits + token * (int64_t)a.V;
+  Lse r = column_pass<true, 64, kBatch>(col, a.V, lane);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) r = combine(r, Lse{__shfl_xor(r.m, o), __shfl_xor(r.s, o)});
+  if (lane == 0) store_loss(a, token, col, r);
 }
 
 // reduced[0] = sum of losses (or their mean over valid targets), reduced[1] =
@@ -128,9 +153,22 @@ __global__ __launch_bounds__(1024) void xent_reduce_kernel(XentArgs a) {
   __shared__ double part[16];
   __shared__ double cnt[16];
   double s = 0.0, c = 0.0;
-  for (int64_t i = threadIdx.x; i < a.N; i += 1024) {
-    if (a.losses != nullptr) s += (double)a.losses[i];
-    c += index_at(a.targets, i, a.index_type) != a.ignore_index ? 1.0 : 0.0;
+  constexpr int kRun = 8;  // loads in flight per thread
+  for (int64_t base = threadIdx.x; base < a.N; base += 1024 * kRun) {
+    float loss[kRun];
+    int64_t t[kRun];
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) {
+      const int64_t i = min(base + 1024 * k, a.N - 1);
+      loss[k] = a.losses != nullptr ? a.losses[i] : 0.0f;
+      t[k] = index_at(a.targets, i, a.index_type);
+    }
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) {
+      if (base + 1024 * k >= a.N) continue;
+      s += (double)loss[k];
+      c += t[k] != a.ignore_index ? 1.0 : 0.0;
+    }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
@@ -153,24 +191,104 @@ __global__ __launch_bounds__(1024) void xent_reduce_kernel(XentArgs a) {
   }
 }
 
+// The gradient's factor: dy / count(valid) ("mean"), dy ("sum"), dy[token]
+// ("none"); the division is the reference's fp32 `dy ./ sum(valid)`.
+__device__ inline float grad_factor(const XentArgs& a, int64_t token) {
+  const float w = a.dy[a.reduction == 0 ? token : 0];
+  return a.reduction == 2 ? w / *a.count : w;
+}
+
+// Gradient with a given log-sum-exp: nothing is summed over a column, so the
+// (token, vocabulary) array is taken as one run of 16-byte chunks, one per
+// thread in address order, whatever V is; a chunk that crosses into the next
+// token's column (V not a multiple of 4) goes value by value.  All accesses are
+// nontemporal.  HBM-bound: the chip sweeps one window of 4 KB blocks instead
+// of 2048 columns at a time, which took 8192 x 32768 (read and written once)
+// from 472 us (one workgroup per column) to 326, 6.6 TB/s, and from 616 us to
+// 497 added into the gradient.  More chunks per thread
+// were slower: 342, 348 and 360 us with 2, 4 and 8, against 331 with one (the
+// same pass with the targets left out), and so was a contiguous eighth of the
+// array per XCD (341).
+// n = N V < 2^31 values; by_V divides a value's index by V.
+// One 16-byte chunk inside one token's column, values j .. j + 3 of it.
+template <bool kOverwrite>
+__device__ inline void grad_chunk(const XentArgs& a, uint32_t token, uint32_t e, uint32_t j) {
+  const f32x4* in = reinterpret_cast<const f32x4*>(a.logits + e);
+  f32x4* out = reinterpret_cast<f32x4*>(a.dlogits + e);
+  const int64_t raw = index_at(a.targets, token, a.index_type);
+  const float lse = a.lse_in[token];
+  if (raw == a.ignore_index) {  // the reference adds zero
+    if (kOverwrite && a.zero_ignored) __builtin_nontemporal_store(f32x4{0.0f, 0.0f, 0.0f, 0.0f}, out);
+    return;
+  }
+  const f32x4 x = __builtin_nontemporal_load(in);
+  f32x4 o;
+  if (!kOverwrite) o = __builtin_nontemporal_load(out);
+  const float w = grad_factor(a, token);
+  const int64_t at = raw - a.index_base;  // outside [0, V): no one-hot term, as the reference's comparison
+  const int t = at >= 0 && at < a.V ? (int)at - (int)j : -1;
+  f32x4 g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float p = exp2f((x[i] - lse) * kLog2e);
+    g[i] = w * (p - (i == t ? 1.0f : 0.0f));
+  }
+  __builtin_nontemporal_store(kOverwrite ? g : o + g, out);
+}
+
+template <bool kOverwrite>
+__global__ __launch_bounds__(256) void xent_grad_kernel(XentArgs a, FastDiv by_V, uint32_t n) {
+  const uint32_t V = (uint32_t)a.V;
+  // A block inside one column has its token, target and log-sum-exp in scalar
+  // registers (the same pass with them per thread took 373 us).
+  const uint32_t e0 = 1024 * blockIdx.x, token0 = divide(e0, by_V), j0 = e0 - token0 * V;
+  if (j0 + 1024 <= V) {
+    grad_chunk<kOverwrite>(a, token0, e0 + 4 * threadIdx.x, j0 + 4 * threadIdx.x);
+    return;
+  }
+  const uint32_t e = e0 + 4 * threadIdx.x;
+  if (e >= n) return;
+  const uint32_t token = divide(e, by_V), j = e - token * V;
+  if (j + 4 <= V) {
+    grad_chunk<kOverwrite>(a, token, e, j);
+    return;
+  }
+  for (uint32_t i = 0; i < 4 && e + i < n; ++i) {
+    const uint32_t tok = divide(e + i, by_V);
+    const int64_t raw = index_at(a.targets, tok, a.index_type);
+    float* out = a.dlogits + e + i;
+    if (raw == a.ignore_index) {
+      if (kOverwrite && a.zero_ignored) *out = 0.0f;
+      continue;
+    }
+    const float p = exp2f((a.logits[e + i] - a.lse_in[tok]) * kLog2e);
+    const float g = grad_factor(a, tok) * (p - ((int64_t)(e + i - tok * V) == raw - a.index_base ? 1.0f : 0.0f));
+    *out = kOverwrite ? g : *out + g;
+  }
+}
+
+// Gradient of one column per workgroup: the log-sum-exp is formed here when
+// the caller has none, and buffers off a 16-byte boundary (kVec false) go
+// value by value.
 template <bool kVec>
 __global__ __launch_bounds__(256) void xent_bwd_kernel(XentArgs a) {
   const int64_t token = blockIdx.x;
   const int64_t raw = index_at(a.targets, token, a.index_type);
-  if (raw == a.ignore_index) return;  // the reference adds zero (uniform per workgroup)
   const float* col = a.logits + token * (int64_t)a.V;
   float* out = a.dlogits + token * (int64_t)a.V;
+  if (raw == a.ignore_index) {  // the reference adds zero (uniform per workgroup)
+    if (a.zero_ignored)
+      for (int j = threadIdx.x; j < a.V; j += 256) out[j] = 0.0f;
+    return;
+  }
   float lse;
   if (a.lse_in != nullptr) {
     lse = a.lse_in[token];
   } else {
-    const Lse r = block_combine(column_pass<kVec>(col, a.V));
+    const Lse r = block_combine(column_pass<false>(col, a.V, threadIdx.x));
     lse = r.m + logf(r.s);
   }
-  // scale = dy / count(valid) ("mean"), dy ("sum"), dy[token] ("none"); the
-  // division is the reference's fp32 `dy ./ sum(valid)`.
-  float w = a.dy[a.reduction == 0 ? token : 0];
-  if (a.reduction == 2) w = w / *a.count;
+  const float w = grad_factor(a, token);
   const int64_t t = raw - a.index_base;  // outside [0, V): no one-hot term, as the reference's comparison
   if (kVec) {
     // rounds of kBwdBatch 16-byte chunks: every load of a round (logits and,
@@ -338,10 +456,11 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(EmbedArgs a) {
 }  // namespace
 
 hipError_t launch_xent_fwd(const XentArgs& a, hipStream_t s) {
-  const bool vec = a.V % 4 == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0;
   const ProfileMark mk = profile_begin(s);
-  if (vec) hipLaunchKernelGGL(xent_fwd_kernel<true>, dim3((unsigned)a.N), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(xent_fwd_kernel<false>, dim3((unsigned)a.N), dim3(256), 0, s, a);
+  const dim3 waves((unsigned)((a.N + 3) / 4)), block(256);
+  if (a.V <= kWaveV / 8) hipLaunchKernelGGL(xent_fwd_wave_kernel<1>, waves, block, 0, s, a);
+  else if (a.V <= kWaveV) hipLaunchKernelGGL(xent_fwd_wave_kernel<4>, waves, block, 0, s, a);
+  else hipLaunchKernelGGL(xent_fwd_kernel, dim3((unsigned)a.N), block, 0, s, a);
   hipError_t e = hipGetLastError();
   profile_end(mk, "xent_fwd", s);
   if (e != hipSuccess || (a.reduced == nullptr && a.count == nullptr)) return e;
@@ -373,12 +492,42 @@ hipError_t launch_xent_fused(const XentArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The one-run gradient, in parts of fewer than 2^31 values whose token counts
+// are multiples of 4 (every part then starts on a 16-byte boundary).
+static hipError_t launch_xent_grad(const XentArgs& a, hipStream_t s) {
+  const int64_t part = ((((int64_t)1 << 31) - 1) / a.V) & ~(int64_t)3;
+  const size_t index_size = a.index_type == 1 ? 8 : 4;
+  for (int64_t at = 0; at < a.N; at += part) {
+    XentArgs p = a;
+    p.N = a.N - at < part ? a.N - at : part;
+    p.logits += at * a.V;
+    p.dlogits += at * a.V;
+    p.lse_in += at;
+    p.targets = static_cast<const char*>(a.targets) + at * index_size;
+    if (a.reduction == 0) p.dy += at;
+    const uint32_t n = (uint32_t)(p.N * p.V);
+    const dim3 grid((n + 1023) / 1024);
+    if (a.overwrite) hipLaunchKernelGGL(xent_grad_kernel<true>, grid, dim3(256), 0, s, p, fast_div((uint32_t)p.V), n);
+    else hipLaunchKernelGGL(xent_grad_kernel<false>, grid, dim3(256), 0, s, p, fast_div((uint32_t)p.V), n);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t launch_xent_bwd(const XentArgs& a, hipStream_t s) {
-  const bool vec = a.V % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.logits) | reinterpret_cast<uintptr_t>(a.dlogits)) & 15) == 0;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(a.logits) | reinterpret_cast<uintptr_t>(a.dlogits)) & 15) == 0;
   const ProfileMark mk = profile_begin(s);
-  if (vec) hipLaunchKernelGGL(xent_bwd_kernel<true>, dim3((unsigned)a.N), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(xent_bwd_kernel<false>, dim3((unsigned)a.N), dim3(256), 0, s, a);
-  const hipError_t e = hipGetLastError();
+  hipError_t e;
+  // One run of chunks needs the log-sum-exp beforehand, 16-byte alignment of
+  // both arrays and parts of at least four columns below 2^31 values.
+  if (a.lse_in != nullptr && aligned && a.V < (1 << 29)) {
+    e = launch_xent_grad(a, s);
+  } else {
+    if (aligned && a.V % 4 == 0) hipLaunchKernelGGL(xent_bwd_kernel<true>, dim3((unsigned)a.N), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(xent_bwd_kernel<false>, dim3((unsigned)a.N), dim3(256), 0, s, a);
+    e = hipGetLastError();
+  }
   profile_end(mk, "xent_bwd", s);
   return e;
 }

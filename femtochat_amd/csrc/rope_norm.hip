@@ -51,8 +51,6 @@ __device__ inline void bf2(float& a, float& b) {
   b = __uint_as_float(w & 0xffff0000u);
 }
 
-__device__ inline uint32_t divide(uint32_t n, FastDiv f) { return (__umulhi(n, f.m) + n) >> f.l; }
-
 // The table row of vector vec (= (b*T + t)*NH + h): positions[b, t], or t.
 // (Whether positions are given is a template parameter: a branch on it
 // would make every vector's loads wait for the previous vector's.)

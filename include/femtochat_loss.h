@@ -62,6 +62,12 @@ fc_status fc_cross_entropy_count(const fc_xent_desc* desc, const void* targets, 
 fc_status fc_cross_entropy_bwd(const fc_xent_desc* desc, float* dlogits, const float* logits, const void* targets,
                                const float* dy, const float* count, const float* lse, void* stream);
 
+/* The same gradient written (whatever desc->flags says) over the whole of
+   dlogits: the columns of tokens with an ignored target become zeros, so
+   dlogits needs no clearing before or after. */
+fc_status fc_cross_entropy_bwd_full(const fc_xent_desc* desc, float* dlogits, const float* logits, const void* targets,
+                                    const float* dy, const float* count, const float* lse, void* stream);
+
 /* Forward and gradient in one pass over the logits, for the loss as the last
    node of the step: the losses (and optionally lse and the reduced value, as
    fc_cross_entropy_fwd) and dlogits += (or, with FC_FLAG_OVERWRITE, =)

@@ -329,3 +329,60 @@ def test_embedding_bench_size(gpu):
     embedding_gradient_(dW, dy, tok)
     ref = torch.zeros(vocab, D, device=gpu, dtype=torch.float64).index_add_(0, tok.long(), dy.double())
     assert rel_err(dW.cpu().numpy(), ref.cpu().numpy()) < TOL
+
+
+@pytest.mark.parametrize("N,V", [(1, 1), (9, 1), (7, 2), (33, 3), (5, 4), (64, 5), (40, 7), (129, 50), (11, 1023),
+                                 (12, 1024), (13, 1025), (3, 4099), (5, 50257)])
+@pytest.mark.parametrize("reduction", ["none", "sum", "mean"])
+def test_gradient_routes_agree(gpu, N, V, reduction):
+    """The gradient over the whole array as one run of chunks (log-sum-exp
+    given, aligned buffers) equals the one-column-per-workgroup kernel (the
+    same call on a buffer 4 bytes off): bit for bit when written; when added, up
+    to one rounding of the gradient (|g| <= dy + 1 <= 2.5) and one of the sum, as
+    a compiler may fuse the last product into the addition; and
+    fc_cross_entropy_bwd_full adds zeros in the ignored columns only."""
+    x, t, xd, td = _ce_case(gpu, N, V, seed=7 * N + V)
+    if N > 1:
+        td[0], td[-1] = V + 3, -1  # outside the vocabulary; ignored
+    lse, count = torch.empty(N, device=gpu), torch.empty(1, device=gpu)
+    cross_entropy_(torch.empty(N, device=gpu), xd, td, -1, reduction, lse=lse, count=count)
+    ref = torch.logsumexp(x.double(), 1)
+    assert float((lse.cpu().double() - ref).abs().max()) < TOL * max(1.0, float(ref.abs().max()))
+    dy = torch.rand(N if reduction == "none" else 1, device=gpu) + 0.5
+    base = torch.randn(N, V, device=gpu)
+    for accumulate in (True, False):
+        one, rows = base.clone(), torch.empty(N * V + 4, device=gpu)[1:N * V + 1].view(N, V)
+        rows.copy_(base)
+        for delta in (one, rows):
+            cross_entropy_gradient_(delta, xd, td, dy, -1, reduction, lse=lse, count=count, accumulate=accumulate)
+        if accumulate:
+            assert float(((one - rows).abs() - 2.0 ** -24 * (one.abs() + 2.5)).max()) <= 2.0 ** -24 * float(one.abs().max())
+        else:
+            assert torch.equal(one, rows)
+        ign = td == -1
+        assert torch.equal(one[ign], base[ign])
+    leaf = xd.clone().requires_grad_(True)
+    loss = CrossEntropyFunction.apply(leaf, td, -1, reduction)
+    (g,) = torch.autograd.grad(loss, leaf, dy if reduction == "none" else dy[0])
+    assert torch.equal(g[~ign], one[~ign]) and not g[ign].any()
+
+
+def test_masked_logits(gpu):
+    """Vocabulary entries at -inf add nothing to the sum, wherever they stand
+    in the column (a whole first round of loads, the head and the tail)."""
+    for V in (4099, 8192, 33):
+        x = torch.randn(6, V, generator=torch.Generator().manual_seed(V))
+        x[:, :V // 2] = -float("inf")
+        x[1, :V - 1] = -float("inf")
+        x[2, V // 2:] = x[2, V // 2:] + 100.0
+        x[3, -2:] = -float("inf")
+        t = torch.full((6,), V - 1)
+        t[3] = V - 3
+        xd = x.to(gpu).requires_grad_(True)
+        losses = CrossEntropyFunction.apply(xd, t.to(gpu), -1, "none")
+        losses.sum().backward()
+        x64 = x.double().requires_grad_(True)
+        ref = F.cross_entropy(x64, t, reduction="none")
+        ref.sum().backward()
+        assert float((losses.detach().cpu().double() - ref.detach()).abs().max()) < 1e-4
+        assert rel_err(xd.grad.cpu().numpy(), x64.grad.numpy()) < TOL
