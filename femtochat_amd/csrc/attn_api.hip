@@ -684,16 +684,41 @@ fc_status fc_embedding_fwd(const fc_embed_desc* desc, const float* weights, cons
   return ok();
 }
 
+static fc_status embed_bwd_args(const char* who, const fc_embed_desc* desc, float* dweights, const void* dy,
+                                const void* tokens, fc::EmbedArgs* a) {
+  const fc_status st = embed_args(desc, tokens, who, a);
+  if (st != FC_OK) return st;
+  if (dweights == nullptr || dy == nullptr) return fail(FC_ERR_INVALID_ARGUMENT, "%s: dweights and dy are required", who);
+  if (!aligned4(dweights) || (reinterpret_cast<uintptr_t>(dy) & (desc->y_dtype == FC_BF16 ? 1 : 3)) != 0)
+    return fail(FC_ERR_INVALID_ARGUMENT, "%s: buffers are not aligned to their element size", who);
+  a->dweights = dweights;
+  a->dy = dy;
+  return FC_OK;
+}
+
 fc_status fc_embedding_bwd(const fc_embed_desc* desc, float* dweights, const void* dy, const void* tokens, void* stream) {
   fc::EmbedArgs a;
-  const fc_status st = embed_args(desc, tokens, "fc_embedding_bwd", &a);
+  const fc_status st = embed_bwd_args("fc_embedding_bwd", desc, dweights, dy, tokens, &a);
   if (st != FC_OK) return st;
-  if (dweights == nullptr || dy == nullptr) return fail(FC_ERR_INVALID_ARGUMENT, "fc_embedding_bwd: dweights and dy are required");
-  if (!aligned4(dweights) || (reinterpret_cast<uintptr_t>(dy) & (desc->y_dtype == FC_BF16 ? 1 : 3)) != 0)
-    return fail(FC_ERR_INVALID_ARGUMENT, "fc_embedding_bwd: buffers are not aligned to their element size");
-  a.dweights = dweights;
-  a.dy = dy;
   const hipError_t e = fc::launch_embed(a, true, desc->y_dtype == FC_BF16, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(FC_ERR_HIP, "embedding gradient launch failed: %s", hipGetErrorString(e));
+  return ok();
+}
+
+fc_status fc_embedding_bwd_full(const fc_embed_desc* desc, float* dweights, const void* dy, const void* tokens,
+                                void* stream) {
+  fc::EmbedArgs a;
+  fc_status st = embed_bwd_args("fc_embedding_bwd_full", desc, dweights, dy, tokens, &a);
+  if (st != FC_OK) return st;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  hipError_t e;
+  if (fc::embed_grad_full_supported(a)) {
+    e = fc::launch_embed_grad_full(a, desc->y_dtype == FC_BF16, s);
+  } else {
+    st = fc_fill_zero(dweights, (size_t)a.vocab * a.D * sizeof(float), stream);
+    if (st != FC_OK) return st;
+    e = fc::launch_embed(a, true, desc->y_dtype == FC_BF16, s);
+  }
   if (e != hipSuccess) return fail(FC_ERR_HIP, "embedding gradient launch failed: %s", hipGetErrorString(e));
   return ok();
 }

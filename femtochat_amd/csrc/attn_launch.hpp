@@ -161,6 +161,10 @@ struct EmbedArgs {
 };
 hipError_t launch_embed(const EmbedArgs& a, bool backward, bool bf16_y, hipStream_t s);
 
+// The gradient into a fresh table (embed_grad.hip).
+bool embed_grad_full_supported(const EmbedArgs& a);
+hipError_t launch_embed_grad_full(const EmbedArgs& a, bool bf16_dy, hipStream_t s);
+
 // Workspace of the sorted (deterministic) embedding gradient: keys and token
 // indices before and after the sort, and the sort's own temporary storage
 // (byte offsets, 256-aligned).

@@ -275,6 +275,10 @@ class EmbeddingFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         (tokens,) = ctx.saved_tensors
-        dw = torch.zeros(ctx.vocab_shape, dtype=torch.float32, device=dy.device)
-        embedding_gradient_(dw, dy.contiguous(), tokens)
+        dw = torch.empty(ctx.vocab_shape, dtype=torch.float32, device=dy.device)
+        dy = dy.contiguous()
+        d = _embed_desc(dw, tokens, dy.dtype, 0)
+        _check_tensor("dy", dy, tuple(tokens.shape) + (dw.shape[1],), (torch.float32, torch.bfloat16), dw.device)
+        _lib.check(_lib.lib().fc_embedding_bwd_full(ctypes.byref(d), _ptr(dw), _ptr(dy), _ptr(tokens),
+                                                    _stream_ptr(dw.device)))
         return dw, None, None

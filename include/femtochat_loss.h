@@ -106,6 +106,13 @@ fc_status fc_embedding_fwd(const fc_embed_desc* desc, const float* weights, cons
 fc_status fc_embedding_bwd(const fc_embed_desc* desc, float* dweights, const void* dy, const void* tokens,
                            void* stream);
 
+/* The same gradient written over the whole of dweights (sums of the tokens'
+   dy columns, zeros elsewhere), so dweights needs no clearing; one kernel, no
+   workspace, and the same bits on every call (a table of more than 2^19
+   columns is cleared and added into with atomics instead). */
+fc_status fc_embedding_bwd_full(const fc_embed_desc* desc, float* dweights, const void* dy, const void* tokens,
+                                void* stream);
+
 /* Bytes of the caller-owned workspace of fc_embedding_bwd_sorted for these
    N and vocab (the sort's keys and token indices and its temporary storage). */
 fc_status fc_embedding_bwd_workspace_bytes(const fc_embed_desc* desc, size_t* bytes);

@@ -11,6 +11,8 @@ token is distinct.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -386,3 +388,49 @@ def test_masked_logits(gpu):
         ref.sum().backward()
         assert float((losses.detach().cpu().double() - ref.detach()).abs().max()) < 1e-4
         assert rel_err(xd.grad.cpu().numpy(), x64.grad.numpy()) < TOL
+
+
+@pytest.mark.parametrize("N,vocab,D,dy_dtype", [
+    (1, 1, 4, torch.float32), (63, 2, 32, torch.bfloat16), (300, 50, 6, torch.float32), (4095, 255, 256, torch.bfloat16),
+    (4096, 256, 260, torch.float32), (4097, 257, 30, torch.bfloat16), (9000, 32768, 512, torch.bfloat16),
+    (20000, 33000, 64, torch.float32), (5000, 50257, 1000, torch.float32), (70, 600000, 8, torch.float32),
+])
+@pytest.mark.parametrize("ids", ["uniform", "words", "one", "three"])
+def test_embedding_gradient_full(gpu, N, vocab, D, dy_dtype, ids):
+    """The gradient written over a fresh table (NaN before) against float64
+    sums: within the rounding of an fp32 sum of that many terms, zeros where no
+    token points, nothing from ids outside the table, the same bits twice; the
+    list's edges (a scan step is 4096 tokens, a list 6144), one id for all
+    tokens, tables around 256 groups of 128 columns, both load widths."""
+    g = torch.Generator().manual_seed(N + vocab + D)
+    if ids == "uniform":
+        tok = torch.randint(0, vocab, (N,), generator=g)
+    elif ids == "words":
+        tok = (vocab * torch.rand(N, generator=g) ** 6).long().clamp(max=vocab - 1)
+    else:
+        tok = torch.randint(0, vocab, (3 if ids == "three" else 1,), generator=g).repeat(N)[:N]
+    if N > 2:
+        tok[1], tok[N // 2] = -1, vocab  # outside the table
+    dy = torch.randn(N, D, generator=g).to(dy_dtype)
+    dy[N // 3] = 0
+    ok = (tok >= 0) & (tok < vocab)
+    ref = torch.zeros(vocab, D, dtype=torch.float64).index_add_(0, tok[ok], dy[ok].double())
+    size = torch.zeros(vocab, D, dtype=torch.float64).index_add_(0, tok[ok], dy[ok].double().abs())
+    terms = torch.bincount(tok[ok], minlength=vocab).double()[:, None]
+    outs = []
+    for itype in (torch.int32, torch.int64):
+        dw = torch.full((vocab, D), float("nan"), device=gpu)
+        d = _lib.EmbedDesc()
+        d.vocab, d.D, d.N, d.index_base = vocab, D, N, 0
+        d.index_type = _lib.FC_INDEX_I64 if itype == torch.int64 else _lib.FC_INDEX_I32
+        d.y_dtype, d.flags = _lib.FC_BF16 if dy_dtype == torch.bfloat16 else _lib.FC_F32, 0
+        dyd, td = dy.to(gpu), tok.to(itype).to(gpu)
+        p = lambda t: ctypes.c_void_p(t.data_ptr())
+        _lib.check(_lib.lib().fc_embedding_bwd_full(ctypes.byref(d), p(dw), p(dyd), p(td),
+                                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        outs.append(dw.cpu())
+    err = (outs[0].double() - ref).abs()
+    assert bool((err <= terms * 2.0 ** -24 * size).all()), float(err.max())
+    assert not outs[0][terms[:, 0] == 0].any()
+    if vocab <= 1 << 19:
+        assert torch.equal(outs[0], outs[1])
