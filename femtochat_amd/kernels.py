@@ -36,6 +36,7 @@ reference's behaviour exactly.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from typing import NamedTuple, Optional, Tuple
 
 import torch
@@ -129,12 +130,14 @@ def window_sizes(sequence_len: int, n_layer: int, window_pattern: str = "L"):
     return windows
 
 
+_DTYPE_CODES = {torch.float32: _lib.FC_F32, torch.bfloat16: _lib.FC_BF16}
+
+
 def _dtype_code(dtype: torch.dtype) -> int:
-    if dtype == torch.float32:
-        return _lib.FC_F32
-    if dtype == torch.bfloat16:
-        return _lib.FC_BF16
-    raise TypeError(f"unsupported dtype {dtype}; the library stores float32 or bfloat16")
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {dtype}; the library stores float32 or bfloat16")
+    return code
 
 
 def instruction(dtype: torch.dtype, device=None, D: Optional[int] = None):
@@ -203,15 +206,23 @@ def attention_inputs(A, Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor):
     return tuple(conv(x) for x in (Q, K, V))
 
 
-def _stream_ptr(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# Host time per call counts at the smallest sizes (a toy layer's step is a few
+# kernels of a few microseconds each), so pointers and streams go to ctypes as
+# plain integers and a valid tensor is checked in one expression.
+def _stream_ptr(device: torch.device) -> int:
+    """The handle of the device's current stream."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _check_tensor(name, t, shape, dtypes, device):
+    if (isinstance(t, torch.Tensor) and t.device == device and t.shape == shape and t.dtype in dtypes
+            and t.is_contiguous()):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.device != device:
@@ -220,8 +231,7 @@ def _check_tensor(name, t, shape, dtypes, device):
         raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
     if t.dtype not in dtypes:
         raise TypeError(f"{name} has dtype {t.dtype}, expected one of {dtypes}")
-    if not t.is_contiguous():
-        raise ValueError(f"{name} must be contiguous")
+    raise ValueError(f"{name} must be contiguous")
 
 
 def _stats_shape(t: torch.Tensor, B: int, H: int, T: int):
@@ -233,19 +243,20 @@ def _desc(A, Q, K, window, out_dtype, dout_dtype, grad_dtype, overwrite=False) -
         raise TypeError(f"expected MFMAExact() or MFMAFast(), got {A!r}")
     if Q.dim() != 4 or K.dim() != 4:
         raise ValueError("Q, K, V must be 4-d (B, T, H, D) tensors")
+    if Q.dim() != 4 or K.dim() != 4:
+        raise ValueError("Q, K, V must be 4-d (B, T, H, D) tensors")
     B, T, H, D = Q.shape
-    Hkv = K.shape[2]
-    left, right = (int(window[0]), int(window[1]))
-    d = _lib.AttnDesc()
-    d.D, d.H, d.Hkv, d.T, d.B = D, H, Hkv, T, B
-    d.win_left, d.win_right = left, right
-    d.mode = A.mode
-    d.in_dtype = _dtype_code(Q.dtype)
-    d.out_dtype = out_dtype
-    d.dout_dtype = dout_dtype
-    d.grad_dtype = grad_dtype
-    d.flags = _lib.FC_FLAG_OVERWRITE if overwrite else 0
-    return d
+    return _lib.AttnDesc(D, H, K.shape[2], T, B, int(window[0]), int(window[1]), A.mode, _dtype_code(Q.dtype), out_dtype,
+                         dout_dtype, grad_dtype, _lib.FC_FLAG_OVERWRITE if overwrite else 0)
+
+
+@lru_cache(maxsize=256)
+def _workspace_bytes(fields: bytes, which: int, with_positions: bool) -> int:
+    """fc_attn_workspace_bytes of a descriptor (its bytes: sizes and options only)."""
+    n = ctypes.c_size_t(0)
+    d = _lib.AttnDesc.from_buffer_copy(fields)
+    _lib.check(_lib.lib().fc_attn_workspace_bytes(ctypes.byref(d), which, int(with_positions), ctypes.byref(n)))
+    return n.value
 
 
 def _check_common(A, Q, K, V, positions):
@@ -285,27 +296,24 @@ def attention_(A, O, l, m, Q, K, V, window: Tuple[int, int], *, positions=None,
     _check_tensor("O", O, (B, T, H, D), out_dtypes, device)
     _check_tensor("l", l, _stats_shape(l, B, H, T), (torch.float32,), device)
     _check_tensor("m", m, _stats_shape(m, B, H, T), (torch.float32,), device)
+    _forward(A, O, l, m, Q, K, V, window, positions, workspace)
+
+
+def _forward(A, O, l, m, Q, K, V, window, positions, workspace=None) -> None:
+    """attention_ on checked tensors."""
+    device = Q.device
     oc = _dtype_code(O.dtype)
     d = _desc(A, Q, K, window, oc, oc, oc)
-    lib = _lib.lib()
-    nbytes = ctypes.c_size_t(0)
-    _lib.check(lib.fc_attn_workspace_bytes(ctypes.byref(d), _lib.FC_PASS_FORWARD, int(positions is not None),
-                                           ctypes.byref(nbytes)))
-    ws, aligned = None, None
-    if nbytes.value > 0:
+    nbytes = _workspace_bytes(bytes(d), _lib.FC_PASS_FORWARD, positions is not None)
+    aligned = None
+    if nbytes > 0:
         if workspace is None:
-            ws = torch.empty(int(nbytes.value) + 256, dtype=torch.uint8, device=device)
-        else:
-            ws = workspace
-            if ws.device != device or ws.numel() * ws.element_size() < int(nbytes.value) + 256:
-                raise ValueError(f"workspace must be a {int(nbytes.value) + 256}-byte tensor on {device}")
-        aligned = ctypes.c_void_p((ws.data_ptr() + 255) & ~255)
-    _lib.check(
-        lib.fc_attn_fwd(
-            ctypes.byref(d), _ptr(Q), _ptr(K), _ptr(V), _ptr(positions), _ptr(O), _ptr(l), _ptr(m),
-            aligned, ctypes.c_size_t(int(nbytes.value) if ws is not None else 0), _stream_ptr(device),
-        )
-    )
+            workspace = torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
+        elif workspace.device != device or workspace.numel() * workspace.element_size() < nbytes + 256:
+            raise ValueError(f"workspace must be a {nbytes + 256}-byte tensor on {device}")
+        aligned = (workspace.data_ptr() + 255) & ~255
+    _lib.check(_lib.lib().fc_attn_fwd(ctypes.byref(d), Q.data_ptr(), K.data_ptr(), V.data_ptr(), _ptr(positions),
+                                      O.data_ptr(), l.data_ptr(), m.data_ptr(), aligned, nbytes, _stream_ptr(device)))
 
 
 def delta_attention_(
@@ -327,30 +335,23 @@ def delta_attention_(
     _check_tensor("dQ", dQ, (B, T, H, D), io_dtypes, device)
     _check_tensor("dK", dK, (B, T, Hkv, D), (dQ.dtype,), device)
     _check_tensor("dV", dV, (B, T, Hkv, D), (dQ.dtype,), device)
+    _backward(A, dQ, dK, dV, dO, Q, K, V, O, l, m, window, positions, accumulate, workspace)
+
+
+def _backward(A, dQ, dK, dV, dO, Q, K, V, O, l, m, window, positions, accumulate, workspace=None) -> None:
+    """delta_attention_ on checked tensors."""
+    device = Q.device
     d = _desc(A, Q, K, window, _dtype_code(O.dtype), _dtype_code(dO.dtype), _dtype_code(dQ.dtype),
               overwrite=not accumulate)
-    lib = _lib.lib()
-    nbytes = ctypes.c_size_t(0)
-    _lib.check(lib.fc_attn_workspace_bytes(ctypes.byref(d), _lib.FC_PASS_BACKWARD, int(positions is not None),
-                                           ctypes.byref(nbytes)))
-    if workspace is None:
-        ws = torch.empty(max(int(nbytes.value), 256) + 256, dtype=torch.uint8, device=device)
-    else:
-        ws = workspace
-        if ws.device != device or ws.numel() * ws.element_size() < int(nbytes.value) + 256:
-            raise ValueError(f"workspace must be a {int(nbytes.value) + 256}-byte tensor on {device}")
-    base = ws.data_ptr()
-    aligned = (base + 255) & ~255
-    _lib.check(
-        lib.fc_attn_bwd(
-            ctypes.byref(d), _ptr(dO), _ptr(Q), _ptr(K), _ptr(V), _ptr(O), _ptr(l), _ptr(m), _ptr(positions),
-            _ptr(dQ), _ptr(dK), _ptr(dV), ctypes.c_void_p(aligned), ctypes.c_size_t(int(nbytes.value)),
-            _stream_ptr(device),
-        )
-    )
-    # An internally allocated workspace must outlive the kernels on this stream.
-    if workspace is None:
-        ws.record_stream(torch.cuda.current_stream(device))
+    nbytes = _workspace_bytes(bytes(d), _lib.FC_PASS_BACKWARD, positions is not None)
+    if workspace is None:  # freed to this stream's pool on return, so later work on the stream comes after the kernels
+        workspace = torch.empty(max(nbytes, 256) + 256, dtype=torch.uint8, device=device)
+    elif workspace.device != device or workspace.numel() * workspace.element_size() < nbytes + 256:
+        raise ValueError(f"workspace must be a {nbytes + 256}-byte tensor on {device}")
+    _lib.check(_lib.lib().fc_attn_bwd(
+        ctypes.byref(d), dO.data_ptr(), Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), l.data_ptr(),
+        m.data_ptr(), _ptr(positions), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
+        (workspace.data_ptr() + 255) & ~255, nbytes, _stream_ptr(device)))
 
 
 def forward_workspace_bytes(A, Q, K, *, positions=None) -> int:
@@ -358,10 +359,8 @@ def forward_workspace_bytes(A, Q, K, *, positions=None) -> int:
     accepts (the library's requirement plus 256 bytes of alignment slack; 0
     when the problem needs none)."""
     d = _desc(A, Q, K, (-1, 0), _dtype_code(Q.dtype), _dtype_code(Q.dtype), _dtype_code(Q.dtype))
-    n = ctypes.c_size_t(0)
-    _lib.check(_lib.lib().fc_attn_workspace_bytes(ctypes.byref(d), _lib.FC_PASS_FORWARD,
-                                                  int(positions is not None), ctypes.byref(n)))
-    return int(n.value) + 256 if n.value > 0 else 0
+    n = _workspace_bytes(bytes(d), _lib.FC_PASS_FORWARD, positions is not None)
+    return n + 256 if n > 0 else 0
 
 
 def backward_workspace_bytes(A, Q, K, *, positions=None, dout_dtype=None) -> int:
@@ -369,13 +368,12 @@ def backward_workspace_bytes(A, Q, K, *, positions=None, dout_dtype=None) -> int
     accepts (the library's requirement plus 256 bytes of alignment slack)."""
     dd = _dtype_code(dout_dtype or Q.dtype)
     d = _desc(A, Q, K, (-1, 0), dd, dd, dd)
-    n = ctypes.c_size_t(0)
-    _lib.check(_lib.lib().fc_attn_workspace_bytes(ctypes.byref(d), _lib.FC_PASS_BACKWARD,
-                                                   int(positions is not None), ctypes.byref(n)))
-    return int(n.value) + 256
+    return _workspace_bytes(bytes(d), _lib.FC_PASS_BACKWARD, positions is not None) + 256
 
 
 def _reject_unknown(options: dict) -> None:
+    if not options:
+        return
     unknown = set(options) - _GEOMETRY_KEYWORDS
     if unknown:
         raise TypeError(f"unexpected keyword(s) {sorted(unknown)}")
@@ -398,7 +396,11 @@ def attention_state(A, Q, K, V, window, *, positions=None, **options) -> Attenti
     F = accumulator_type(A, Q.dtype)
     l = torch.empty((B, H, T), dtype=F, device=Q.device)
     m = torch.empty((B, H, T), dtype=F, device=Q.device)
-    attention_(A, O, l, m, Qc, Kc, Vc, window, positions=positions, **options)
+    if options:
+        attention_(A, O, l, m, Qc, Kc, Vc, window, positions=positions, **options)
+    else:  # O, l and m need no checks
+        _check_common(A, Qc, Kc, Vc, positions)
+        _forward(A, O, l, m, Qc, Kc, Vc, window, positions)
     return AttentionState(A, Qc, Kc, Vc, O, l, m)
 
 
@@ -428,15 +430,14 @@ class AttentionFunction(torch.autograd.Function):
     def forward(ctx, Q, K, V, window, A=None, positions=None):
         A = A if A is not None else instruction(Q.dtype, Q.device, Q.shape[-1])
         st = attention_state(A, Q, K, V, window, positions=positions)
-        ctx.save_for_backward(st.Q, st.K, st.V, st.O, st.l, st.m, positions if positions is not None else Q.new_empty(0))
-        ctx.A, ctx.window, ctx.has_pos = A, window, positions is not None
+        ctx.save_for_backward(st.Q, st.K, st.V, st.O, st.l, st.m, positions)
+        ctx.A, ctx.window = A, window
         ctx.dtypes = (Q.dtype, K.dtype, V.dtype)
         return st.O
 
     @staticmethod
     def backward(ctx, dO):
-        Q, K, V, O, l, m, pos = ctx.saved_tensors
-        positions = pos if ctx.has_pos else None
+        Q, K, V, O, l, m, positions = ctx.saved_tensors
         dO = dO.contiguous()
         if dO.dtype != O.dtype:
             dO = dO.to(O.dtype)

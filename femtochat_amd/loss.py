@@ -61,15 +61,8 @@ def _xent_desc(logits, targets, ignore_index, reduction, index_base, overwrite=F
     dev = _device(logits)
     _check_tensor("logits", logits, tuple(logits.shape), (torch.float32,), dev)
     _check_tensor("targets", targets, tuple(targets.shape), tuple(_INDEX), dev)
-    d = _lib.XentDesc()
-    d.V = logits.shape[-1]
-    d.N = targets.numel()
-    d.index_base = index_base
-    d.ignore_index = ignore_index
-    d.index_type = _INDEX[targets.dtype]
-    d.reduction = _REDUCTIONS[reduction]
-    d.flags = _lib.FC_FLAG_OVERWRITE if overwrite else 0
-    return d
+    return _lib.XentDesc(logits.shape[-1], index_base, targets.numel(), ignore_index, _INDEX[targets.dtype],
+                         _REDUCTIONS[reduction], _lib.FC_FLAG_OVERWRITE if overwrite else 0)
 
 
 def cross_entropy_(losses: torch.Tensor, logits: torch.Tensor, targets: torch.Tensor, ignore_index: int = -1,
@@ -132,7 +125,8 @@ def _gradient(entry, d, delta, logits, targets, dy, ignore_index, reduction, lse
     _check_tensor("delta", delta, tuple(logits.shape), (torch.float32,), dev)
     if not isinstance(dy, torch.Tensor):
         dy = torch.full((1,), float(dy), dtype=torch.float32, device=dev)
-    dy = dy.to(device=dev, dtype=torch.float32).contiguous()
+    if dy.dtype != torch.float32 or dy.device != dev or not dy.is_contiguous():
+        dy = dy.to(device=dev, dtype=torch.float32).contiguous()
     need = targets.numel() if reduction == "none" else 1
     if dy.numel() != need:
         raise ValueError(f"dy must hold {need} value(s) for reduction {reduction!r}, got {dy.numel()}")
@@ -206,14 +200,9 @@ def _embed_desc(weights, tokens, y_dtype, index_base) -> _lib.EmbedDesc:
         raise ValueError("weights must be (vocab, D)")
     _check_tensor("weights", weights, tuple(weights.shape), (torch.float32,), dev)
     _check_tensor("tokens", tokens, tuple(tokens.shape), tuple(_INDEX), dev)
-    d = _lib.EmbedDesc()
-    d.vocab, d.D = weights.shape
-    d.N = tokens.numel()
-    d.index_base = index_base
-    d.index_type = _INDEX[tokens.dtype]
-    d.y_dtype = _lib.FC_BF16 if y_dtype == torch.bfloat16 else _lib.FC_F32
-    d.flags = 0
-    return d
+    vocab, D = weights.shape
+    return _lib.EmbedDesc(D, vocab, tokens.numel(), index_base, _INDEX[tokens.dtype],
+                          _lib.FC_BF16 if y_dtype == torch.bfloat16 else _lib.FC_F32, 0)
 
 
 def embedding_(y: torch.Tensor, weights: torch.Tensor, tokens: torch.Tensor, *, index_base: int = 0) -> None:

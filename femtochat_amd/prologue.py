@@ -66,12 +66,8 @@ def rotary_embeddings(seq_len: int, head_dim: int, base: float = 100_000.0, devi
 
 def _desc(X: torch.Tensor, table_len: int, overwrite: bool) -> _lib.RopeNormDesc:
     B, T, NH, D = X.shape
-    d = _lib.RopeNormDesc()
-    d.D, d.NH, d.T, d.B = D, NH, T, B
-    d.table_len = table_len
-    d.dtype = _lib.FC_BF16 if X.dtype == torch.bfloat16 else _lib.FC_F32
-    d.flags = _lib.FC_FLAG_OVERWRITE if overwrite else 0
-    return d
+    return _lib.RopeNormDesc(D, NH, T, B, table_len, _lib.FC_BF16 if X.dtype == torch.bfloat16 else _lib.FC_F32,
+                             _lib.FC_FLAG_OVERWRITE if overwrite else 0)
 
 
 def _check(X: torch.Tensor, sin_cos, positions):
@@ -135,16 +131,14 @@ class AttentionPrologueFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, X, sin, cos, positions=None):
         X = X.contiguous()
-        ctx.save_for_backward(X, sin, cos, positions if positions is not None else torch.empty(0))
-        ctx.has_positions = positions is not None
+        ctx.save_for_backward(X, sin, cos, positions)
         return attention_prologue(X, (sin, cos), positions)
 
     @staticmethod
     def backward(ctx, dY):
-        X, sin, cos, pos = ctx.saved_tensors
+        X, sin, cos, positions = ctx.saved_tensors
         dX = torch.empty_like(X)
-        delta_attention_prologue_(dX, dY.contiguous().to(X.dtype), X, (sin, cos),
-                                  pos if ctx.has_positions else None, accumulate=False)
+        delta_attention_prologue_(dX, dY.contiguous().to(X.dtype), X, (sin, cos), positions, accumulate=False)
         return dX, None, None, None
 
 
