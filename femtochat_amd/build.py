@@ -28,11 +28,14 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-# Per-source additions.  The dK/dV kernel at head dims up to 64 selects the
-# vector-register form of every MFMA, so that S and dP are not copied out of
-# the accumulation registers element by element (at D = 128 the compiler's
-# default, accumulation-register form stays: that kernel needs both files).
-EXTRA_FLAGS = {"attn_bwd_dkdv_vgpr.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source additions.  These units select the vector-register form of every
+# MFMA: dK/dV at head dims up to 64, so that S and dP are not copied out of the
+# accumulation registers element by element (at D = 128 the compiler's default,
+# accumulation-register form stays: that kernel needs both files), and the
+# exact-mode backward (dK/dV at D = 128 spills 115 registers without it: 1336
+# against 696 us for 8 x 2048 tokens, H6).
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+EXTRA_FLAGS = {"attn_bwd_dkdv_vgpr.hip": _VGPR_FORM, "attn_bwd.hip": _VGPR_FORM}
 
 
 def hipcc() -> str:

@@ -8,18 +8,19 @@
 // with a single visible key gets dS = 0, fp32 accumulation, optional add into
 // the caller's gradients before the one final rounding).
 //
-// Three kernels, all deterministic (no atomics):
+// Three kernels, all deterministic (no atomics); the last two here are the
+// exact-mode ones:
 //  * attn_bwd_pre  : Delta and the base-2 log-sum-exp per query, and a bf16
 //                    copy of dO when the caller hands fp32 dO in fast mode;
 //  * attn_bwd_dkdv : one workgroup per (key tile of 128, KV head, batch); the
-//                    4 waves own 32 keys each with K and V resident in
-//                    registers, and loop over every query head of the GQA
-//                    group and every query tile that can see the keys, so the
-//                    group's contributions to dK/dV are summed in registers;
+//                    4 waves own 32 keys each and loop over every query head of
+//                    the GQA group and every query tile that can see the keys,
+//                    so the group's contributions to dK/dV are summed in
+//                    registers;
 //  * attn_bwd_dq   : one workgroup per (query tile of 128, head, batch); it
 //                    recomputes S^T and dP^T with the query as the lane index
 //                    so dS^T is directly the B operand of dQ^T += K^T dS^T.
-#include "attn_device.hpp"
+#include "attn_exact.hpp"
 #include "attn_launch.hpp"
 
 #include <type_traits>
@@ -177,60 +178,71 @@ __global__ __launch_bounds__(kOrderThreads) void attn_order_kernel(OrderArgs a) 
 }
 
 // ---------------------------------------------------------------------------
-template <typename E, int D>
-struct DkdvCfg {
-  static constexpr bool kBF = std::is_same<E, bf16>::value;
-  static constexpr int kBK = 128;               // keys per workgroup (4 x 32)
-  static constexpr int kBQ = kBF ? 64 : 32;     // queries per tile
-  static constexpr int kKC = D / 16;
-  static constexpr int kDP = D < 32 ? 32 : D;
-  static constexpr int kDB = kDP / 32;
-  static constexpr int kLD = kBF ? D + 8 : D + 4;  // natural tile row stride
-  static constexpr int kLDT = kBQ + 4;             // transposed tile row stride
-  static constexpr int kNat = kBQ * kLD;
-  static constexpr int kTr = kBF ? kDP * kLDT : 0;
-  // Q, dO natural (+ transposed in bf16): one stage
-  static constexpr int kStage = 2 * kNat + 2 * kTr;
-};
+// dK and dV, exact mode (products in bf16 parts, attn_exact.hpp): 128 keys of
+// one (batch, KV head) per workgroup, 32 per wave with K and V resident as B
+// operands, their first two parts in registers and the third in LDS (all three
+// in registers spilled 69-218 of them and took 0.90-2.1 ms at D = 128); the
+// loop runs over the group's query heads and the 32-query tiles that can see
+// the keys, whose Q and dO are split once per workgroup into swizzled LDS.
+// At one wave per SIMD (D = 128) the LDS reads bound it next to the products:
+// a wave reads 112 KB of parts per tile for 192 products.  8 x 2048 tokens,
+// causal, H6 D128: 676 us (fp32 MFMA 1142-1183), H12 D64: 535 (1278).
+constexpr int kExactBK = 128;  // keys per workgroup
+constexpr int kExactBT = 32;   // rows per staged tile (queries here, keys in dQ)
 
-template <typename E, int D>
-__global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(BwdArgs a) {
-  using M = Mma<E>;
-  using C = DkdvCfg<E, D>;
-  constexpr int BQ = C::kBQ, KC = C::kKC, DB = C::kDB, NQB = BQ / 32;
-  __shared__ __attribute__((aligned(16))) E smem[2 * C::kStage];
+template <int D>
+__global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact_kernel(BwdArgs a) {
+  constexpr int BQ = kExactBT, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  constexpr int kTile = SplitTile<D>::kBytes;
+  __shared__ __attribute__((aligned(1024))) char Qbuf[2][kTile];
+  __shared__ __attribute__((aligned(1024))) char Os[kTile];  // dO
+  __shared__ __attribute__((aligned(1024))) bf16x8 s_low[kWaves][2][KC][kWave];  // third parts of K and V, per lane
   __shared__ __attribute__((aligned(16))) float s_lse[2][BQ];
   __shared__ __attribute__((aligned(16))) float s_delta[2][BQ];
   __shared__ __attribute__((aligned(16))) int s_lb[2][BQ];
+  __shared__ int s_outside;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 5, l32 = lane & 31;
   const int T = a.T;
-  const int n_kt = (T + C::kBK - 1) / C::kBK;
   // Key tiles that the most query tiles can see come first, over the whole grid.
   const GridItem it0 = heavy_first(blockIdx.x, a.Hkv * a.B);
-  const int bkv = it0.row;
-  const int kt = it0.rank;
-  const int b = bkv / a.Hkv, kvh = bkv - b * a.Hkv;
-  const int k0 = kt * C::kBK;
-  const int k1 = min(k0 + C::kBK, T) - 1;
-  const int kw0 = k0 + 32 * wave, kw1 = kw0 + 31;
+  const int b = it0.row / a.Hkv, kvh = it0.row - b * a.Hkv;
+  const int k0 = it0.rank * kExactBK;
+  const int k1 = min(k0 + kExactBK, T) - 1;
+  const int kw0 = k0 + 32 * __builtin_amdgcn_readfirstlane(wave), kw1 = kw0 + 31;
   const int key = kw0 + l32;
 
   const int64_t qpitch = (int64_t)a.H * D, kpitch = (int64_t)a.Hkv * D;
-  const E* Kb = static_cast<const E*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
-  const E* Vb = static_cast<const E*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Kb = static_cast<const float*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Vb = static_cast<const float*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
   const int32_t* pos = a.pos ? a.pos + (int64_t)b * T : nullptr;
   const int nchunks = (T + 31) / 32;
   const int32_t* clb = a.chunk_lb ? a.chunk_lb + (int64_t)b * nchunks * 2 : nullptr;
+  if (tid == 0) s_outside = 0;
 
-  // K and V of this wave's 32 keys, as B operands (lane = key).
-  typename M::frag kf[KC], vf[KC];
+  bf16x8 kf[KC][2], vf[KC][2];
+  const int64_t krow = (int64_t)min(key, T - 1) * kpitch;
+  bool outside;
+  {
+    Split8 f[KC];
+    outside = split_rows<D>(Kb + krow, key < T, g, f);
 #pragma unroll
-  for (int c = 0; c < KC; ++c) {
-    kf[c] = key < T ? M::load8(Kb + (int64_t)key * kpitch + 16 * c + 8 * g) : M::zero();
-    vf[c] = key < T ? M::load8(Vb + (int64_t)key * kpitch + 16 * c + 8 * g) : M::zero();
+    for (int c = 0; c < KC; ++c) {
+      kf[c][0] = f[c].part[0];
+      kf[c][1] = f[c].part[1];
+      s_low[wave][0][c][lane] = f[c].part[2];
+    }
+    outside |= split_rows<D>(Vb + krow, key < T, g, f);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      vf[c][0] = f[c].part[0];
+      vf[c][1] = f[c].part[1];
+      s_low[wave][1][c][lane] = f[c].part[2];
+    }
   }
+  FragOffsets<D> fo;
+  fo.init(lane);
   f32x16 dk[DB], dv[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
@@ -247,145 +259,181 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(BwdArgs a) {
   const int total_steps = n_qt_tiles > 0 ? n_qt_tiles * a.group : 0;
 
   // A step is (head in group, query tile); tiles no document can see are
-  // skipped when positions are given.
-  auto tile_visible = [&](int qt) -> bool {
-    if (clb == nullptr) return true;
-    const int c0 = (qt * BQ) / 32;
-    int lo = clb[2 * c0];
-#pragma unroll
-    for (int c = 1; c < BQ / 32; ++c)
-      if (c0 + c < nchunks) lo = min(lo, clb[2 * (c0 + c)]);
-    return lo <= k1;
-  };
+  // skipped when positions are given (a tile is one chunk of the bounds).
   auto next_step = [&](int st) -> int {
-    while (st < total_steps && !tile_visible(qt_begin + st % n_qt_tiles)) ++st;
+    while (clb != nullptr && st < total_steps && clb[2 * (qt_begin + st % n_qt_tiles)] > k1) ++st;
     return st;
   };
 
-  TileStage<E, D, BQ> qst, ost;
-  auto stage_load = [&](int st) {
-    const int h = kvh * a.group + st / n_qt_tiles;
-    const int q0 = (qt_begin + st % n_qt_tiles) * BQ;
-    const E* Qb = static_cast<const E*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
-    const E* Ob = static_cast<const E*>(a.dO) + ((int64_t)b * T * a.H + h) * D;
-    qst.load(Qb, qpitch, q0, T, tid);
-    ost.load(Ob, qpitch, q0, T, tid);
+  SplitStage<D> qst, ost;
+  float r_lse, r_delta;
+  int r_lb;
+  auto head_of = [&](int st) { return ((int64_t)b * T * a.H + kvh * a.group + st / n_qt_tiles) * D; };
+  auto q0_of = [&](int st) { return (qt_begin + st % n_qt_tiles) * BQ; };
+  auto load_q = [&](int st) {
+    qst.load(static_cast<const float*>(a.Q) + head_of(st), qpitch, q0_of(st), T, tid);
+    const int q = q0_of(st) + (tid & (BQ - 1));
+    const int64_t si = ((int64_t)b * a.H + kvh * a.group + st / n_qt_tiles) * T + min(q, T - 1);
+    r_lse = q < T ? a.lse2[si] : INFINITY;
+    r_delta = q < T ? a.delta[si] : 0.0f;
+    r_lb = key_lb(q, T, a.left, pos);
   };
-  auto stage_store = [&](int st, int buf) {
-    const int h = kvh * a.group + st / n_qt_tiles;
-    const int q0 = (qt_begin + st % n_qt_tiles) * BQ;
-    E* base = smem + buf * C::kStage;
-    qst.store_nat(base, C::kLD, tid);
-    ost.store_nat(base + C::kNat, C::kLD, tid);
-    if constexpr (C::kBF) {
-      qst.store_tr(base + 2 * C::kNat, C::kLDT, tid);
-      ost.store_tr(base + 2 * C::kNat + C::kTr, C::kLDT, tid);
-    }
+  auto load_o = [&](int st) { ost.load(static_cast<const float*>(a.dO) + head_of(st), qpitch, q0_of(st), T, tid); };
+  auto store_rows = [&](int buf) {
     if (tid < BQ) {
-      const int q = q0 + tid;
-      const int64_t si = ((int64_t)b * a.H + h) * T + q;
-      s_lse[buf][tid] = q < T ? a.lse2[si] : INFINITY;
-      s_delta[buf][tid] = q < T ? a.delta[si] : 0.0f;
-      s_lb[buf][tid] = key_lb(q, T, a.left, pos);
+      s_lse[buf][tid] = r_lse;
+      s_delta[buf][tid] = r_delta;
+      s_lb[buf][tid] = r_lb;
     }
   };
 
-  int st = next_step(0);
-  if (st < total_steps) {
-    stage_load(st);
-    stage_store(st, 0);
-  }
-  int buf = 0;
-  while (st < total_steps) {
-    const int st_next = next_step(st + 1);
-    const bool more = st_next < total_steps;
-    if (more) stage_load(st_next);
-    __syncthreads();
-
-    const int q0 = (qt_begin + st % n_qt_tiles) * BQ;
-    const E* Qs = smem + buf * C::kStage;
-    const E* Os = Qs + C::kNat;
-    const int* lbs = s_lb[buf];
-    // Tile bounds on the key range of its queries (queries >= T have lb = T).
-    int lbmin = lbs[0], lbmax = lbs[0];
-    {
-      const int v = lane < BQ ? lbs[lane] : lbs[0];
-      lbmin = wave_min64(v);
-      lbmax = wave_max64(v);
+  // P of a tile in place of the scores, dS in place of dP.
+  auto softmax = [&](auto need_mask, f32x16& s, f32x16& dp, int q0, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i0 = 8 * j + 4 * g;
+      const f32x4 L = *reinterpret_cast<const f32x4*>(&s_lse[buf][i0]);
+      const f32x4 Dl = *reinterpret_cast<const f32x4*>(&s_delta[buf][i0]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 4 * j + t;
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -L[t]));
+        float ds = p * (dp[r] - Dl[t]);
+        if constexpr (decltype(need_mask)::value) {
+          const int lbq = s_lb[buf][i0 + t], ubq = key_ub(q0 + i0 + t, T, a.right);
+          const bool vis = (key >= lbq) & (key <= ubq);
+          p = vis ? p : 0.0f;
+          ds = vis & (ubq > lbq) ? ds : 0.0f;
+        }
+        s[r] = p;
+        dp[r] = ds;
+      }
     }
-    const int ubmin = q0 + BQ - 1 >= T ? -1 : key_ub(q0, T, a.right);  // ub is monotone in q
+  };
+
+  // The tile's rows (staged) times this wave's keys (kf or vf), even and odd
+  // chunks summed apart.
+  auto product = [&](const char* tile, const bf16x8 (&f)[KC][2], int which) __attribute__((always_inline)) {
+    auto keys = [&](int c) { return Split8{{f[c][0], f[c][1], s_low[wave][which][c][lane]}}; };
+    f32x16 even = zero16(), odd = zero16();
+    if constexpr (KC == 1) return mma_split(split_nat<D>(tile, fo, 0), keys(0), even);
+#pragma unroll
+    for (int c = 0; c + 1 < KC; c += 2)
+      mma_split_pair(split_nat<D>(tile, fo, c), keys(c), even, split_nat<D>(tile, fo, c + 1), keys(c + 1), odd);
+    return even + odd;
+  };
+
+  int st = next_step(0), st_next = total_steps;
+  if (st < total_steps) {
+    load_q(st);
+    load_o(st);
+    outside |= qst.store(Qbuf[0], tid);
+    store_rows(0);
+    st_next = next_step(st + 1);
+  }
+  __syncthreads();
+  int buf = 0;
+  // A step: S while this tile's dO is split and stored (all waves are done with
+  // the previous one), a barrier, then dP, P and dS, dV and dK while the next
+  // tile's Q is.  With no next tile, rows of the slice go to the idle buffer.
+  while (st < total_steps) {
+    const bool more = st_next < total_steps;
+    const int q0 = q0_of(st);
+    const char* Qs = Qbuf[buf];
+    // The tile's bounds on its queries' key ranges (queries >= T have lb = T,
+    // ub = -1); without positions both are monotone in the query.
+    int lbmin, lbmax;
+    if (clb != nullptr) {
+      lbmin = clb[2 * (q0 / BQ)];
+      lbmax = clb[2 * (q0 / BQ) + 1];
+    } else {
+      lbmin = key_lb(q0, T, a.left, nullptr);
+      lbmax = key_lb(q0 + BQ - 1, T, a.left, nullptr);
+    }
+    const int ubmin = q0 + BQ - 1 >= T ? -1 : key_ub(q0, T, a.right);
     const int ubmax = key_ub(min(q0 + BQ - 1, T - 1), T, a.right);
     const bool active = !(lbmin > kw1 || ubmax < kw0);
+    f32x16 s = zero16();
     if (active) {
-      f32x16 s[NQB], dp[NQB];
-#pragma unroll
-      for (int qb = 0; qb < NQB; ++qb) {
-        s[qb] = zero16();
-        dp[qb] = zero16();
-      }
-#pragma unroll
-      for (int c = 0; c < KC; ++c) {
-#pragma unroll
-        for (int qb = 0; qb < NQB; ++qb) {
-          const auto qfrag = M::load8(Qs + (32 * qb + l32) * C::kLD + 16 * c + 8 * g);
-          s[qb] = M::mma(qfrag, kf[c], s[qb]);
-          const auto ofrag = M::load8(Os + (32 * qb + l32) * C::kLD + 16 * c + 8 * g);
-          dp[qb] = M::mma(ofrag, vf[c], dp[qb]);
-        }
-      }
-      const bool need_mask = !(lbmax <= kw0 && kw1 <= ubmin);
-#pragma unroll
-      for (int qb = 0; qb < NQB; ++qb) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i0 = 32 * qb + 8 * j + 4 * g;
-          const f32x4 L = *reinterpret_cast<const f32x4*>(&s_lse[buf][i0]);
-          const f32x4 Dl = *reinterpret_cast<const f32x4*>(&s_delta[buf][i0]);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const int r = 4 * j + t;
-            float p = __builtin_amdgcn_exp2f(s[qb][r] * a.scale_log2 - L[t]);
-            float ds = p * (dp[qb][r] - Dl[t]);
-            if (need_mask) {
-              const int qq = q0 + i0 + t;
-              const int lbq = lbs[i0 + t];
-              const int ubq = key_ub(qq, T, a.right);
-              const bool vis = key >= lbq && key <= ubq;
-              p = vis ? p : 0.0f;
-              ds = (vis && ubq > lbq) ? ds : 0.0f;
-            }
-            s[qb][r] = p;
-            dp[qb][r] = ds;
-          }
-        }
-      }
+      s = product(Qs, kf, 0);
+      outside |= ost.store(Os, tid);
+    } else {
+      outside |= ost.store(Os, tid);
+    }
+    load_q(more ? st_next : st);
+    load_o(more ? st_next : st);
+    __syncthreads();
+    if (active) {
+      f32x16 dp = product(Os, vf, 1);
+      if (!(lbmax <= kw0 && kw1 <= ubmin)) softmax(std::true_type{}, s, dp, q0, buf);
+      else softmax(std::false_type{}, s, dp, q0, buf);
+      outside |= !(max_abs16(dp) < kSplitMax);
       // dV += P^T dO, dK += dS^T Q  (k = query, accumulator order)
-      const E* Qt = Qs + 2 * C::kNat;
-      const E* Ot = Qt + C::kTr;
 #pragma unroll
-      for (int kc = 0; kc < BQ / 16; ++kc) {
-        const auto pf = (kc & 1) ? M::template from_acc<1>(s[kc >> 1]) : M::template from_acc<0>(s[kc >> 1]);
-        const auto sf = (kc & 1) ? M::template from_acc<1>(dp[kc >> 1]) : M::template from_acc<0>(dp[kc >> 1]);
+      for (int kc = 0; kc < 2; ++kc) {
+        const Split8 pf = kc ? split_acc<1>(s) : split_acc<0>(s);
+        const Split8 sf = kc ? split_acc<1>(dp) : split_acc<0>(dp);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+          mma_split_pair(pf, split_tr<D>(Os, fo, kc, db), dv[db], sf, split_tr<D>(Qs, fo, kc, db), dk[db]);
+      }
+      outside |= qst.store(Qbuf[buf ^ 1], tid);
+    } else {
+      outside |= qst.store(Qbuf[buf ^ 1], tid);
+    }
+    store_rows(buf ^ 1);
+    st = st_next;
+    if (more) st_next = next_step(st + 1);
+    buf ^= 1;
+    __syncthreads();
+  }
+
+  if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
+  __syncthreads();
+  if (s_outside != 0) {
+    // fp32 MFMA from global memory.
+    using M = Mma<float>;
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      dk[i] = zero16();
+      dv[i] = zero16();
+    }
+    for (int step = next_step(0); step < total_steps; step = next_step(step + 1)) {
+      const int h = kvh * a.group + step / n_qt_tiles;
+      const int q0 = (qt_begin + step % n_qt_tiles) * BQ;
+      const float* Qb = static_cast<const float*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
+      const float* Ob = static_cast<const float*>(a.dO) + ((int64_t)b * T * a.H + h) * D;
+      __syncthreads();
+      if (tid < BQ) {
+        const int q = q0 + tid;
+        const int64_t si = ((int64_t)b * a.H + h) * T + min(q, T - 1);
+        s_lse[0][tid] = q < T ? a.lse2[si] : INFINITY;
+        s_delta[0][tid] = q < T ? a.delta[si] : 0.0f;
+        s_lb[0][tid] = key_lb(q, T, a.left, pos);
+      }
+      __syncthreads();
+      f32x16 s = zero16(), dp = zero16();
+      const int64_t qrow = (int64_t)min(q0 + l32, T - 1) * qpitch;
+      for (int c = 0; c < KC; ++c) {
+        const int at = 16 * c + 8 * g;
+        s = M::mma(M::load8(Qb + qrow + at), key < T ? M::load8(Kb + krow + at) : M::zero(), s);
+        dp = M::mma(M::load8(Ob + qrow + at), key < T ? M::load8(Vb + krow + at) : M::zero(), dp);
+      }
+      softmax(std::true_type{}, s, dp, q0, 0);
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+        const f32x8 pf = kc ? M::from_acc<1>(s) : M::from_acc<0>(s);
+        const f32x8 sf = kc ? M::from_acc<1>(dp) : M::from_acc<0>(dp);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          typename M::frag of, qfr;
-          if constexpr (C::kBF) {
-            of = load_tr_bf16(Ot + (32 * db + l32) * C::kLDT + 16 * kc, g);
-            qfr = load_tr_bf16(Qt + (32 * db + l32) * C::kLDT + 16 * kc, g);
-          } else {
-            const int col = D < 32 ? min(32 * db + l32, D - 1) : 32 * db + l32;
-            of = load_kt_f32(Os + 16 * kc * C::kLD + col, C::kLD, g);
-            qfr = load_kt_f32(Qs + 16 * kc * C::kLD + col, C::kLD, g);
-          }
+          f32x8 of, qf;
+          load_rows_f32<D>(Ob, qpitch, q0 + 16 * kc, T, 32 * db + l32, g, of);
+          load_rows_f32<D>(Qb, qpitch, q0 + 16 * kc, T, 32 * db + l32, g, qf);
           dv[db] = M::mma(pf, of, dv[db]);
-          dk[db] = M::mma(sf, qfr, dk[db]);
+          dk[db] = M::mma(sf, qf, dk[db]);
         }
       }
     }
-
-    if (more) stage_store(st_next, buf ^ 1);
-    buf ^= 1;
-    st = st_next;
   }
 
   // Store: accumulator row = key, column = head-dim index.
@@ -399,25 +447,14 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(BwdArgs a) {
         if (kk < T) {
           const int64_t off = ((int64_t)b * T + kk) * kpitch + (int64_t)kvh * D + d;
           float vk = dk[db][r] * a.scale, vv = dv[db][r];
-          if (a.grad_bf16) {
-            bf16* pk = static_cast<bf16*>(a.dK) + off;
-            bf16* pv = static_cast<bf16*>(a.dV) + off;
-            if (a.accumulate) {
-              vk += to_f32(*pk);
-              vv += to_f32(*pv);
-            }
-            *pk = static_cast<bf16>(vk);
-            *pv = static_cast<bf16>(vv);
-          } else {
-            float* pk = static_cast<float*>(a.dK) + off;
-            float* pv = static_cast<float*>(a.dV) + off;
-            if (a.accumulate) {
-              vk += *pk;
-              vv += *pv;
-            }
-            *pk = vk;
-            *pv = vv;
+          float* pk = static_cast<float*>(a.dK) + off;
+          float* pv = static_cast<float*>(a.dV) + off;
+          if (a.accumulate) {
+            vk += *pk;
+            vv += *pv;
           }
+          *pk = vk;
+          *pv = vv;
         }
       }
     }
@@ -425,33 +462,26 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename E, int D>
-struct DqCfg {
-  static constexpr bool kBF = std::is_same<E, bf16>::value;
-  static constexpr int kBM = 128;             // queries per workgroup
-  static constexpr int kBN = kBF ? 64 : 32;   // keys per tile
-  static constexpr int kKC = D / 16;
-  static constexpr int kDP = D < 32 ? 32 : D;
-  static constexpr int kDB = kDP / 32;
-  static constexpr int kLD = kBF ? D + 8 : D + 4;
-  static constexpr int kLDT = kBN + 4;
-  static constexpr int kNat = kBN * kLD;
-  static constexpr int kTr = kBF ? kDP * kLDT : 0;
-  static constexpr int kStage = 2 * kNat + kTr;  // K, V natural + K^T
-};
-
-template <typename E, int D>
-__global__ __launch_bounds__(kThreads, 1) void attn_bwd_dq_kernel(BwdArgs a) {
-  using M = Mma<E>;
-  using C = DqCfg<E, D>;
-  constexpr int BN = C::kBN, KC = C::kKC, DB = C::kDB, NKB = BN / 32;
-  __shared__ __attribute__((aligned(16))) E smem[2 * C::kStage];
+// dQ, exact mode: 128 queries of one (batch, head) per workgroup, 32 per wave
+// with Q and dO resident in parts; S^T and dP^T are recomputed with the query
+// as the lane index, so dS^T is directly the B operand of dQ^T += K^T dS^T.
+// K and V tiles of 32 keys are split once per workgroup into double-buffered
+// LDS, a tile ahead.  8 x 2048 tokens, causal, H6 D128: 500 us (fp32 MFMA
+// 782-798), H12 D64: 394 (769).  Loading a further tile ahead, alternating
+// products of two sums and fixed orders of reads and products measured within
+// 3% (slower at D = 64, where they spill).
+template <int D>
+__global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_kernel(BwdArgs a) {
+  constexpr int BN = kExactBT, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  constexpr int kTile = SplitTile<D>::kBytes, kBM = 128;
+  __shared__ __attribute__((aligned(1024))) char bufs[2][2 * kTile];  // K, V
   __shared__ int s_bounds[2][kWaves];
+  __shared__ int s_outside;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 5, l32 = lane & 31;
   const int T = a.T;
-  const int n_qt = (T + C::kBM - 1) / C::kBM;
+  const int n_qt = (T + kBM - 1) / kBM;
   const GridItem it0 = heavy_first(blockIdx.x, a.H * a.B);
   const int qt = n_qt - 1 - it0.rank;  // longest query tiles first, over the whole grid
   int b, h;
@@ -459,31 +489,31 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dq_kernel(BwdArgs a) {
   const int kvh = h / a.group;
 
   const int64_t qpitch = (int64_t)a.H * D, kpitch = (int64_t)a.Hkv * D;
-  const E* Qb = static_cast<const E*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
-  const E* Ob = static_cast<const E*>(a.dO) + ((int64_t)b * T * a.H + h) * D;
-  const E* Kb = static_cast<const E*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
-  const E* Vb = static_cast<const E*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Qb = static_cast<const float*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
+  const float* Ob = static_cast<const float*>(a.dO) + ((int64_t)b * T * a.H + h) * D;
+  const float* Kb = static_cast<const float*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Vb = static_cast<const float*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
   const int32_t* pos = a.pos ? a.pos + (int64_t)b * T : nullptr;
 
-  const int q = qt * C::kBM + wave * 32 + l32;
+  const int q = qt * kBM + wave * 32 + l32;
   const int lb = key_lb(q, T, a.left, pos), ub = key_ub(q, T, a.right);
   const bool multiple = ub > lb;
-  const int wlb_min = wave_min32(lb), wlb_max = wave_max32(lb);
-  const int wub_min = wave_min32(ub), wub_max = wave_max32(ub);
+  const int wlb_min = __builtin_amdgcn_readfirstlane(wave_min32(lb)), wlb_max = __builtin_amdgcn_readfirstlane(wave_max32(lb));
+  const int wub_min = __builtin_amdgcn_readfirstlane(wave_min32(ub)), wub_max = __builtin_amdgcn_readfirstlane(wave_max32(ub));
   if (lane == 0) {
     s_bounds[0][wave] = wlb_min;
     s_bounds[1][wave] = wub_max;
   }
-  const int64_t si = ((int64_t)b * a.H + h) * T + q;
+  if (tid == 0) s_outside = 0;
+  const int64_t si = ((int64_t)b * a.H + h) * T + min(q, T - 1);
   const float lse = q < T ? a.lse2[si] : INFINITY;
   const float dlt = q < T ? a.delta[si] : 0.0f;
 
-  typename M::frag qf[KC], of[KC];
-#pragma unroll
-  for (int c = 0; c < KC; ++c) {
-    qf[c] = q < T ? M::load8(Qb + (int64_t)q * qpitch + 16 * c + 8 * g) : M::zero();
-    of[c] = q < T ? M::load8(Ob + (int64_t)q * qpitch + 16 * c + 8 * g) : M::zero();
-  }
+  Split8 qf[KC], of[KC];
+  const int64_t qrow = (int64_t)min(q, T - 1) * qpitch;
+  bool outside = split_rows<D>(Qb + qrow, q < T, g, qf) | split_rows<D>(Ob + qrow, q < T, g, of);
+  FragOffsets<D> fo;
+  fo.init(lane);
   f32x16 dq[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) dq[i] = zero16();
@@ -495,79 +525,104 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dq_kernel(BwdArgs a) {
     kmin = min(kmin, s_bounds[0][w]);
     kmax = max(kmax, s_bounds[1][w]);
   }
-  const int kt0 = (kmin / BN) * BN;
-  const int ntiles = kmax >= kmin ? (kmax - kt0) / BN + 1 : 0;
+  const int kt0 = __builtin_amdgcn_readfirstlane((kmin / BN) * BN);
+  const int ntiles = __builtin_amdgcn_readfirstlane(kmax >= kmin ? (kmax - (kmin / BN) * BN) / BN + 1 : 0);
 
-  TileStage<E, D, BN> kst, vst;
-  auto store_stage = [&](int buf) {
-    E* base = smem + buf * C::kStage;
-    kst.store_nat(base, C::kLD, tid);
-    vst.store_nat(base + C::kNat, C::kLD, tid);
-    if constexpr (C::kBF) kst.store_tr(base + 2 * C::kNat, C::kLDT, tid);
+  // dS of a tile into dp.
+  auto softmax = [&](auto need_mask, const f32x16& s, f32x16& dp, int kt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -lse));
+      const float ds = p * (dp[r] - dlt);
+      if constexpr (decltype(need_mask)::value) {
+        const int kk = kt + acc_row(r, g);
+        dp[r] = ((kk >= lb) & (kk <= ub) & multiple) ? ds : 0.0f;
+      } else {
+        dp[r] = ds;
+      }
+    }
+  };
+
+  SplitStage<D> kst, vst;
+  // One tile: the next tile's K is split and stored between S and dP, its V
+  // between dP and dQ (past the last tile, rows of the slice go to the idle
+  // buffer); a mask is a uniform branch of its own, so that one copy of the
+  // products serves all tiles.
+  auto body = [&](int kt, int buf, bool more, bool need_mask) __attribute__((always_inline)) {
+    const char* Ks = bufs[buf];
+    const char* Vs = Ks + kTile;
+    char* next = bufs[buf ^ 1];
+    f32x16 s = zero16(), dp = zero16();
+    vst.load(Vb, kpitch, kt + BN, T, tid);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) s = mma_split(split_nat<D>(Ks, fo, c), qf[c], s);
+    bool out = kst.store(next, tid);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) dp = mma_split(split_nat<D>(Vs, fo, c), of[c], dp);
+    out |= vst.store(next + kTile, tid);
+    __builtin_amdgcn_sched_barrier(0);
+    if (need_mask) softmax(std::true_type{}, s, dp, kt);
+    else softmax(std::false_type{}, s, dp, kt);
+    outside |= !(max_abs16(dp) < kSplitMax);
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const Split8 sf = kc ? split_acc<1>(dp) : split_acc<0>(dp);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) dq[db] = mma_split(split_tr<D>(Ks, fo, kc, db), sf, dq[db]);
+    }
+    outside |= out & more;
   };
   if (ntiles > 0) {
     kst.load(Kb, kpitch, kt0, T, tid);
     vst.load(Vb, kpitch, kt0, T, tid);
-    store_stage(0);
+    outside |= kst.store(bufs[0], tid) | vst.store(bufs[0] + kTile, tid);
+    kst.load(Kb, kpitch, kt0 + BN, T, tid);
   }
+  __syncthreads();
   for (int it = 0; it < ntiles; ++it) {
     const int kt = kt0 + it * BN;
-    const E* Ks = smem + (it & 1) * C::kStage;
-    const E* Vs = Ks + C::kNat;
-    const E* Kt = Vs + C::kNat;
     const bool more = it + 1 < ntiles;
-    if (more) {
-      kst.load(Kb, kpitch, kt + BN, T, tid);
+    if (wlb_min > kt + BN - 1 || wub_max < kt) {
       vst.load(Vb, kpitch, kt + BN, T, tid);
+      char* next = bufs[(it + 1) & 1];
+      const bool out = kst.store(next, tid) | vst.store(next + kTile, tid);
+      outside |= out & more;
+    } else {
+      body(kt, it & 1, more, !(wlb_max <= kt && kt + BN - 1 <= wub_min));
     }
+    kst.load(Kb, kpitch, kt + 2 * BN, T, tid);
     __syncthreads();
+  }
 
-    const bool active = !(wlb_min > kt + BN - 1 || wub_max < kt);
-    if (active) {
-      f32x16 s[NKB], dp[NKB];
+  if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
+  __syncthreads();
+  if (s_outside != 0) {
+    // fp32 MFMA from global memory.
+    using M = Mma<float>;
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        s[kb] = zero16();
-        dp[kb] = zero16();
-      }
-#pragma unroll
+    for (int i = 0; i < DB; ++i) dq[i] = zero16();
+#pragma unroll 1
+    for (int kt = (wlb_min / BN) * BN; kt <= wub_max; kt += BN) {
+      f32x16 s = zero16(), dp = zero16();
+      const int64_t krow = (int64_t)min(kt + l32, T - 1) * kpitch;
       for (int c = 0; c < KC; ++c) {
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-          const auto kfrag = M::load8(Ks + (32 * kb + l32) * C::kLD + 16 * c + 8 * g);
-          s[kb] = M::mma(kfrag, qf[c], s[kb]);
-          const auto vfrag = M::load8(Vs + (32 * kb + l32) * C::kLD + 16 * c + 8 * g);
-          dp[kb] = M::mma(vfrag, of[c], dp[kb]);
-        }
+        const int at = 16 * c + 8 * g;
+        s = M::mma(M::load8(Kb + krow + at), q < T ? M::load8(Qb + qrow + at) : M::zero(), s);
+        dp = M::mma(M::load8(Vb + krow + at), q < T ? M::load8(Ob + qrow + at) : M::zero(), dp);
       }
-      const bool need_mask = !(wlb_max <= kt && kt + BN - 1 <= wub_min);
+      softmax(std::true_type{}, s, dp, kt);
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(s[kb][r] * a.scale_log2 - lse);
-          float ds = p * (dp[kb][r] - dlt);
-          if (need_mask) {
-            const int kk = kt + 32 * kb + acc_row(r, g);
-            const bool vis = kk >= lb && kk <= ub;
-            ds = (vis && multiple) ? ds : 0.0f;
-          }
-          dp[kb][r] = ds;
-        }
-      }
-#pragma unroll
-      for (int kc = 0; kc < BN / 16; ++kc) {
-        const auto sf = (kc & 1) ? M::template from_acc<1>(dp[kc >> 1]) : M::template from_acc<0>(dp[kc >> 1]);
+      for (int kc = 0; kc < 2; ++kc) {
+        const f32x8 sf = kc ? M::from_acc<1>(dp) : M::from_acc<0>(dp);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          typename M::frag kfr;
-          if constexpr (C::kBF) kfr = load_tr_bf16(Kt + (32 * db + l32) * C::kLDT + 16 * kc, g);
-          else kfr = load_kt_f32(Ks + 16 * kc * C::kLD + (D < 32 ? min(32 * db + l32, D - 1) : 32 * db + l32), C::kLD, g);
+          f32x8 kfr;
+          load_rows_f32<D>(Kb, kpitch, kt + 16 * kc, T, 32 * db + l32, g, kfr);
           dq[db] = M::mma(kfr, sf, dq[db]);
         }
       }
     }
-    if (more) store_stage((it + 1) & 1);
   }
 
   if (q < T) {
@@ -581,8 +636,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dq_kernel(BwdArgs a) {
           f32x4 v;
 #pragma unroll
           for (int t = 0; t < 4; ++t) v[t] = dq[db][4 * j + t] * a.scale;
-          if (a.grad_bf16) store4(static_cast<bf16*>(a.dQ) + orow * D + d0, v, a.accumulate);
-          else store4(static_cast<float*>(a.dQ) + orow * D + d0, v, a.accumulate);
+          store4(static_cast<float*>(a.dQ) + orow * D + d0, v, a.accumulate);
         }
       }
     }
@@ -640,45 +694,45 @@ hipError_t launch_order(const Problem& p, const OrderArgs& a, hipStream_t s) {
   return e;
 }
 
-template <typename E, int D>
-static hipError_t launch_dkdv_t(const Problem& p, const BwdArgs& a, hipStream_t s) {
-  const int n_kt = (p.T + DkdvCfg<E, D>::kBK - 1) / DkdvCfg<E, D>::kBK;
+template <int D>
+static hipError_t launch_dkdv_exact(const Problem& p, const BwdArgs& a, hipStream_t s) {
+  const int n_kt = (p.T + kExactBK - 1) / kExactBK;
   const dim3 grid(n_kt * p.Hkv * p.B), block(kThreads);
   const ProfileMark mk = profile_begin(s);
-  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<E, D>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((attn_bwd_dkdv_exact_kernel<D>), grid, block, 0, s, a);
   const hipError_t e = hipGetLastError();
-  profile_end(mk, p.bf16 ? "attn_bwd_dkdv_bf16" : "attn_bwd_dkdv_f32", s);
+  profile_end(mk, "attn_bwd_dkdv_f32", s);
   return e;
 }
 
-template <typename E, int D>
-static hipError_t launch_dq_t(const Problem& p, const BwdArgs& a, hipStream_t s) {
-  const int n_qt = (p.T + DqCfg<E, D>::kBM - 1) / DqCfg<E, D>::kBM;
+template <int D>
+static hipError_t launch_dq_exact(const Problem& p, const BwdArgs& a, hipStream_t s) {
+  const int n_qt = (p.T + 127) / 128;
   const dim3 grid(n_qt * p.H * p.B), block(kThreads);
   const ProfileMark mk = profile_begin(s);
-  hipLaunchKernelGGL((attn_bwd_dq_kernel<E, D>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((attn_bwd_dq_exact_kernel<D>), grid, block, 0, s, a);
   const hipError_t e = hipGetLastError();
-  profile_end(mk, p.bf16 ? "attn_bwd_dq_bf16" : "attn_bwd_dq_f32", s);
+  profile_end(mk, "attn_bwd_dq_f32", s);
   return e;
 }
 
-#define FC_DISPATCH_D(FN, E)                       \
-  switch (p.Dk) {                                   \
-    case 16: return FN<E, 16>(p, a, s);            \
-    case 32: return FN<E, 32>(p, a, s);            \
-    case 64: return FN<E, 64>(p, a, s);            \
-    case 128: return FN<E, 128>(p, a, s);          \
+#define FC_DISPATCH_D(FN)                          \
+  switch (p.Dk) {                                  \
+    case 16: return FN<16>(p, a, s);               \
+    case 32: return FN<32>(p, a, s);               \
+    case 64: return FN<64>(p, a, s);               \
+    case 128: return FN<128>(p, a, s);             \
     default: return hipErrorInvalidValue;          \
   }
 
 hipError_t launch_bwd_dkdv(const Problem& p, const BwdArgs& a, hipStream_t s) {
   if (p.bf16) return launch_bwd_dkdv_fast(p, a, s);
-  FC_DISPATCH_D(launch_dkdv_t, float)
+  FC_DISPATCH_D(launch_dkdv_exact)
 }
 
 hipError_t launch_bwd_dq(const Problem& p, const BwdArgs& a, hipStream_t s) {
   if (p.bf16) return launch_bwd_dq_fast(p, a, s);
-  FC_DISPATCH_D(launch_dq_t, float)
+  FC_DISPATCH_D(launch_dq_exact)
 }
 
 }  // namespace fc

@@ -1,57 +1,68 @@
-// Flash-attention forward for gfx950.
+// Flash-attention forward, exact mode (fp32 in and out), gfx950.
 //
 // Behaviour follows the reference forward (src/kernels.jl:131-219 for the
-// semantics of O, l and m; ext/FemtoChatCUDAExt.jl:1295-1463 for the fast
-// mode: fp32 statistics, P rounded to the input format before P.V, l summed
-// from the unrounded probabilities).  The design is this file's own:
+// semantics of O, l and m).  The design is this file's own:
 //
-//  * one workgroup = 4 waves x 32 queries of one (batch, head); the grid is
-//    spread over the 8 XCDs so that the query tiles of one head share an L2;
-//  * each wave computes S^T = K Q^T (keys x queries) with 32x32 MFMA, so a
-//    lane owns one query column: the online softmax needs one cross-lane
-//    exchange (lane l <-> l^32) per key tile and the probabilities are already
-//    the B operand of O^T += V^T P^T;
-//  * K is staged in LDS in natural layout, V transposed (bf16) so that the
-//    V^T operand is two 8-byte LDS reads per fragment; both double-buffered
-//    with register prefetch, one barrier per key tile;
+//  * one workgroup = 4 waves x 32 queries of one (batch, head), two workgroups
+//    per CU; the grid takes the longest query tiles first;
+//  * every product runs as six bf16 products of the operands' three parts
+//    (attn_exact.hpp); Q stays in registers in parts, K and V tiles of 32 keys
+//    are split once per workgroup as they are staged in swizzled LDS;
+//  * each wave computes S^T = K Q^T (keys x queries), so a lane owns one query
+//    column: the softmax needs one exchange between half-waves per key tile and
+//    the probabilities are already the B operand of O^T += V^T P^T;
+//  * K and V are single-buffered: while the S products read K, the V tile is
+//    split and stored; while the P V products read V, the next K tile is, each
+//    loaded a phase ahead (16 registers per thread in flight);
+//  * the exponent reference of a row is the maximum of the first tile in which
+//    it sees a key and never moves (as in the fast kernel: O is not rescaled),
+//    and a row that outgrows it by 2^64 is recomputed;
 //  * key tiles outside [min lb, max ub] of the workgroup are never visited,
 //    fully visible tiles skip the mask, and waves with no visible key in a
 //    tile skip its products.
-#include "attn_device.hpp"
+//
+// Bound by the matrix cores and, next to them, by LDS (48 KB of parts read per
+// wave and tile for 96 products): 8 x 2048 tokens, causal, H6 D128 in 303 us
+// (1.02 PFLOP/s of bf16 products; 475 us with fp32 MFMA), H12 D64 in 296 (523).
+#include "attn_exact.hpp"
 #include "attn_launch.hpp"
 
 #include <type_traits>
 
 namespace fc {
 
-template <typename E, int D>
-struct FwdCfg {
-  static constexpr bool kBF = std::is_same<E, bf16>::value;
-  static constexpr int kBM = 128;                // queries per workgroup
-  static constexpr int kBN = kBF ? 64 : 32;      // keys per tile
-  static constexpr int kKC = D / 16;             // 16-wide head-dim chunks
-  static constexpr int kDP = D < 32 ? 32 : D;    // head dim padded to 32
-  static constexpr int kDB = kDP / 32;           // 32-wide head-dim blocks
-  static constexpr int kLDK = kBF ? D + 8 : D + 4;   // K row stride
-  static constexpr int kLDVT = kBN + 4;              // V^T row stride (bf16)
-  static constexpr int kLDV = D + 4;                 // V row stride (fp32)
-  static constexpr int kKElems = kBN * kLDK;
-  static constexpr int kVElems = kBF ? kDP * kLDVT : kBN * kLDV;
-  static constexpr int kStage = kKElems + kVElems;
-};
+constexpr int kExactBM = 128;  // queries per workgroup
+constexpr int kExactBN = 32;   // keys per tile
+constexpr float kExactGrowth = 64.0f;  // log2 units above the reference that send a row to the recomputation
 
-template <typename E, int D>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(FwdArgs a) {
-  using M = Mma<E>;
-  using C = FwdCfg<E, D>;
-  constexpr int BN = C::kBN, KC = C::kKC, DB = C::kDB, NKB = BN / 32;
-  __shared__ __attribute__((aligned(16))) E smem[2 * C::kStage];
+// S^T of 32 keys from k0 in fp32 MFMA, K straight from global memory, masked.
+template <int D>
+__device__ inline f32x16 exact_scores(const float* Kb, int64_t kpitch, const f32x8 (&qf)[D / 16], int k0, int T, int l32,
+                                      int g, int lb, int ub) {
+  using M = Mma<float>;
+  f32x16 s = zero16();
+  const float* row = Kb + (int64_t)min(k0 + l32, T - 1) * kpitch;
+  for (int c = 0; c < D / 16; ++c) s = M::mma(M::load8(row + 16 * c + 8 * g), qf[c], s);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int key = k0 + acc_row(r, g);
+    if (key < lb || key > ub) s[r] = -INFINITY;
+  }
+  return s;
+}
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) {
+  constexpr int BN = kExactBN, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  __shared__ __attribute__((aligned(1024))) char Ks[SplitTile<D>::kBytes];
+  __shared__ __attribute__((aligned(1024))) char Vs[SplitTile<D>::kBytes];
   __shared__ int s_bounds[2][kWaves];
+  __shared__ int s_outside;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 5, l32 = lane & 31;
   const int T = a.T;
-  const int n_qt = (T + C::kBM - 1) / C::kBM;
+  const int n_qt = (T + kExactBM - 1) / kExactBM;
   const GridItem it0 = heavy_first(blockIdx.x, a.H * a.B);
   const int qt = n_qt - 1 - it0.rank;  // longest query tiles first, over the whole grid
   int b, h;
@@ -59,29 +70,31 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(FwdArgs a) {
   const int kvh = h / a.group;
 
   const int64_t qpitch = (int64_t)a.H * D, kpitch = (int64_t)a.Hkv * D;
-  const E* Qb = static_cast<const E*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
-  const E* Kb = static_cast<const E*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
-  const E* Vb = static_cast<const E*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Qb = static_cast<const float*>(a.Q) + ((int64_t)b * T * a.H + h) * D;
+  const float* Kb = static_cast<const float*>(a.K) + ((int64_t)b * T * a.Hkv + kvh) * D;
+  const float* Vb = static_cast<const float*>(a.V) + ((int64_t)b * T * a.Hkv + kvh) * D;
   const int32_t* pos = a.pos ? a.pos + (int64_t)b * T : nullptr;
 
-  const int q = qt * C::kBM + wave * 32 + l32;
+  const int q = qt * kExactBM + wave * 32 + l32;
   const int lb = key_lb(q, T, a.left, pos), ub = key_ub(q, T, a.right);
-  const int wlb_min = wave_min32(lb), wlb_max = wave_max32(lb);
-  const int wub_min = wave_min32(ub), wub_max = wave_max32(ub);
+  const int wlb_min = __builtin_amdgcn_readfirstlane(wave_min32(lb)), wlb_max = __builtin_amdgcn_readfirstlane(wave_max32(lb));
+  const int wub_min = __builtin_amdgcn_readfirstlane(wave_min32(ub)), wub_max = __builtin_amdgcn_readfirstlane(wave_max32(ub));
   if (lane == 0) {
     s_bounds[0][wave] = wlb_min;
     s_bounds[1][wave] = wub_max;
   }
+  if (tid == 0) s_outside = 0;
 
-  typename M::frag qf[KC];
-#pragma unroll
-  for (int c = 0; c < KC; ++c)
-    qf[c] = q < T ? M::load8(Qb + (int64_t)q * qpitch + 16 * c + 8 * g) : M::zero();
+  Split8 qf[KC];
+  bool outside = split_rows<D>(Qb + (int64_t)min(q, T - 1) * qpitch, q < T, g, qf);
+  FragOffsets<D> fo;
+  fo.init(lane);
 
   f32x16 o[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) o[i] = zero16();
-  float m_run = -INFINITY, l_run = 0.0f;
+  float m_ref = -INFINITY, m_true = -INFINITY, l_run = 0.0f;  // unscaled scores
+  const float c2 = a.scale_log2;
 
   __syncthreads();
   int kmin = s_bounds[0][0], kmax = s_bounds[1][0];
@@ -90,99 +103,115 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(FwdArgs a) {
     kmin = min(kmin, s_bounds[0][w]);
     kmax = max(kmax, s_bounds[1][w]);
   }
-  const int kt0 = (kmin / BN) * BN;
-  const int ntiles = kmax >= kmin ? (kmax - kt0) / BN + 1 : 0;
+  const int kt0 = __builtin_amdgcn_readfirstlane((kmin / BN) * BN);
+  const int ntiles = __builtin_amdgcn_readfirstlane(kmax >= kmin ? (kmax - (kmin / BN) * BN) / BN + 1 : 0);
 
-  TileStage<E, D, BN> kst, vst;
+  SplitStage<D> kst, vst;
+  bool grown = false;
   if (ntiles > 0) {
     kst.load(Kb, kpitch, kt0, T, tid);
     vst.load(Vb, kpitch, kt0, T, tid);
-    kst.store_nat(smem, C::kLDK, tid);
-    if constexpr (C::kBF) vst.store_tr(smem + C::kKElems, C::kLDVT, tid);
-    else vst.store_nat(smem + C::kKElems, C::kLDV, tid);
+    outside |= kst.store(Ks, tid);
   }
+  __syncthreads();
 
   for (int it = 0; it < ntiles; ++it) {
     const int kt = kt0 + it * BN;
-    const E* Ks = smem + (it & 1) * C::kStage;
-    const E* Vs = Ks + C::kKElems;
     const bool more = it + 1 < ntiles;
+    const bool active = !(wlb_min > kt + BN - 1 || wub_max < kt);
+    f32x16 s = zero16();
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < KC; ++c) s = mma_split(split_nat<D>(Ks, fo, c), qf[c], s);
+      outside |= vst.store(Vs, tid);
+    } else {
+      outside |= vst.store(Vs, tid);
+    }
+    if (more) kst.load(Kb, kpitch, kt + BN, T, tid);
+    __syncthreads();
+
+    if (active) {
+      const bool need_mask = !(wlb_max <= kt && kt + BN - 1 <= wub_min);
+      if (need_mask) {
+        const int x = kt + 4 * g - lb, y = ub - (kt + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = 8 * (r >> 2) + (r & 3);
+          s[r] = (x >= -c) & (y >= c) ? s[r] : -INFINITY;
+        }
+      }
+      float mx = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      m_true = fmaxf(m_true, mx);
+      m_ref = m_ref == -INFINITY ? mx : m_ref;  // a row's first visible key sets the reference
+      grown |= (mx - m_ref) * c2 > kExactGrowth;
+      const float ref = m_ref == -INFINITY ? 0.0f : m_ref;
+      float psum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        // The difference first: the largest probability is exactly 1.
+        s[r] = __builtin_amdgcn_exp2f((s[r] - ref) * c2);
+        psum += s[r];
+      }
+      l_run += psum;
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+        const Split8 pf = kc ? split_acc<1>(s) : split_acc<0>(s);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db] = mma_split(split_tr<D>(Vs, fo, kc, db), pf, o[db]);
+      }
+    }
     if (more) {
-      kst.load(Kb, kpitch, kt + BN, T, tid);
+      outside |= kst.store(Ks, tid);
       vst.load(Vb, kpitch, kt + BN, T, tid);
     }
     __syncthreads();
+  }
 
-    const bool active = !(wlb_min > kt + BN - 1 || wub_max < kt);
-    if (active) {
-      f32x16 s[NKB];
+  // Probabilities above 1 may have carried a sum past the float32 range that
+  // those against the exact maximum stay in.
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) s[kb] = zero16();
+  for (int db = 0; db < DB; ++db) grown |= !(max_abs16(o[db]) < INFINITY);
+  if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
+  __syncthreads();
+  if (s_outside != 0 || __builtin_amdgcn_ballot_w64(grown) != 0) {
+    // fp32 MFMA from global memory, with the exact maximum first.
+    using M = Mma<float>;
+    f32x8 q32[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) {
+    for (int c = 0; c < KC; ++c) q32[c] = q < T ? M::load8(Qb + (int64_t)q * qpitch + 16 * c + 8 * g) : M::zero();
+    const int klo = (wlb_min / 32) * 32;
+    m_true = -INFINITY;
+    for (int k0 = klo; k0 <= wub_max; k0 += 32) {
+      const f32x16 s = exact_scores<D>(Kb, kpitch, q32, k0, T, l32, g, lb, ub);
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-          const auto kfrag = M::load8(Ks + (32 * kb + l32) * C::kLDK + 16 * c + 8 * g);
-          s[kb] = M::mma(kfrag, qf[c], s[kb]);
-        }
+      for (int r = 0; r < 16; ++r) m_true = fmaxf(m_true, s[r]);
+    }
+    m_true = fmaxf(m_true, __shfl_xor(m_true, 32));
+    m_ref = m_true;
+    l_run = 0.0f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o[db] = zero16();
+    for (int k0 = klo; k0 <= wub_max; k0 += 32) {
+      f32x16 s = exact_scores<D>(Kb, kpitch, q32, k0, T, l32, g, lb, ub);
+      const float safe = m_ref == -INFINITY ? 0.0f : m_ref;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] = __builtin_amdgcn_exp2f((s[r] - safe) * c2);
+        l_run += s[r];
       }
-
-      const bool need_mask = !(wlb_max <= kt && kt + BN - 1 <= wub_min);
-      float mx = -INFINITY;
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float x = s[kb][r] * a.scale_log2;
-          if (need_mask) {
-            const int key = kt + 32 * kb + acc_row(r, g);
-            if (key < lb || key > ub) x = -INFINITY;
-          }
-          s[kb][r] = x;
-          mx = fmaxf(mx, x);
-        }
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float m_new = fmaxf(m_run, mx);
-      const float safe = m_new == -INFINITY ? 0.0f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - safe);
-      float psum = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(s[kb][r] - safe);
-          s[kb][r] = p;
-          psum += p;
-        }
-      }
-      l_run = l_run * alpha + psum;
-      m_run = m_new;
-#pragma unroll
-      for (int db = 0; db < DB; ++db) o[db] *= alpha;
-
-#pragma unroll
-      for (int kc = 0; kc < BN / 16; ++kc) {
-        const auto pf = (kc & 1) ? M::template from_acc<1>(s[kc >> 1]) : M::template from_acc<0>(s[kc >> 1]);
+      for (int kc = 0; kc < 2; ++kc) {
+        const f32x8 pf = kc ? M::from_acc<1>(s) : M::from_acc<0>(s);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          typename M::frag vfrag;
-          if constexpr (C::kBF) {
-            vfrag = load_tr_bf16(Vs + (32 * db + l32) * C::kLDVT + 16 * kc, g);
-          } else {
-            const int col = D < 32 ? min(32 * db + l32, D - 1) : 32 * db + l32;  // rows >= D unused
-            vfrag = load_kt_f32(Vs + 16 * kc * C::kLDV + col, C::kLDV, g);
-          }
-          o[db] = M::mma(vfrag, pf, o[db]);
+          f32x8 vf;
+          load_rows_f32<D>(Vb, kpitch, k0 + 16 * kc, T, 32 * db + l32, g, vf);
+          o[db] = M::mma(vf, pf, o[db]);
         }
       }
-    }
-
-    if (more) {
-      E* Kn = smem + ((it + 1) & 1) * C::kStage;
-      kst.store_nat(Kn, C::kLDK, tid);
-      if constexpr (C::kBF) vst.store_tr(Kn + C::kKElems, C::kLDVT, tid);
-      else vst.store_nat(Kn + C::kKElems, C::kLDV, tid);
     }
   }
 
@@ -199,44 +228,39 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(FwdArgs a) {
           f32x4 v;
 #pragma unroll
           for (int t = 0; t < 4; ++t) v[t] = o[db][4 * j + t] * inv;
-          if (a.out_bf16) store4(static_cast<bf16*>(a.O) + orow * D + d0, v, false);
-          else store4(static_cast<float*>(a.O) + orow * D + d0, v, false);
+          store4(static_cast<float*>(a.O) + orow * D + d0, v, false);
         }
       }
     }
     if (g == 0) {
       const int64_t si = ((int64_t)b * a.H + h) * T + q;
-      a.l[si] = lt;
-      a.m[si] = m_run == -INFINITY ? -kFltMax : m_run * kLn2;
+      const bool any = m_true != -INFINITY;
+      a.l[si] = any ? lt * __builtin_amdgcn_exp2f((m_ref - m_true) * c2) : lt;
+      a.m[si] = any ? m_true * c2 * kLn2 : -kFltMax;
     }
   }
 }
 
-template <typename E, int D>
-static hipError_t launch_fwd_t(const Problem& p, const FwdArgs& a, hipStream_t s) {
-  const int n_qt = (p.T + FwdCfg<E, D>::kBM - 1) / FwdCfg<E, D>::kBM;
+template <int D>
+static hipError_t launch_fwd_exact(const Problem& p, const FwdArgs& a, hipStream_t s) {
+  const int n_qt = (p.T + kExactBM - 1) / kExactBM;
   const dim3 grid(n_qt * p.H * p.B), block(kThreads);
   const ProfileMark mk = profile_begin(s);
-  hipLaunchKernelGGL((attn_fwd_kernel<E, D>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((attn_fwd_exact_kernel<D>), grid, block, 0, s, a);
   const hipError_t e = hipGetLastError();
-  profile_end(mk, p.bf16 ? "attn_fwd_bf16" : "attn_fwd_f32", s);
+  profile_end(mk, "attn_fwd_f32", s);
   return e;
 }
 
-template <typename E>
-static hipError_t launch_fwd_e(const Problem& p, const FwdArgs& a, hipStream_t s) {
+hipError_t launch_fwd(const Problem& p, const FwdArgs& a, hipStream_t s) {
+  if (p.bf16) return launch_fwd_fast(p, a, s);
   switch (p.Dk) {
-    case 16: return launch_fwd_t<E, 16>(p, a, s);
-    case 32: return launch_fwd_t<E, 32>(p, a, s);
-    case 64: return launch_fwd_t<E, 64>(p, a, s);
-    case 128: return launch_fwd_t<E, 128>(p, a, s);
+    case 16: return launch_fwd_exact<16>(p, a, s);
+    case 32: return launch_fwd_exact<32>(p, a, s);
+    case 64: return launch_fwd_exact<64>(p, a, s);
+    case 128: return launch_fwd_exact<128>(p, a, s);
     default: return hipErrorInvalidValue;
   }
 }
-
-hipError_t launch_fwd(const Problem& p, const FwdArgs& a, hipStream_t s) {
-  return p.bf16 ? launch_fwd_fast(p, a, s) : launch_fwd_e<float>(p, a, s);
-}
-
 
 }  // namespace fc

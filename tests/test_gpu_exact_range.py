@@ -1,0 +1,106 @@
+"""Exact mode outside the range its bf16 parts hold: the products of three
+bf16 parts stand for float32 products while values are below 2^127 and eight
+of a row are not all below 2^-96; workgroups that meet others (or scores that
+outgrow the first tile's maximum by 2^64) recompute with fp32 products.
+
+Scaling by a power of two is exact, so a scaled problem must give the scaled
+results of the plain one (itself compared with the float64 oracle); both
+paths differ from the exact value by at most a few 1e-6 (2-norm: float32
+sums of up to 300 terms, n 2^-24 = 2e-5 at the very worst), and the bound is
+twice that.
+"""
+import numpy as np
+import pytest
+import torch
+
+from femtochat_amd import MFMAExact
+from femtochat_amd import kernels as Kn
+from oracle import attention_ref as R
+from tests.helpers import TOL, rel_err, to_np
+
+pytestmark = pytest.mark.gpu
+BOUND = 4e-5
+
+
+def _inputs(D, T=300, B=2, H=4, Hkv=2, seed=0):
+    rng = np.random.Generator(np.random.PCG64(seed + D))
+    Q, K, V, dO = (rng.standard_normal((B, T, h, D), dtype=np.float32) for h in (H, Hkv, Hkv, H))
+    return [np.clip(x, -1.9, 1.9) for x in (Q, K, V)] + [0.1 * dO]
+
+
+def _run(gpu, Q, K, V, dO, window=(-1, 0)):
+    t = [torch.from_numpy(np.ascontiguousarray(x)).to(gpu) for x in (Q, K, V, dO)]
+    st = Kn.attention_state(MFMAExact(), *t[:3], window)
+    g = [torch.empty_like(x) for x in t[:3]]
+    Kn.delta_attention_(MFMAExact(), *g, t[3], *t[:3], st.O, st.l, st.m, window, accumulate=False)
+    torch.cuda.synchronize()
+    return [to_np(x).astype(np.float64) for x in (st.O, *g)]
+
+
+def _close(x, y):
+    return np.linalg.norm(x - y) <= BOUND * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("q,k,v,do", [(-100, 100, 0, 0), (110, -110, 0, 0), (0, 0, 116, -126), (0, 0, 0, -110),
+                                      (0, 0, -112, 0), (0, 0, -60, 60)])
+def test_scaled_inputs(gpu, D, q, k, v, do):
+    Q, K, V, dO = _inputs(D)
+    plain = _run(gpu, Q, K, V, dO)
+    l_ref = R.forward(Q, K, V, (-1, 0))
+    assert rel_err(plain[0], l_ref[0]) <= TOL["exact"]
+    f = [np.float32(2.0) ** np.float32(e) for e in (q, k, v, do)]
+    scaled = _run(gpu, Q * f[0], K * f[1], V * f[2], dO * f[3])
+    fs = [float(x) for x in f]
+    for x, y, s in zip(scaled, plain, (fs[2], fs[2] * fs[3] / fs[0], fs[2] * fs[3] / fs[1], fs[3])):
+        assert np.all(np.isfinite(x)) and _close(x / s, y)
+
+
+@pytest.mark.parametrize("D", [32, 128])
+def test_infinite_value_and_nan_query(gpu, D):
+    """An infinite V element reaches the queries that see its key (and, as 0
+    times infinity, those whose 32-key tile holds it), in its column alone; a
+    NaN in a query stays in that query's row."""
+    Q, K, V, dO = _inputs(D, B=1, H=2, Hkv=1)
+    plain = _run(gpu, Q, K, V, dO)[0]
+    V2 = V.copy()
+    V2[0, 150, 0, 3] = np.inf
+    O = _run(gpu, Q, K, V2, dO)[0]
+    assert np.all(O[0, 150:, :, 3] == np.inf) and np.all(np.isfinite(O[0, :128]))
+    others = [d for d in range(D) if d != 3]
+    assert _close(O[..., others], plain[..., others]) and _close(O[0, :128], plain[0, :128])
+    Q2 = Q.copy()
+    Q2[0, 77, 1, 5] = np.nan
+    O = _run(gpu, Q2, K, V, dO)[0]
+    assert np.all(np.isnan(O[0, 77, 1]))
+    O[0, 77, 1] = plain[0, 77, 1]
+    assert _close(O, plain)
+
+
+@pytest.mark.parametrize("D", [16, 128])
+def test_large_values_behind_growing_scores(gpu, D):
+    """Probabilities of up to 2^40 against the first tile's maximum times values
+    of 2^100: the sum leaves the float32 range unless the exact maximum is the
+    reference."""
+    Q, K, V, dO = _inputs(D, B=1, H=2, Hkv=1)
+    Q, K = np.abs(Q) + 0.5, np.abs(K) + 0.5
+    K *= np.where(np.arange(K.shape[1]) < 256, 0.1, 1.0).astype(np.float32)[None, :, None, None]
+    S = np.einsum("thd,kd->htk", Q[0], K[0, :, 0]) * np.log2(np.e) / np.sqrt(D)
+    Q *= np.float32(45.0 / S.max())  # base-2 scores up to 45, at most 6 in the first 256 keys
+    V *= np.float32(2.0) ** np.float32(100)
+    O = _run(gpu, Q, K, V, dO)[0]
+    assert np.all(np.isfinite(O)) and rel_err(O, R.forward(Q, K, V, (-1, 0))[0]) <= TOL["exact"]
+
+
+@pytest.mark.parametrize("D", [16, 128])
+def test_growing_scores(gpu, D):
+    """Scores that grow along the keys by far more than 2^64 between tiles."""
+    Q, K, V, dO = _inputs(D, seed=9)
+    Q = np.abs(Q) + 0.5
+    K = (np.abs(K) + 0.5) * (np.arange(K.shape[1], dtype=np.float32)[None, :, None, None] / 4)
+    O, dQ, dK, dV = _run(gpu, Q, K, V, dO)
+    O_ref, l_ref, m_ref = R.forward(Q, K, V, (-1, 0))
+    g_ref = R.backward(dO, Q, K, V, O_ref, l_ref, m_ref, (-1, 0))
+    # scores of up to 600 carry a rounding of 600 log2(e) 2^-24 in the exponent
+    for x, r in zip((O, dV), (O_ref, g_ref[2])):
+        assert rel_err(x, r) <= 3 * TOL["exact"]
