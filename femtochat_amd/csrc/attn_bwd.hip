@@ -31,7 +31,7 @@ namespace fc {
 // Preprocess: Delta = sum_d dO*O (fp32), lse2 = m*log2(e) + log2(max(l, eps)).
 template <int D, typename TO, typename TD>
 __global__ __launch_bounds__(kThreads) void attn_bwd_pre_kernel(PreArgs a) {
-  constexpr int LPQ = D / 8;            // lanes per query, 8 elements each
+  constexpr int LPQ = tile_width(D) / 8;  // lanes per query, 8 elements each (idle past D)
   constexpr int QPB = kThreads / LPQ;   // queries per block
   const int tid = threadIdx.x;
   const int sub = tid % LPQ;
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_pre_kernel(PreArgs a) {
   const int64_t n = (int64_t)a.B * a.T * a.H;
   if (a.queue != nullptr && blockIdx.x == 0 && tid < kXcds) a.queue[tid] = 0;
   float acc = 0.0f;
-  if (idx < n) {
+  if (idx < n && 8 * sub < D) {
     const TD* dO = static_cast<const TD*>(a.dO) + idx * D + 8 * sub;
     const TO* O = static_cast<const TO*>(a.O) + idx * D + 8 * sub;
     float x[8];
@@ -192,7 +192,7 @@ constexpr int kExactBT = 32;   // rows per staged tile (queries here, keys in dQ
 
 template <int D>
 __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact_kernel(BwdArgs a) {
-  constexpr int BQ = kExactBT, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  constexpr int BQ = kExactBT, KC = D / 16, DB = (D + 31) / 32;
   constexpr int kTile = SplitTile<D>::kBytes;
   __shared__ __attribute__((aligned(1024))) char Qbuf[2][kTile];
   __shared__ __attribute__((aligned(1024))) char Os[kTile];  // dO
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
       s_low[wave][1][c][lane] = f[c].part[2];
     }
   }
-  FragOffsets<D> fo;
+  FragOffsets<tile_width(D)> fo;
   fo.init(lane);
   f32x16 dk[DB], dv[DB];
 #pragma unroll
@@ -316,10 +316,11 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
   auto product = [&](const char* tile, const bf16x8 (&f)[KC][2], int which) __attribute__((always_inline)) {
     auto keys = [&](int c) { return Split8{{f[c][0], f[c][1], s_low[wave][which][c][lane]}}; };
     f32x16 even = zero16(), odd = zero16();
-    if constexpr (KC == 1) return mma_split(split_nat<D>(tile, fo, 0), keys(0), even);
 #pragma unroll
     for (int c = 0; c + 1 < KC; c += 2)
       mma_split_pair(split_nat<D>(tile, fo, c), keys(c), even, split_nat<D>(tile, fo, c + 1), keys(c + 1), odd);
+    if constexpr (KC % 2 == 1) even = mma_split(split_nat<D>(tile, fo, KC - 1), keys(KC - 1), even);
+    if constexpr (KC == 1) return even;
     return even + odd;
   };
 
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
 // 3% (slower at D = 64, where they spill).
 template <int D>
 __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_kernel(BwdArgs a) {
-  constexpr int BN = kExactBT, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  constexpr int BN = kExactBT, KC = D / 16, DB = (D + 31) / 32;
   constexpr int kTile = SplitTile<D>::kBytes, kBM = 128;
   __shared__ __attribute__((aligned(1024))) char bufs[2][2 * kTile];  // K, V
   __shared__ int s_bounds[2][kWaves];
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
   Split8 qf[KC], of[KC];
   const int64_t qrow = (int64_t)min(q, T - 1) * qpitch;
   bool outside = split_rows<D>(Qb + qrow, q < T, g, qf) | split_rows<D>(Ob + qrow, q < T, g, of);
-  FragOffsets<D> fo;
+  FragOffsets<tile_width(D)> fo;
   fo.init(lane);
   f32x16 dq[DB];
 #pragma unroll
@@ -647,7 +648,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
 
 template <int D, typename TO, typename TD>
 static hipError_t launch_pre_t(const Problem& p, const PreArgs& a, hipStream_t s) {
-  constexpr int QPB = kThreads / (D / 8);
+  constexpr int QPB = kThreads / (tile_width(D) / 8);
   const int64_t n = (int64_t)p.B * p.T * p.H;
   const dim3 grid((unsigned)((n + QPB - 1) / QPB)), block(kThreads);
   const ProfileMark mk = profile_begin(s);
@@ -663,16 +664,6 @@ static hipError_t launch_pre_d(const Problem& p, const PreArgs& a, hipStream_t s
     return a.dO_bf16 ? launch_pre_t<D, bf16, bf16>(p, a, s) : launch_pre_t<D, bf16, float>(p, a, s);
   }
   return a.dO_bf16 ? launch_pre_t<D, float, bf16>(p, a, s) : launch_pre_t<D, float, float>(p, a, s);
-}
-
-hipError_t launch_bwd_pre(const Problem& p, const PreArgs& a, hipStream_t s) {
-  switch (p.Dk) {
-    case 16: return launch_pre_d<16>(p, a, s);
-    case 32: return launch_pre_d<32>(p, a, s);
-    case 64: return launch_pre_d<64>(p, a, s);
-    case 128: return launch_pre_d<128>(p, a, s);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 hipError_t launch_bounds(const Problem& p, const BoundsArgs& a, hipStream_t s) {
@@ -717,13 +708,19 @@ static hipError_t launch_dq_exact(const Problem& p, const BwdArgs& a, hipStream_
 }
 
 #define FC_DISPATCH_D(FN)                          \
-  switch (p.Dk) {                                  \
+  switch (p.D) {                                   \
     case 16: return FN<16>(p, a, s);               \
     case 32: return FN<32>(p, a, s);               \
+    case 48: return FN<48>(p, a, s);               \
     case 64: return FN<64>(p, a, s);               \
+    case 80: return FN<80>(p, a, s);               \
+    case 96: return FN<96>(p, a, s);               \
+    case 112: return FN<112>(p, a, s);             \
     case 128: return FN<128>(p, a, s);             \
     default: return hipErrorInvalidValue;          \
   }
+
+hipError_t launch_bwd_pre(const Problem& p, const PreArgs& a, hipStream_t s) { FC_DISPATCH_D(launch_pre_d) }
 
 hipError_t launch_bwd_dkdv(const Problem& p, const BwdArgs& a, hipStream_t s) {
   if (p.bf16) return launch_bwd_dkdv_fast(p, a, s);

@@ -1,8 +1,8 @@
 // Flash-attention backward, fast mode: the dK/dV kernel (persistent,
 // KV-stationary) and its launcher template.  Included by the translation
-// units that instantiate it: attn_bwd_fast.hip (D = 128) and
+// units that instantiate it: attn_bwd_fast.hip (D > 64) and
 // attn_bwd_dkdv_vgpr.hip (D <= 64, built so that every MFMA result lands in
-// ordinary vector registers; at D = 128 the accumulators need the
+// ordinary vector registers; above that the accumulators need the
 // accumulation registers).
 #pragma once
 
@@ -18,8 +18,9 @@ struct DkdvFastCfg {
   static constexpr int kBK = 128;  // keys per workgroup
   static constexpr int kBQ = 128;  // queries per step
   static constexpr int kKC = D / 16;
-  static constexpr int kDB = D < 32 ? 1 : D / 32;
-  static constexpr int kTileBytes = kBQ * 2 * D;
+  static constexpr int kDB = (D + 31) / 32;
+  static constexpr int kW = tile_width(D);
+  static constexpr int kTileBytes = kBQ * 2 * kW;
   static constexpr int kStageBytes = 2 * kTileBytes;  // Q, dO
 };
 
@@ -49,7 +50,7 @@ struct DkdvStep {
   template <typename Dma>
   __device__ __attribute__((always_inline)) static inline void run(const Dma& dma, const char* Qs, const char* Os, const float* lse,
                                     const float* delta, const int* lbs, const int* lbc, const bf16x8* kf,
-                                    const bf16x8* vf, f32x16* dk, f32x16* dv, const FragOffsets<D>& fo, int q0,
+                                    const bf16x8* vf, f32x16* dk, f32x16* dv, const FragOffsets<DkdvFastCfg<D>::kW>& fo, int q0,
                                     int key, int kw0, int kw1, int g, int T, int right, float c2) {
     // Smallest and largest key lower bound over the tile's queries, from the
     // per-chunk bounds published with the tile (no cross-lane reduction).
@@ -136,15 +137,15 @@ struct DkdvStep {
     sf[1] = M::from_acc<1>(dp);
   }
 
-  __device__ static inline bf16x8 trq(const char* tile, int qb, int i, const FragOffsets<D>& fo) {
+  __device__ static inline bf16x8 trq(const char* tile, int qb, int i, const FragOffsets<DkdvFastCfg<D>::kW>& fo) {
     const int h = i / DB, db = i - h * DB;
-    return lds_tr_frag(tile + (32 * qb + 16 * h) * 2 * D, fo.tr(0, db), fo.tr(1, db));
+    return lds_tr_frag(tile + (32 * qb + 16 * h) * 2 * C::kW, fo.tr(0, db), fo.tr(1, db));
   }
 
   template <int kSides, typename Dma>
   __device__ __attribute__((always_inline)) static inline void body(const Dma& dma, const char* Qs, const char* Os, const float* lse,
                                      const float* delta, const int* lbs, const bf16x8* kf, const bf16x8* vf,
-                                     f32x16* dk, f32x16* dv, const FragOffsets<D>& fo, int q0, int key, int g,
+                                     f32x16* dk, f32x16* dv, const FragOffsets<DkdvFastCfg<D>::kW>& fo, int q0, int key, int g,
                                      int T, int right, float c2) {
     constexpr int M1 = 2 * KC;   // MFMAs of S, dP per block
     constexpr int M2 = 2 * NTR;  // MFMAs of dV, dK per block
@@ -160,8 +161,8 @@ struct DkdvStep {
       dma(ph);
       __builtin_amdgcn_sched_barrier(0);
       if (b1 < NQB) {
-        const char* qt = Qs + 32 * b1 * 2 * D;
-        const char* ot = Os + 32 * b1 * 2 * D;
+        const char* qt = Qs + 32 * b1 * 2 * C::kW;
+        const char* ot = Os + 32 * b1 * 2 * C::kW;
         bf16x8 qa[KC], oa[KC];
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_fast_kernel(BwdArgs
     t_first = first_tile(0);
     G = t_first < n_qt_tiles ? a.group : 0;  // no visible tile: no step
   };
-  FragOffsets<D> fo;
+  FragOffsets<DkdvFastCfg<D>::kW> fo;
   fo.init(lane);
   DmaPlan<D, BQ> plan;
   plan.init(wave, lane, qpitch);
@@ -538,7 +539,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_fast_kernel(BwdArgs
       // (2 bytes per value, straight from the accumulators) into a row-major
       // tile of its own, 16-byte units XOR-swizzled by the row, then stores
       // 16 bytes per lane, a store instruction covering 64 / U whole rows.
-      constexpr int RB = 2 * D, U = RB / 16, RPI = 64 / U;
+      constexpr int RB = 2 * C::kW, U = RB / 16, RPI = 64 / U;
       static_assert(kWaves * 2 * 32 * RB <= C::kStageBytes, "dK and dV tiles of every wave fit a stage buffer");
       // An opaque zero in the tile address keeps its offsets from being
       // hoisted out of the item loop (where they would only take registers).
@@ -569,7 +570,8 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_fast_kernel(BwdArgs
         const int off = row * RB + 16 * (u ^ (row & (U - 1)));
         const uint4 k4 = *reinterpret_cast<const uint4*>(tile + off);
         const uint4 v4 = *reinterpret_cast<const uint4*>(tile + 32 * RB + off);
-        const int voff = (int)(((int64_t)(ekw0 + row) * row_elems + 8 * u) * 2);
+        // (lanes past the head dim store out of range)
+        const int voff = D == C::kW || 8 * u < D ? (int)(((int64_t)(ekw0 + row) * row_elems + 8 * u) * 2) : kPastEnd;
         __builtin_amdgcn_raw_buffer_store_b128(u32x4{k4.x, k4.y, k4.z, k4.w}, rk, voff, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b128(u32x4{v4.x, v4.y, v4.z, v4.w}, rv, voff, 0, 0);
       }
@@ -578,7 +580,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_fast_kernel(BwdArgs
       // each wave's part of the idle stage buffer and read back 16 bytes
       // (four values) per lane, added to the caller's values when
       // accumulating, rounded once and stored as whole rows.
-      constexpr int RB = 4 * D, U = RB / 16, RPI = 64 / U;  // fp32 rows
+      constexpr int RB = 4 * C::kW, U = RB / 16, RPI = 64 / U;  // fp32 rows
       static_assert(kWaves * 32 * RB <= C::kStageBytes, "a tensor's tiles of every wave fit a stage buffer");
       int z;  // an opaque zero, as above
       asm volatile("v_mov_b32 %0, 0" : "=v"(z));
@@ -588,7 +590,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_fast_kernel(BwdArgs
         constexpr int NI = 32 / RPI;
         auto voff_of = [&](int i) {
           const int row = i * RPI + (lane + z) / U, u = (lane + z) % U;
-          return (int)(((int64_t)(ekw0 + row) * row_elems + 4 * u) * esz);
+          return D == C::kW || 4 * u < D ? (int)(((int64_t)(ekw0 + row) * row_elems + 4 * u) * esz) : kPastEnd;
         };
         // The caller's values, all requested before any is used (out-of-range
         // loads read zero).

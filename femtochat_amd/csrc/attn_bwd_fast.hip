@@ -20,7 +20,7 @@
 //    and K is also read transposed; dQ leaves through LDS in whole rows.
 //
 // The dK/dV kernel itself is in attn_bwd_dkdv_fast.hpp; this unit
-// instantiates it for D = 128, attn_bwd_dkdv_vgpr.hip for D <= 64.
+// instantiates it for D > 64, attn_bwd_dkdv_vgpr.hip for D <= 64.
 #include "attn_bwd_dkdv_fast.hpp"
 
 #include <type_traits>
@@ -33,8 +33,9 @@ struct DqFastCfg {
   static constexpr int kBM = 128;  // queries per workgroup
   static constexpr int kBN = 64;   // keys per tile
   static constexpr int kKC = D / 16;
-  static constexpr int kDB = D < 32 ? 1 : D / 32;
-  static constexpr int kTileBytes = kBN * 2 * D;
+  static constexpr int kDB = (D + 31) / 32;
+  static constexpr int kW = tile_width(D);
+  static constexpr int kTileBytes = kBN * 2 * kW;
   static constexpr int kStageBytes = 2 * kTileBytes;  // K, V
 };
 
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
       for (int c = 0; c < KC; ++c) ov[c] = as_bf16x8(buf_load16(rO, qoff + 32 * c, 0));
     }
   }
-  FragOffsets<D> fo;
+  FragOffsets<C::kW> fo;
   fo.init(lane);
   DmaPlan<D, BN> plan;
   plan.init(wave, lane, kpitch);
@@ -202,12 +203,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
         dp[b1] = zero16();
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
-          const bf16x8 ka = as_bf16x8(lds_load16(Ks + 32 * b1 * 2 * D, fo.nat(c)));
+          const bf16x8 ka = as_bf16x8(lds_load16(Ks + 32 * b1 * 2 * C::kW, fo.nat(c)));
           s[b1] = M::mma(ka, qf[c], s[b1]);
         }
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
-          const bf16x8 va = as_bf16x8(lds_load16(Vs + 32 * b1 * 2 * D, fo.nat(c)));
+          const bf16x8 va = as_bf16x8(lds_load16(Vs + 32 * b1 * 2 * C::kW, fo.nat(c)));
           dp[b1] = M::mma(va, of[c], dp[b1]);
         }
       }
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
         // dQ^T += K^T dS^T for the block's 2 chunks of 16 keys.
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-          const char* kchunk = Ks + 16 * (2 * b2 + hh) * 2 * D;
+          const char* kchunk = Ks + 16 * (2 * b2 + hh) * 2 * C::kW;
 #pragma unroll
           for (int db = 0; db < DB; ++db) {
             const bf16x8 kfr = lds_tr_frag(kchunk, fo.tr(0, db), fo.tr(1, db));
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
   // takes whole rows, 16 bytes of output per lane (plus the caller's values
   // when accumulating, added in fp32 before the one rounding).
   {
-    constexpr int RB = 4 * D;  // bytes per staged fp32 row
+    constexpr int RB = 4 * C::kW;  // bytes per staged fp32 row
     constexpr int U = RB / 16;
     static_assert(2 * 32 * RB <= C::kStageBytes, "two waves' tiles per stage buffer");
     char* tile = (wave < 2 ? bufA : bufB) + (wave & 1) * (32 * RB);
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
     auto emit = [&](auto elem) __attribute__((always_inline)) {
       using E = decltype(elem);
       constexpr int EPL = 16 / (int)sizeof(E);  // output elements per lane
-      constexpr int LPR = D / EPL;              // lanes per row
+      constexpr int LPR = C::kW / EPL;          // lanes per row, the last of them idle when D is below the width
       constexpr int RPI = 64 / LPR;             // rows per instruction
       constexpr int NI = 32 / RPI;
       E* base = static_cast<E*>(a.dQ) + ((int64_t)b * T * a.H + h) * D;
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
         for (int i = 0; i < NI; ++i) {
           const int row = i * RPI + lane / LPR, e0 = EPL * (lane % LPR);
           const int qr = epilogue_row(q0w, row, T);
-          old[i] = *reinterpret_cast<const uint4*>(base + (int64_t)qr * a.H * D + e0);
+          old[i] = *reinterpret_cast<const uint4*>(base + (int64_t)qr * a.H * D + min(e0, D - EPL));
         }
       }
 #pragma unroll
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
           v[4 * k] = __uint_as_float(w.x), v[4 * k + 1] = __uint_as_float(w.y);
           v[4 * k + 2] = __uint_as_float(w.z), v[4 * k + 3] = __uint_as_float(w.w);
         }
-        if (q0w + row < T) {
+        if (q0w + row < T && (D == C::kW || e0 < D)) {
           E* p = base + (int64_t)(q0w + row) * a.H * D + e0;
           if (a.accumulate) {
             const E* o = reinterpret_cast<const E*>(&old[i]);
@@ -368,20 +369,28 @@ static hipError_t launch_dq_fast_t(const Problem& p, const BwdArgs& a, hipStream
 }
 
 hipError_t launch_bwd_dkdv_fast(const Problem& p, const BwdArgs& a, hipStream_t s) {
-  switch (p.Dk) {
+  switch (p.D) {
     case 16:
     case 32:
+    case 48:
     case 64: return launch_bwd_dkdv_fast_vgpr(p, a, s);
+    case 80: return launch_dkdv_fast_t<80>(p, a, s);
+    case 96: return launch_dkdv_fast_t<96>(p, a, s);
+    case 112: return launch_dkdv_fast_t<112>(p, a, s);
     case 128: return launch_dkdv_fast_t<128>(p, a, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_bwd_dq_fast(const Problem& p, const BwdArgs& a, hipStream_t s) {
-  switch (p.Dk) {
+  switch (p.D) {
     case 16: return launch_dq_fast_t<16>(p, a, s);
     case 32: return launch_dq_fast_t<32>(p, a, s);
+    case 48: return launch_dq_fast_t<48>(p, a, s);
     case 64: return launch_dq_fast_t<64>(p, a, s);
+    case 80: return launch_dq_fast_t<80>(p, a, s);
+    case 96: return launch_dq_fast_t<96>(p, a, s);
+    case 112: return launch_dq_fast_t<112>(p, a, s);
     case 128: return launch_dq_fast_t<128>(p, a, s);
     default: return hipErrorInvalidValue;
   }

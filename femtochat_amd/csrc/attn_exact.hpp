@@ -109,7 +109,8 @@ __device__ inline void mma_split_pair(const Split8& a0, const Split8& b0, f32x16
 // A tile of 32 token rows x D in LDS: three swizzled bf16 tiles, one per part.
 template <int D>
 struct SplitTile {
-  using Tile = SwzTile<D>;
+  static constexpr int kW = tile_width(D);  // values past D are never used
+  using Tile = SwzTile<kW>;
   static constexpr int kPlane = 32 * Tile::kRowBytes;
   static constexpr int kBytes = 3 * kPlane;
 };
@@ -117,18 +118,18 @@ struct SplitTile {
 // Natural fragment (chunk c, row l32) and transposed fragment (16-row chunk
 // kc, column block db) of all three parts.
 template <int D>
-__device__ inline Split8 split_nat(const char* tile, const FragOffsets<D>& fo, int c) {
+__device__ inline Split8 split_nat(const char* tile, const FragOffsets<tile_width(D)>& fo, int c) {
   Split8 s;
 #pragma unroll
   for (int p = 0; p < 3; ++p) s.part[p] = as_bf16x8(lds_load16(tile + p * SplitTile<D>::kPlane, fo.nat(c)));
   return s;
 }
 template <int D>
-__device__ inline Split8 split_tr(const char* tile, const FragOffsets<D>& fo, int kc, int db) {
+__device__ inline Split8 split_tr(const char* tile, const FragOffsets<tile_width(D)>& fo, int kc, int db) {
   Split8 s;
 #pragma unroll
   for (int p = 0; p < 3; ++p)
-    s.part[p] = lds_tr_frag(tile + p * SplitTile<D>::kPlane + 16 * kc * 2 * D, fo.tr(0, db), fo.tr(1, db));
+    s.part[p] = lds_tr_frag(tile + p * SplitTile<D>::kPlane + 16 * kc * 2 * SplitTile<D>::kW, fo.tr(0, db), fo.tr(1, db));
   return s;
 }
 
@@ -155,7 +156,7 @@ struct SplitStage {
     const int unit = min(tid + i * kThreads, kUnits - 1);  // past the end: the same values to the same place again
     const float x[8] = {v[i][0][0], v[i][0][1], v[i][0][2], v[i][0][3], v[i][1][0], v[i][1][1], v[i][1][2], v[i][1][3]};
     const Split8 s = split8(x);
-    const int at = SwzTile<D>::offset(unit / kUPR, unit % kUPR);
+    const int at = SplitTile<D>::Tile::offset(unit / kUPR, unit % kUPR);
 #pragma unroll
     for (int p = 0; p < 3; ++p) lds_store16(tile + p * SplitTile<D>::kPlane, at, __builtin_bit_cast(uint4, s.part[p]));
     return outside_split(max_abs8(x));

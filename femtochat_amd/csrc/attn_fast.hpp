@@ -51,6 +51,16 @@ __device__ inline uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// Values per row of an LDS tile of head dim D: the next power of two, which the
+// swizzle needs.  Head dims between (48, 80, 96, 112) read their own rows from
+// global memory; the rest of a tile row is zero (DMA lanes past the head dim
+// read out of range) and costs no products beyond whole 16-value chunks (S, dP)
+// and 32-value blocks (the other products).  A bf16 step of 4 x 2048 tokens, H8
+// at D = 48 / 80 / 96 / 112 takes 167 / 181 / 185 / 214 us; on zero-padded copies
+// of Q, K, V, O, dO and fp32 gradients it took 276 / 392 / 425 / 440 (less some 80
+// of gradient conversions), and D = 64 / 128 take 163 / 212.
+constexpr int tile_width(int D) { return D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : 128; }
+
 template <int D>
 struct SwzTile {
   static constexpr int kUPR = D / 8;          // 16-byte units per row
@@ -209,9 +219,13 @@ __device__ inline void wait_vmcnt(int n) {
   }
 }
 
+// A byte offset past every descriptor's records (slices are below 2^31 bytes):
+// loads there give zero, stores are dropped.
+constexpr int kPastEnd = 0x7ffffff0;
+
 template <int D, int R, int NW = kWaves>
 struct DmaPlan {
-  using Tile = SwzTile<D>;
+  using Tile = SwzTile<tile_width(D)>;
   static constexpr int kInstr = R * Tile::kUPR / 64;  // 1 KB blocks per tile
   static_assert(R * Tile::kUPR % 64 == 0, "tile must be a whole number of 1 KB blocks");
   static constexpr int kPerWave = (kInstr + NW - 1) / NW;
@@ -223,7 +237,8 @@ struct DmaPlan {
       const int i = wave + NW * j;
       const int P = 64 * i + lane;
       const int row = P / Tile::kUPR, pu = P % Tile::kUPR;
-      goff[j] = row * pitch_bytes + 16 * (pu ^ Tile::swz(row));
+      const int u = pu ^ Tile::swz(row);
+      goff[j] = u < D / 8 ? row * pitch_bytes + 16 * u : kPastEnd;
     }
   }
   // Issues this wave's share of one tile's loads into the LDS tile at lds_addr.

@@ -53,7 +53,7 @@ __device__ inline f32x16 exact_scores(const float* Kb, int64_t kpitch, const f32
 
 template <int D>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) {
-  constexpr int BN = kExactBN, KC = D / 16, DB = D < 32 ? 1 : D / 32;
+  constexpr int BN = kExactBN, KC = D / 16, DB = (D + 31) / 32;
   __shared__ __attribute__((aligned(1024))) char Ks[SplitTile<D>::kBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[SplitTile<D>::kBytes];
   __shared__ int s_bounds[2][kWaves];
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
 
   Split8 qf[KC];
   bool outside = split_rows<D>(Qb + (int64_t)min(q, T - 1) * qpitch, q < T, g, qf);
-  FragOffsets<D> fo;
+  FragOffsets<tile_width(D)> fo;
   fo.init(lane);
 
   f32x16 o[DB];
@@ -254,10 +254,14 @@ static hipError_t launch_fwd_exact(const Problem& p, const FwdArgs& a, hipStream
 
 hipError_t launch_fwd(const Problem& p, const FwdArgs& a, hipStream_t s) {
   if (p.bf16) return launch_fwd_fast(p, a, s);
-  switch (p.Dk) {
+  switch (p.D) {
     case 16: return launch_fwd_exact<16>(p, a, s);
     case 32: return launch_fwd_exact<32>(p, a, s);
+    case 48: return launch_fwd_exact<48>(p, a, s);
     case 64: return launch_fwd_exact<64>(p, a, s);
+    case 80: return launch_fwd_exact<80>(p, a, s);
+    case 96: return launch_fwd_exact<96>(p, a, s);
+    case 112: return launch_fwd_exact<112>(p, a, s);
     case 128: return launch_fwd_exact<128>(p, a, s);
     default: return hipErrorInvalidValue;
   }

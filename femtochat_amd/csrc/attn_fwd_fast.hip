@@ -44,8 +44,9 @@ struct FwdFastCfg {
   static constexpr int kNQB = kWQ / 32;       // query blocks per wave
   static constexpr int kNKB = kBN / 32;       // key blocks per tile
   static constexpr int kKC = D / 16;
-  static constexpr int kDB = D < 32 ? 1 : D / 32;
-  static constexpr int kTileBytes = kBN * 2 * D;
+  static constexpr int kDB = (D + 31) / 32;
+  static constexpr int kW = tile_width(D);
+  static constexpr int kTileBytes = kBN * 2 * kW;
   static constexpr int kStageBytes = 2 * kTileBytes;  // K, V
 };
 
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
     }
   }
 
-  FragOffsets<D> fo;
+  FragOffsets<C::kW> fo;
   fo.init(lane);
   DmaPlan<D, BN> plan;
   plan.init(wave, lane, kpitch);
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
         // S^T = K Q^T for key block bS and both query blocks.
         bf16x8 kfr[KC];
 #pragma unroll
-        for (int c = 0; c < KC; ++c) kfr[c] = as_bf16x8(lds_load16(Ks + 32 * bS * 2 * D, fo.nat(c)));
+        for (int c = 0; c < KC; ++c) kfr[c] = as_bf16x8(lds_load16(Ks + 32 * bS * 2 * C::kW, fo.nat(c)));
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) s[bS][qb] = zero16();
 #pragma unroll
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
         // O^T += V^T P^T, 16 keys per product, each V fragment for both query blocks.
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-          const char* vchunk = Vs + 16 * (2 * bP + hh) * 2 * D;
+          const char* vchunk = Vs + 16 * (2 * bP + hh) * 2 * C::kW;
 #pragma unroll
           for (int db = 0; db < DB; ++db) {
             const bf16x8 vfr = lds_tr_frag(vchunk, fo.tr(0, db), fo.tr(1, db));
@@ -396,8 +397,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
   static_assert(NQB == 1, "one 32-query block per wave");
   auto store_o = [&](auto elem) __attribute__((always_inline)) {
     using E = decltype(elem);
-    constexpr int RB = D * (int)sizeof(E);  // bytes per output row
-    constexpr int U = RB / 16;              // 16-byte units per row
+    constexpr int RB = C::kW * (int)sizeof(E);  // bytes per staged row
+    constexpr int U = RB / 16;                  // 16-byte units per row, of which the first UD hold values
+    constexpr int OB = D * (int)sizeof(E), UD = OB / 16;  // of an output row
     static_assert(2 * 32 * RB <= C::kStageBytes, "two waves' tiles per stage buffer");
     char* tile = (wave < 2 ? bufA : bufB) + (wave & 1) * (32 * RB);
     const float lt = l_half[0] + other_half(l_half[0]);
@@ -430,12 +432,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
     constexpr int RPI = 64 / U;  // rows per store instruction
     const int q0w = qv[0] - l32;  // the wave's first query
     char* obase = static_cast<char*>(a.O) + (((int64_t)b * T * a.H + h) * D) * (int64_t)sizeof(E);
-    const int64_t opitch = (int64_t)a.H * RB;  // bytes between consecutive queries
+    const int64_t opitch = (int64_t)a.H * OB;  // bytes between consecutive queries
 #pragma unroll
     for (int i = 0; i < 32 / RPI; ++i) {
       const int row = i * RPI + lane / U, u = lane % U;
       const uint4 val = *reinterpret_cast<const uint4*>(tile + row * RB + 16 * (u ^ (row & (U - 1))));
-      if (q0w + row < T) *reinterpret_cast<uint4*>(obase + (q0w + row) * opitch + 16 * u) = val;
+      if (q0w + row < T && (UD == U || u < UD)) *reinterpret_cast<uint4*>(obase + (q0w + row) * opitch + 16 * u) = val;
     }
   };
   if (a.out_bf16) store_o(bf16{});
@@ -469,10 +471,14 @@ static hipError_t launch_fwd_fast_t(const Problem& p, const FwdArgs& a, hipStrea
 }
 
 hipError_t launch_fwd_fast(const Problem& p, const FwdArgs& a, hipStream_t s) {
-  switch (p.Dk) {
+  switch (p.D) {
     case 16: return launch_fwd_fast_t<16>(p, a, s);
     case 32: return launch_fwd_fast_t<32>(p, a, s);
+    case 48: return launch_fwd_fast_t<48>(p, a, s);
     case 64: return launch_fwd_fast_t<64>(p, a, s);
+    case 80: return launch_fwd_fast_t<80>(p, a, s);
+    case 96: return launch_fwd_fast_t<96>(p, a, s);
+    case 112: return launch_fwd_fast_t<112>(p, a, s);
     case 128: return launch_fwd_fast_t<128>(p, a, s);
     default: return hipErrorInvalidValue;
   }

@@ -17,7 +17,7 @@ namespace fc {
 // sentinel (-1,0) replaced by (T,0) and both extents clamped to [-T-1, T].
 struct Problem {
   int D;   // the caller's head dim (the scale is 1/sqrt(D))
-  int Dk;  // the head dim the kernels run with: D, or the compiled width D is zero-padded to
+  int Dk;  // D, or the next width whose tiles fill whole LDS rows
   int H, Hkv, T, B, group;
   int left, right;
   bool bf16;        // fast mode (bf16 inputs) vs exact mode (fp32)
@@ -57,9 +57,10 @@ inline bool windowed(const Problem& p) {
   return p.bf16 && !p.positions && (int64_t)p.left + std::max(p.right, 0) + 1 <= p.T / 2;
 }
 
-// Head dims the kernels are compiled for; every other multiple of 16 up to
-// 128 runs on copies zero-padded to the next of them (a zero column adds
-// nothing to Q.K, dO.V or dO.O, and the padded output columns are dropped).
+// Head dims whose tiles fill whole rows of LDS, and the tile width of every
+// other multiple of 16 up to 128 (48, 80, 96, 112): those read and write their
+// own rows too, and differ only in the workspace their callers bring
+// (PadWorkspace).
 inline bool head_dim_compiled(int D) { return D == 16 || D == 32 || D == 64 || D == 128; }
 inline bool head_dim_supported(int D) { return D >= 16 && D <= 128 && D % 16 == 0; }
 inline int kernel_head_dim(int D) { return D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : 128; }
@@ -147,19 +148,16 @@ inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 inline size_t chunk_bounds_bytes(const Problem& p) { return (size_t)p.B * ((p.T + 31) / 32) * 2 * sizeof(int32_t); }
 inline size_t order_bytes(const Problem& p) { return (size_t)p.B * ((p.T + kOrderRows - 1) / kOrderRows) * sizeof(int32_t); }
 
-// Workspace layout of the forward pass (byte offsets, 256-aligned): the
-// padded copies of a non-compiled head dim (required then), and when the
-// work order applies the per-32-query key bounds and the query tiles' order
-// (optional: the forward of a compiled head dim runs without a workspace,
-// in the default order).
+// Workspace layout of the forward pass (byte offsets, 256-aligned): PadWorkspace
+// (required where it is not empty), and when the work order applies the
+// per-32-query key bounds and the query tiles' order (optional: without a
+// workspace the forward runs in the default order).
 struct FwdWorkspace {
   size_t chunk_lb, qorder, total;
 };
 
-// The problem the kernels run: a padded problem's head dim replaced by the
-// compiled width (the scale still follows p.D).  A padded backward runs with
-// float32 gradients that it overwrites; they are added to (or written into)
-// the caller's gradients afterwards, rounded once.
+// A problem with float32 gradients that are overwritten, the widest case of a
+// backward workspace with PadWorkspace.
 inline Problem kernel_problem(const Problem& p, bool backward) {
   Problem k = p;
   if (padded(p) && backward) {
@@ -169,10 +167,13 @@ inline Problem kernel_problem(const Problem& p, bool backward) {
   return k;
 }
 
-// Padded copies of a non-compiled head dim (byte offsets, 256-aligned):
-// Q, K, V (input format), O (its format), and in the backward dO (its
-// format) and float32 dQ, dK, dV, all with rows of Dk values.  The kernels'
-// own workspace of the padded problem follows at `inner`.
+// What the workspace of head dims 48, 80, 96 and 112 begins with (byte
+// offsets, 256-aligned): room for Q, K, V (input format), O (its format), and
+// in the backward dO (its format) and float32 dQ, dK, dV with rows of Dk
+// values.  The kernels once ran on zero-padded copies held there and no longer
+// touch it, but the sizes fc_attn_workspace_bytes gives, and the forward's
+// refusal to run without a workspace, are what callers were built against.
+// The kernels' own workspace follows at `inner`.
 struct PadWorkspace {
   size_t Q, K, V, O, dO, dQ, dK, dV, inner;
 };
@@ -204,7 +205,7 @@ inline PadWorkspace pad_workspace(const Problem& p, bool backward) {
 
 inline FwdWorkspace fwd_workspace(const Problem& p) {
   FwdWorkspace w{};
-  size_t off = pad_workspace(p, false).inner;  // padded copies first, if any
+  size_t off = pad_workspace(p, false).inner;
   if (ordered(p)) {
     w.chunk_lb = off;
     off = align256(off + chunk_bounds_bytes(p));
@@ -215,8 +216,8 @@ inline FwdWorkspace fwd_workspace(const Problem& p) {
   return w;
 }
 
-// Workspace layout of the backward pass (byte offsets, 256-aligned): the
-// padded copies of a non-compiled head dim, then Delta and the base-2
+// Workspace layout of the backward pass (byte offsets, 256-aligned):
+// PadWorkspace, then Delta and the base-2
 // log-sum-exp per query, per-32-query key bounds with
 // positions, a bf16 copy of an fp32 dO in fast mode, in fast mode the
 // dK/dV kernel's work counters, and the dQ and dK/dV orders when the work
@@ -228,7 +229,7 @@ struct BwdWorkspace {
 inline BwdWorkspace bwd_workspace(const Problem& p) {
   BwdWorkspace w{};
   const size_t nq = (size_t)p.B * p.H * p.T;
-  size_t off = pad_workspace(p, true).inner;  // padded copies first, if any
+  size_t off = pad_workspace(p, true).inner;
   w.delta = off;
   off = align256(off + nq * sizeof(float));
   w.lse2 = off;

@@ -19,19 +19,21 @@ typedef __bf16 bf16_t;
 constexpr int kConvThreads = 256;
 constexpr int64_t kMaxBlocks = 8192;
 
+__device__ inline uint4 round8(float4 a, float4 b) {
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    w[k] = (uint32_t)__builtin_bit_cast(unsigned short, static_cast<bf16_t>(v[2 * k])) |
+           ((uint32_t)__builtin_bit_cast(unsigned short, static_cast<bf16_t>(v[2 * k + 1])) << 16);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // float32 -> bfloat16, round to nearest even (the hardware conversion).
 __global__ __launch_bounds__(kConvThreads) void f32_to_bf16_vec(const float4* __restrict__ src,
                                                                  uint4* __restrict__ dst, int64_t n8) {
   for (int64_t i = (int64_t)blockIdx.x * kConvThreads + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kConvThreads) {
-    const float4 a = src[2 * i];
-    const float4 b = src[2 * i + 1];
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t w[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      w[k] = (uint32_t)__builtin_bit_cast(unsigned short, static_cast<bf16_t>(v[2 * k])) |
-             ((uint32_t)__builtin_bit_cast(unsigned short, static_cast<bf16_t>(v[2 * k + 1])) << 16);
-    dst[i] = make_uint4(w[0], w[1], w[2], w[3]);
+    dst[i] = round8(src[2 * i], src[2 * i + 1]);
   }
 }
 
@@ -75,52 +77,7 @@ unsigned blocks_for(int64_t items) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Rows of src_cols values copied into rows of dst_cols values (eight per
-// thread; both counts are multiples of 16): columns past src_cols become
-// zero, columns past dst_cols are dropped; with accumulate the destination's
-// values are added in fp32 before the one rounding.  Pads a head dim to a
-// compiled width and drops the padding again (attn_api.hip).
-template <typename S, typename T>
-__global__ __launch_bounds__(kConvThreads) void repack_rows(const S* __restrict__ src, T* __restrict__ dst,
-                                                            int64_t rows, int src_cols, int dst_cols, int accumulate) {
-  const int groups = dst_cols / 8;
-  const int64_t n = rows * groups;
-  for (int64_t i = (int64_t)blockIdx.x * kConvThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kConvThreads) {
-    const int64_t row = i / groups;
-    const int c0 = 8 * (int)(i - row * groups);
-    float v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = c0 < src_cols ? static_cast<float>(src[row * src_cols + c0 + e]) : 0.0f;
-    T* d = dst + row * dst_cols + c0;
-    if (accumulate) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += static_cast<float>(d[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) d[e] = static_cast<T>(v[e]);
-  }
-}
-
 }  // namespace
-
-hipError_t launch_repack(const RepackArgs& a, hipStream_t s) {
-  const int64_t items = a.rows * (a.dst_cols / 8);
-  const dim3 grid(blocks_for(items)), block(kConvThreads);
-  if (a.src_bf16 && a.dst_bf16)
-    hipLaunchKernelGGL((repack_rows<bf16_t, bf16_t>), grid, block, 0, s, static_cast<const bf16_t*>(a.src),
-                       static_cast<bf16_t*>(a.dst), a.rows, a.src_cols, a.dst_cols, a.accumulate);
-  else if (a.src_bf16)
-    hipLaunchKernelGGL((repack_rows<bf16_t, float>), grid, block, 0, s, static_cast<const bf16_t*>(a.src),
-                       static_cast<float*>(a.dst), a.rows, a.src_cols, a.dst_cols, a.accumulate);
-  else if (a.dst_bf16)
-    hipLaunchKernelGGL((repack_rows<float, bf16_t>), grid, block, 0, s, static_cast<const float*>(a.src),
-                       static_cast<bf16_t*>(a.dst), a.rows, a.src_cols, a.dst_cols, a.accumulate);
-  else
-    hipLaunchKernelGGL((repack_rows<float, float>), grid, block, 0, s, static_cast<const float*>(a.src),
-                       static_cast<float*>(a.dst), a.rows, a.src_cols, a.dst_cols, a.accumulate);
-  return hipGetLastError();
-}
-
 }  // namespace fc
 
 extern "C" {

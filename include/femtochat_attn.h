@@ -94,9 +94,9 @@ fc_status fc_attn_workspace_bytes(const fc_attn_desc* desc, int32_t pass,
    64 and 128: in fast mode with positions, a workspace of
    fc_attn_workspace_bytes(FC_PASS_FORWARD) bytes, 256-byte aligned, lets the
    kernel take the query tiles in order of decreasing work (long documents
-   first); the results are the same.  Every other head_dim (48, 80, 96, 112)
-   runs on copies zero-padded to the next of those widths held in the
-   workspace, which is then required (FC_ERR_WORKSPACE without it). */
+   first); the results are the same.  At every other head_dim (48, 80, 96,
+   112) the workspace is required (FC_ERR_WORKSPACE without it; the kernels
+   read and write the caller's rows directly and leave most of it alone). */
 fc_status fc_attn_fwd(const fc_attn_desc* desc, const void* Q, const void* K,
                       const void* V, const int32_t* positions, void* O,
                       float* l, float* m, void* workspace,
@@ -210,8 +210,7 @@ fc_status fc_capabilities(int32_t device, fc_caps* caps);
 /* Supported head dims are reported as a bitmask: bit (D/16 - 1) set when
    head_dim D is supported (every multiple of 16 up to 128, as the
    reference's tensor-core path accepts, ext/FemtoChatCUDAExt.jl:214-223;
-   the kernels are compiled for 16, 32, 64 and 128 and the other widths run
-   zero-padded to the next of them). */
+   the kernels are compiled for each). */
 uint32_t fc_attn_supported_head_dims(void);
 
 int32_t fc_abi_version(void);
