@@ -37,6 +37,25 @@ __global__ __launch_bounds__(kConvThreads) void f32_to_bf16_vec(const float4* __
   }
 }
 
+// The same for three tensors in one launch (an attention call's Q, K and V):
+// item i of the three, one after another.  At the smallest calls three launches
+// are three times 2.4 us of GPU and 4 us of host time for little work.
+struct Convert3 {
+  const float4* src[3];
+  uint4* dst[3];
+  int64_t n8[3];
+};
+__global__ __launch_bounds__(kConvThreads) void f32_to_bf16_vec3(Convert3 a) {
+  const int64_t n = a.n8[0] + a.n8[1] + a.n8[2];
+  for (int64_t i = (int64_t)blockIdx.x * kConvThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kConvThreads) {
+    const int64_t at1 = i - a.n8[0], at2 = at1 - a.n8[1];
+    const int64_t at = at1 < 0 ? i : at2 < 0 ? at1 : at2;
+    const float4* src = at1 < 0 ? a.src[0] : at2 < 0 ? a.src[1] : a.src[2];
+    uint4* dst = at1 < 0 ? a.dst[0] : at2 < 0 ? a.dst[1] : a.dst[2];
+    dst[at] = round8(src[2 * at], src[2 * at + 1]);
+  }
+}
+
 // bfloat16 -> float32 (exact).
 __global__ __launch_bounds__(kConvThreads) void bf16_to_f32_vec(const uint4* __restrict__ src,
                                                                  float4* __restrict__ dst, int64_t n8) {
@@ -122,6 +141,41 @@ fc_status fc_convert(const void* src, int32_t src_dtype, void* dst, int32_t dst_
   const hipError_t e = hipGetLastError();
   fc::profile_end(mk, "convert", s);
   if (e != hipSuccess) return fc::set_error(FC_ERR_HIP, "fc_convert: launch failed");
+  fc::clear_error();
+  return FC_OK;
+}
+
+fc_status fc_convert3(const void* const* src, int32_t src_dtype, void* const* dst, int32_t dst_dtype, const int64_t* n,
+                      void* stream) {
+  if (src == nullptr || dst == nullptr || n == nullptr)
+    return fc::set_error(FC_ERR_INVALID_ARGUMENT, "fc_convert3: an array is null");
+  // One launch when all three are whole runs of 8 values on 16-byte boundaries
+  // that overlap nowhere; otherwise tensor by tensor.
+  bool one = src_dtype == FC_F32 && dst_dtype == FC_BF16;
+  fc::Convert3 a;
+  for (int i = 0; i < 3 && one; ++i) {
+    one = n[i] > 0 && n[i] % 8 == 0 && src[i] != nullptr && dst[i] != nullptr && fc::aligned16(src[i]) && fc::aligned16(dst[i]);
+    for (int j = 0; j < 3 && one; ++j) {
+      const uintptr_t s0 = reinterpret_cast<uintptr_t>(src[j]), d0 = reinterpret_cast<uintptr_t>(dst[i]);
+      one = n[j] > 0 && !(s0 < d0 + (uintptr_t)n[i] * 2 && d0 < s0 + (uintptr_t)n[j] * 4);
+    }
+    a.src[i] = static_cast<const float4*>(src[i]);
+    a.dst[i] = static_cast<uint4*>(dst[i]);
+    a.n8[i] = n[i] / 8;
+  }
+  if (!one) {
+    for (int i = 0; i < 3; ++i) {
+      const fc_status st = fc_convert(src[i], src_dtype, dst[i], dst_dtype, n[i], stream);
+      if (st != FC_OK) return st;
+    }
+    return FC_OK;
+  }
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const fc::ProfileMark mk = fc::profile_begin(s);
+  hipLaunchKernelGGL(fc::f32_to_bf16_vec3, dim3(fc::blocks_for(a.n8[0] + a.n8[1] + a.n8[2])), dim3(fc::kConvThreads), 0, s, a);
+  const hipError_t e = hipGetLastError();
+  fc::profile_end(mk, "convert", s);
+  if (e != hipSuccess) return fc::set_error(FC_ERR_HIP, "fc_convert3: launch failed");
   fc::clear_error();
   return FC_OK;
 }

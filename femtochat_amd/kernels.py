@@ -194,6 +194,15 @@ def attention_inputs(A, Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor):
     else:
         return Q, K, V
 
+    if Q.dtype == K.dtype == V.dtype != target and Q.dtype in _DTYPE_CODES and Q.is_cuda and Q.device == K.device == V.device:
+        src = [x.contiguous() for x in (Q, K, V)]
+        dst = tuple(torch.empty(x.shape, dtype=target, device=x.device) for x in src)
+        _lib.check(_lib.lib().fc_convert3(
+            (ctypes.c_void_p * 3)(*[x.data_ptr() for x in src]), _DTYPE_CODES[Q.dtype],
+            (ctypes.c_void_p * 3)(*[x.data_ptr() for x in dst]), _DTYPE_CODES[target],
+            (ctypes.c_int64 * 3)(*[x.numel() for x in src]), _stream_ptr(Q.device)))
+        return dst
+
     def conv(x):
         if x.dtype == target:
             return x

@@ -185,6 +185,12 @@ fc_status fc_rope_norm_bwd(const fc_rope_norm_desc* desc, const void* dY,
 fc_status fc_convert(const void* src, int32_t src_dtype, void* dst,
                      int32_t dst_dtype, int64_t n, void* stream);
 
+/* fc_convert of three tensors (an attention call's Q, K and V) between the
+   same pair of dtypes, in one launch where sizes and alignment allow: n[i]
+   values from src[i] to dst[i]. */
+fc_status fc_convert3(const void* const* src, int32_t src_dtype, void* const* dst,
+                      int32_t dst_dtype, const int64_t* n, void* stream);
+
 /* bytes bytes of dst set to zero by a kernel (not a memset, so a captured
    graph replays it correctly).  Replaces zero(x) / fill!(x, 0) of a device
    buffer (the reference's zeroed gradients, ext/FemtoChatEnzymeExt.jl). */

@@ -93,3 +93,22 @@ def test_attention_inputs_convert_through_the_library(gpu):
         assert torch.equal(a.view(torch.int16), b.to(torch.bfloat16).view(torch.int16))
     q2, k2, v2 = attention_inputs(MFMAExact(), q, k, v)
     assert q2.dtype == torch.float32 and torch.equal(q2, q.float())
+
+
+@pytest.mark.parametrize("sizes,offset", [((4096, 2048, 2048), 0), ((8, 16, 24), 0), ((1000, 8, 8), 1), ((13, 8, 0), 0)])
+def test_convert_three_tensors(gpu, sizes, offset):
+    """fc_convert3 writes what three fc_convert calls write (one launch, or one
+    by one for sizes and pointers off 8 values), and nothing beyond."""
+    import ctypes
+
+    from femtochat_amd import _lib
+
+    src = [_f32_cases(n + offset, 7 + i)[offset:].to(gpu) for i, n in enumerate(sizes)]
+    flat = [torch.full((n + 16,), 7.0, dtype=torch.bfloat16, device=gpu) for n in sizes]
+    s = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.lib().fc_convert3((ctypes.c_void_p * 3)(*[x.data_ptr() for x in src]), _lib.FC_F32,
+                                      (ctypes.c_void_p * 3)(*[x.data_ptr() for x in flat]), _lib.FC_BF16,
+                                      (ctypes.c_int64 * 3)(*sizes), s))
+    torch.cuda.synchronize()
+    for x, y, n in zip(src, flat, sizes):
+        assert torch.equal(y[:n].view(torch.int16), x.to(torch.bfloat16).view(torch.int16)) and bool((y[n:] == 7).all())
