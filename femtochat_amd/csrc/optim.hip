@@ -357,7 +357,12 @@ __device__ inline void wait_vmcnt() {
 // each wave 64 x 32 (2 x 1 blocks); the Q tile is 64 rows by 64 values (128 B
 // per row; k-major, its units are swizzled by 4 ((r/2) mod 2), which keeps
 // its transposed reads free of bank conflicts).
-template <bool kTr, int kStages, bool kNarrow = false>
+// kSym (D symmetric in exact arithmetic, M = N: A = X X^T and B = c A A + b A):
+// only the tiles on and below the diagonal are computed, 10 of 16 at lo = 512,
+// and each one below it is also written transposed to its place above; D is then
+// its own transpose bit for bit.  A of 8 matrices of 512 x 2048 in a grouped call:
+// 27 -> 18.5 us.
+template <bool kTr, int kStages, bool kNarrow = false, bool kSym = false>
 __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(PolarGemm a) {
   constexpr int kTN = kNarrow ? 64 : kGemmTile;  // tile width (j)
   constexpr int kNY = kTN / 64;                   // 32-column blocks per wave
@@ -368,13 +373,22 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
   constexpr int kLds = kStageBytes * kStages > 4 * kQuadBytes ? kStageBytes * kStages : 4 * kQuadBytes;
   __shared__ __attribute__((aligned(1024))) char lds[kLds];
   auto tile = [&](int stage, int which) __attribute__((always_inline)) { return lds + kStageBytes * stage + 16384 * which; };
-  const int tm = a.M / kGemmTile, tiles = tm * (a.N / kTN);
+  const int tm = a.M / kGemmTile, tiles = kSym ? tm * (tm + 1) / (kNarrow ? 1 : 2) : tm * (a.N / kTN);
   // XCD-aware order: workgroup w runs on XCD w mod 8, so the eight XCDs take
   // contiguous runs of tiles (whole matrices, sharing operands in their L2)
   int w = blockIdx.x;
   if ((gridDim.x & 7) == 0) w = (w & 7) * (gridDim.x >> 3) + (w >> 3);
   const int b = w / tiles, t = w - b * tiles;
-  const int i0 = (t % tm) * kGemmTile, j0 = (t / tm) * kTN;
+  int ti = t % tm, tj = t / tm;
+  if constexpr (kSym) {  // row block ti holds (ti + 1) (128 / kTN) tiles
+    ti = 0, tj = t;
+    for (int row = kGemmTile / kTN; tj >= row; row += kGemmTile / kTN) {
+      tj -= row;
+      ++ti;
+    }
+  }
+  const int i0 = ti * kGemmTile, j0 = tj * kTN;
+  const bool mirror = kSym && j0 + kTN <= i0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wi = wave & 1, wj = wave >> 1, l32 = lane & 31, g = lane >> 5;
 
@@ -531,6 +545,10 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
     if (a.gmode == 0) {
       __builtin_amdgcn_raw_buffer_store_b128(u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])},
                                              rd, out_off(t), 0, 0);
+      if (mirror && has_c) {  // the finished values, for the transposed pass
+        *reinterpret_cast<f32x4*>(const_cast<char*>(src)) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(const_cast<char*>(src) + 16) = f32x4{v[4], v[5], v[6], v[7]};
+      }
       continue;
     }
 #pragma unroll
@@ -543,6 +561,22 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
     } else {  // back into the quadrant, for the transposed pass
       *reinterpret_cast<f32x4*>(const_cast<char*>(src)) = f32x4{v[0], v[1], v[2], v[3]};
       *reinterpret_cast<f32x4*>(const_cast<char*>(src) + 16) = f32x4{v[4], v[5], v[6], v[7]};
+    }
+  }
+  if (mirror) {
+    // As the transposed G below, in bf16: lane l, pass t writes D(j, i) for
+    // eight consecutive j of quadrant row i = (64/kLpr) t + l/kLpr.
+    __syncthreads();
+    constexpr int kLpr = 4 * kNY;
+    const int c0 = 8 * (lane % kLpr);
+#pragma unroll
+    for (int t = 0; t < kPasses; ++t) {
+      const int r = (64 / kLpr) * t + lane / kLpr;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const float*>(quad + (c0 + e) * kQuadPitch + 4 * r);
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])},
+                                             rd, 2 * ((i0 + 64 * wi + r) * a.M + j0 + 32 * kNY * wj + c0), 0, 0);
     }
   }
   if (a.gmode == 2) {
@@ -582,20 +616,34 @@ int cu_count() {
   return c;
 }
 
-// Two stages (two workgroups per CU) when the grid fills the GPU twice over,
-// otherwise three (one workgroup per CU, two k steps in flight); products
-// whose 128 x 128 grid would leave CUs idle take 128 x 64 tiles.
-void polar_gemm(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus) {
-  const int64_t grid = (int64_t)(a.M / kGemmTile) * (a.N / kGemmTile) * batch;
-  const bool deep = grid < 2 * (int64_t)cus;
-  const dim3 g((unsigned)grid), b(256);
-  if (grid < (int64_t)cus) {
-    if (tr) hipLaunchKernelGGL((polar_gemm_kernel<true, 3, true>), dim3((unsigned)(2 * grid)), b, 0, s, a);
-    else hipLaunchKernelGGL((polar_gemm_kernel<false, 3, true>), dim3((unsigned)(2 * grid)), b, 0, s, a);
-  } else if (tr && deep) hipLaunchKernelGGL((polar_gemm_kernel<true, 3>), g, b, 0, s, a);
-  else if (tr) hipLaunchKernelGGL((polar_gemm_kernel<true, 2>), g, b, 0, s, a);
-  else if (deep) hipLaunchKernelGGL((polar_gemm_kernel<false, 3>), g, b, 0, s, a);
-  else hipLaunchKernelGGL((polar_gemm_kernel<false, 2>), g, b, 0, s, a);
+// One product.  128 x 128 tiles, or 128 x 64 when those would leave CUs idle;
+// three stages (one workgroup per CU, two k steps in flight) when the grid
+// leaves room for no more, else two (two workgroups per CU): 384 workgroups of
+// the narrow kind took two rounds at three stages (24 matrices of 384 x 384, 5
+// steps: 135 -> 124 us).
+template <bool kSym>
+void polar_launch(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus) {
+  const int64_t tm = a.M / kGemmTile, per = kSym ? tm * (tm + 1) / 2 : tm * (a.N / kGemmTile), grid = per * batch;
+  const bool narrow = grid < (int64_t)cus;
+  const dim3 g((unsigned)(narrow ? 2 * grid : grid)), b(256);
+  const bool deep = narrow ? 2 * grid <= (int64_t)cus : grid < (kSym ? 1 : 2) * (int64_t)cus;
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, s, a); };
+  if (narrow && deep) tr ? go(polar_gemm_kernel<true, 3, true, kSym>) : go(polar_gemm_kernel<false, 3, true, kSym>);
+  else if (narrow) tr ? go(polar_gemm_kernel<true, 2, true, kSym>) : go(polar_gemm_kernel<false, 2, true, kSym>);
+  else if (deep) tr ? go(polar_gemm_kernel<true, 3, false, kSym>) : go(polar_gemm_kernel<false, 3, false, kSym>);
+  else tr ? go(polar_gemm_kernel<true, 2, false, kSym>) : go(polar_gemm_kernel<false, 2, false, kSym>);
+}
+
+// A symmetric result (M = N) takes the lower tiles only where that saves a
+// round of workgroups, or where the full grid would leave CUs idle (what the
+// rest leaves free, the other stacks of a grouped call use).  16 matrices of 640 x
+// 640: 323 -> 232 us; for 32 of 512 x 512 both grids take two rounds and the
+// transposed stores made the call 282 us instead of 268, so they stay whole.
+void polar_gemm(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus, bool symmetric = false) {
+  const int64_t tm = a.M / kGemmTile, full = tm * (a.N / kGemmTile) * batch, lower = tm * (tm + 1) / 2 * batch;
+  auto rounds = [&](int64_t grid) { return (grid + cus - 1) / cus; };
+  if (symmetric && (full < (int64_t)cus || rounds(lower) < rounds(full))) polar_launch<true>(tr, a, batch, s, cus);
+  else polar_launch<false>(tr, a, batch, s, cus);
 }
 
 // The untransposed copy in (m <= n: X has G's layout): X = G / scale per
@@ -633,6 +681,47 @@ __global__ __launch_bounds__(256) void scale_copy_kernel(int64_t size, const flo
       for (int e = 0; e < 4; ++e) o[e] = v[e] / sc;
       *reinterpret_cast<f32x4*>(x + 4 * c) = o;
     }
+  }
+}
+
+// The transposed copy in for bf16 (m > n): X = (G / scale)^T in 64 x 64 tiles
+// through LDS, 16-byte loads along G's columns and 16-byte stores along X's (the
+// element-wise 32 x 32 copy took 25 us for 8 matrices of 2048 x 512, FIGURES_TR).
+// R, C multiples of 64, G and X 16-byte aligned; d (rows R, cols C), s as in
+// copy_scaled_kernel.
+__global__ __launch_bounds__(256) void copy_in_transposed_kernel(int R, int C, const float* src, bf16* dst,
+                                                                 const double* partial, float* scale_out) {
+  __shared__ float s_scale;
+  __shared__ float tile[64][65];  // [r][c]
+  if (threadIdx.x < 64) {
+    double v = partial[blockIdx.z * kNormParts + threadIdx.x];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    if (threadIdx.x == 0) {
+      s_scale = 1.01f * sqrtf((float)v) + 1e-6f;
+      if (blockIdx.x == 0 && blockIdx.y == 0) scale_out[blockIdx.z] = s_scale;
+    }
+  }
+  const int64_t mat = (int64_t)R * C;
+  const float* s = src + blockIdx.z * mat + (int64_t)(64 * blockIdx.x) * C + 64 * blockIdx.y;
+  bf16* d = dst + blockIdx.z * mat + (int64_t)(64 * blockIdx.y) * R + 64 * blockIdx.x;
+  f32x4 in[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    in[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(s + (int64_t)(16 * k + threadIdx.x / 16) * C + 4 * (threadIdx.x & 15)));
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[16 * k + threadIdx.x / 16][4 * (threadIdx.x & 15) + e] = in[k][e];
+  __syncthreads();
+  const float sc = s_scale;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = 32 * k + threadIdx.x / 8, r = 8 * (threadIdx.x & 7);
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = static_cast<bf16>(tile[r + e][c] / sc);
+    *reinterpret_cast<bf16x8*>(d + (int64_t)c * R + r) = o;
   }
 }
 
@@ -849,6 +938,8 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
     hipLaunchKernelGGL(scale_copy_kernel<bf16>, flat_grid, dim3(256), 0, s, msize, G, reinterpret_cast<bf16*>(X), partial, scale);
   } else if (flat) {
     hipLaunchKernelGGL(scale_copy_kernel<float>, flat_grid, dim3(256), 0, s, msize, G, reinterpret_cast<float*>(X), partial, scale);
+  } else if (half && transposed && lo % 64 == 0 && hi % 64 == 0 && aligned16(G) && aligned16(X)) {
+    hipLaunchKernelGGL(copy_in_transposed_kernel, dim3(lo / 64, hi / 64, k), dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
   } else if (half) {
     if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, bf16>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
     else hipLaunchKernelGGL((copy_scaled_kernel<false, float, bf16>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
@@ -868,10 +959,10 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
       bf16* a = reinterpret_cast<bf16*>(A);
       bf16* b = reinterpret_cast<bf16*>(B);
       // A = X X^T: P(i, p) = X(i, p), Q(p, j) = X(j, p), both contiguous in i, j
-      polar_gemm(true, PolarGemm{x, x, none, a, sx, sx, sa, lo, lo, lo, lo, hi, 1.0f, 0.0f}, k, s, cus);
+      polar_gemm(true, PolarGemm{x, x, none, a, sx, sx, sa, lo, lo, lo, lo, hi, 1.0f, 0.0f}, k, s, cus, true);
       // B = c A A + b A: Q(q, j) = A(q, j), contiguous in q; A is symmetric
       // (X X^T), so P(i, q) is read as A(q, i), also contiguous in q
-      polar_gemm(false, PolarGemm{a, a, a, b, sa, sa, sa, lo, lo, lo, lo, lo, c[2], c[1]}, k, s, cus);
+      polar_gemm(false, PolarGemm{a, a, a, b, sa, sa, sa, lo, lo, lo, lo, lo, c[2], c[1]}, k, s, cus, true);
       // Y = B X + a X: Q(q, p) = X(q, p), contiguous in q; P(i, q) read as
       // B(q, i) (B = c A A + b A is symmetric)
       // (the last step writes G itself: the bf16 iterate widened to fp32, as

@@ -253,3 +253,16 @@ def test_grouped_equals_separate_calls(gpu, compute_type):
     torch.cuda.synchronize()
     for a, b in zip(separate, grouped):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m,n,k", [(384, 384, 1), (640, 640, 11), (512, 512, 40), (2048, 128, 3), (128, 192, 300)])
+def test_polar_bf16_tile_choices(gpu, m, n, k):
+    """The library's GEMM in each tile width and stage count with whole and with
+    lower-tiles-only grids (transposed copies of the tiles below the diagonal),
+    the 64 x 64 transposed copy in, and its sizes' remainders."""
+    g = torch.Generator().manual_seed(m + n + k)
+    G = torch.randn(k, n, m, generator=g)
+    out = polar_express(G.to(gpu), compute_type=torch.bfloat16).cpu()
+    for j in sorted({0, k // 2, k - 1}):
+        ref = O.polar_express(G[j].numpy()[None], 5)[0]
+        assert rel_err(out[j].numpy(), ref) <= POLAR_TOL_BF16
