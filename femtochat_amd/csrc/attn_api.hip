@@ -204,6 +204,8 @@ fc_status fc_attn_fwd(const fc_attn_desc* desc, const void* Q, const void* K, co
   a.left = p.left;
   a.right = p.right;
   a.out_bf16 = p.out_bf16 ? 1 : 0;
+  e = fc::device_cus(&a.cus);
+  if (e != hipSuccess) return fail(FC_ERR_HIP, "forward: %s", hipGetErrorString(e));
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)p.D));
   e = fc::launch_fwd(p, a, s);
   if (e != hipSuccess) return fail(FC_ERR_HIP, "forward launch failed: %s", hipGetErrorString(e));
@@ -302,6 +304,8 @@ fc_status bwd_launch(const fc::Problem& p, const void* dO, const void* Q, const 
   a.right = p.right;
   a.grad_bf16 = p.grad_bf16 ? 1 : 0;
   a.accumulate = p.accumulate ? 1 : 0;
+  e = fc::device_cus(&a.cus);
+  if (e != hipSuccess) return fail(FC_ERR_HIP, "backward: %s", hipGetErrorString(e));
   a.scale = (float)(1.0 / std::sqrt((double)p.D));
   a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)p.D));
   if (fused_stats) {

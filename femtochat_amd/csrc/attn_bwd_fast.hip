@@ -60,7 +60,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_fast_kernel(BwdArgs a
   if (a.qorder != nullptr) {
     ordered_query_item(blockIdx.x, a.qorder, n_qt, a.H, a.Hkv, a.group, b, h, qt);
   } else {
-    const GridItem it0 = heavy_first(blockIdx.x, a.H * a.B);
+    const GridItem it0 = heavy_first(paired_position(blockIdx.x, (int)gridDim.x, a.cus), a.H * a.B);
     qt = n_qt - 1 - it0.rank;  // longest query tiles first
     query_row(it0.row, a.B, a.Hkv, a.group, b, h);
   }

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
   const int g = lane >> 5, l32 = lane & 31;
   const int T = a.T;
   const int n_qt = (T + kExactBM - 1) / kExactBM;
-  const GridItem it0 = heavy_first(blockIdx.x, a.H * a.B);
+  const GridItem it0 = heavy_first(paired_position(blockIdx.x, (int)gridDim.x, a.cus), a.H * a.B);
   const int qt = n_qt - 1 - it0.rank;  // longest query tiles first, over the whole grid
   int b, h;
   query_row(it0.row, a.B, a.Hkv, a.group, b, h);

@@ -27,6 +27,20 @@ struct GridItem {
 };
 FC_HD inline GridItem heavy_first(int id, int rows) { return {id % rows, id / rows}; }
 
+// Position in the heaviest-first list of workgroup id of a grid of n that two
+// workgroups per CU hold at once (cus < n <= 2 cus): the second workgroup of a
+// CU starts beside the heaviest first, so the part of the list beyond the first
+// cus goes out lightest first, in groups of eight that keep each item's XCD.
+// Larger grids refill slots as they empty and smaller ones have none to share:
+// the list's own order.  4 x 2048 tokens, H8 (512 workgroups), causal: dQ 44.6 ->
+// 42.4 us at D64 and 66.4 -> 62.8 at D128, the forward 52.1 -> 51.2 at D128, the
+// fp32 forward 127 -> 123 at D64; 2 x 2048, H10 (320): dQ 53.5 -> 52.0.
+FC_HD inline int paired_position(int id, int n, int cus) {
+  if (n <= cus || n > 2 * cus || id < cus) return id;
+  if (n % 8 == 0 && cus % 8 == 0) return n - 8 * ((id - cus) / 8 + 1) + id % 8;
+  return n - 1 - (id - cus);
+}
+
 // (batch, query head) of query-side row r, numbered KV group member outer
 // and (batch, KV head) inner: the heads that share a KV head are B*Hkv rows
 // apart, on one XCD whenever B*Hkv is divisible by 8.

@@ -23,6 +23,7 @@ struct FwdArgs {
   float* m;
   int H, Hkv, T, B, group, left, right;
   int out_bf16;
+  int cus;  // compute units (paired_position)
   float scale_log2;
 };
 
@@ -83,6 +84,7 @@ struct BwdArgs {
   int* queue;
   int H, Hkv, T, B, group, left, right;
   int grad_bf16, accumulate;
+  int cus;  // compute units (paired_position)
   float scale;       // 1/sqrt(D)
   float scale_log2;  // log2(e)/sqrt(D)
 };

@@ -245,9 +245,33 @@ static void grid_orders() {
   }
 }
 
+// paired_position (the order of grids of up to two workgroups per CU) is a
+// permutation that starts with the list's first cus items, puts the lightest
+// beside the heaviest, and keeps every id's XCD when the sizes divide into 8.
+static void paired_grids() {
+  for (int cus : {256, 304, 255}) {
+    for (int n : {1, 8, 255, 256, 257, 264, 320, 336, 399, 504, 512, 513, 608, 609, 2000}) {
+      std::vector<int> seen((size_t)n, 0);
+      bool ok = true;
+      for (int id = 0; id < n; ++id) {
+        const int at = fc::paired_position(id, n, cus);
+        ok = ok && at >= 0 && at < n;
+        if (at >= 0 && at < n) ++seen[at];
+        if (id < cus || n > 2 * cus) ok = ok && at == id;
+        if (n % 8 == 0 && cus % 8 == 0) ok = ok && at % 8 == id % 8;
+        if (n > cus && n <= 2 * cus && id >= cus && id < cus + 8) ok = ok && at >= n - 8;
+      }
+      for (int c : seen) ok = ok && c == 1;
+      if (!ok) std::fprintf(stderr, "paired order n=%d cus=%d\n", n, cus);
+      CHECK(ok);
+    }
+  }
+}
+
 int main() {
   validation();
   grid_orders();
+  paired_grids();
   restatement(16, 2, 1, 37, 2, -1, 0, 1, false);
   restatement(32, 4, 2, 600, 1, 100, 0, 0, false);  // two key blocks, a ragged one
   restatement(16, 2, 2, 530, 1, 50, 20, 0, true);
