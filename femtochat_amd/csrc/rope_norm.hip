@@ -22,9 +22,14 @@
 // Work split: one head vector per D/16 consecutive threads, each holding
 // eight rotation pairs (elements j..j+7 and j+d..j+d+7, one 16-byte bf16
 // load per half), so the rotation needs no cross-lane exchange and the sum
-// of squares is a butterfly over D/16 lanes; each thread takes four vectors
-// and issues all their loads before any arithmetic.  Memory-bound: a vector
-// is read and written once; the tables stay in L2.
+// of squares is a butterfly over D/16 lanes.  Memory-bound: a vector is read
+// and written once; the tables stay in L2.  Results are stored non-temporally:
+// the kernel never reads them and the stores leave the inputs in the caches.
+// 16 x 2048 tokens, D128, H10, bf16, packed positions: forward 67 -> 61 us of
+// Q and K together, backward 74 -> 65 (5.8 TB/s of its bytes); with H = Hkv =
+// 12 the backward 115 -> 102; 777 tokens, forward 18 -> 13.  Non-temporal loads
+// as well measured slower (the gradient at D64 32 -> 39: its inputs fit the
+// last-level cache).
 #include <type_traits>
 
 #include "attn_launch.hpp"
@@ -100,8 +105,8 @@ struct Eight<float> {
       a += *reinterpret_cast<const f32x4*>(p);
       b += *reinterpret_cast<const f32x4*>(p + 4);
     }
-    *reinterpret_cast<f32x4*>(p) = a;
-    *reinterpret_cast<f32x4*>(p + 4) = b;
+    __builtin_nontemporal_store(a, reinterpret_cast<f32x4*>(p));
+    __builtin_nontemporal_store(b, reinterpret_cast<f32x4*>(p + 4));
   }
 };
 
@@ -127,7 +132,7 @@ struct Eight<bf16> {
 #pragma unroll
       for (int i = 0; i < 8; ++i) w[i] += static_cast<float>(o[i]);
     }
-    *reinterpret_cast<bf16x8*>(p) = __builtin_convertvector(w, bf16x8);
+    __builtin_nontemporal_store(__builtin_convertvector(w, bf16x8), reinterpret_cast<bf16x8*>(p));
   }
 };
 
@@ -234,55 +239,47 @@ struct Share {
 // Thread geometry: G = D/16 lanes per vector, each thread NV vectors spaced
 // by the number of groups in the grid (consecutive groups take consecutive
 // vectors, so a wave's loads are contiguous); every load of a thread is
-// issued before its arithmetic.  The forward takes four vectors per thread,
-// the backward (which holds dY too) two: the fastest of 2, 4 and 8 for each.
-// (The forward is bound by its VALU instructions, about 25 per element for
-// bf16 at four cycles each; a grid-stride loop that prefetches the next
-// sweep's loads during the current sweep's arithmetic measured slower.)
-constexpr int kFwdNV = 4, kBwdNV = 2;
+// issued before its arithmetic.  The forward takes one vector per thread (37
+// registers, eight waves per SIMD; two and four vectors: 60 and 61-66 us of
+// the case above), the backward two (one: fp32 135 -> 150 us, three: bf16 D64
+// 32 -> 35).  Five heads of a token per thread with their table entries
+// loaded once measured slower (68 and 80 us: fewer waves).
+constexpr int kBwdNV = 2;
 
 template <int D, typename E, bool kPos>
 __global__ __launch_bounds__(256) void rope_norm_fwd_kernel(RopeNormArgs a) {
-  constexpr int G = D / 16, d = D / 2, kNV = kFwdNV;
+  constexpr int G = D / 16, d = D / 2;
   constexpr bool kB = sizeof(E) == 2;
-  const uint32_t tid = blockIdx.x * 256 + threadIdx.x;
-  const int j0 = 8 * (int)(tid % G);
-  const uint32_t group = tid / G, ngroups = gridDim.x * (256 / G);
-  Share<D, E> sh[kNV];
+  const int j0 = 8 * (int)(threadIdx.x % G);
+  const uint32_t vec = (blockIdx.y * gridDim.x + blockIdx.x) * (256 / G) + threadIdx.x / G;
+  const uint32_t last = (uint32_t)a.vectors - 1;
+  const uint32_t src = min(vec, last);  // clamped: loads stay in range
+  Share<D, E> sh;
+  sh.load(static_cast<const E*>(a.X) + (int64_t)src * D, a.sin_t, a.cos_t, position_of<kPos>(a, src), a.table_len, j0);
+  sh.rotate();
+  const float r = sh.rms();
+  if (vec > last) return;  // whole groups (G divides 64), after the group's shuffles
+  E* yv = static_cast<E*>(a.Y) + (int64_t)vec * D;
+  // y = bf(bf(u / r) * 1.2) (fp32: u / r * 1.2); each branch computes and
+  // stores on its own so no array lives across the branch.
+  auto emit = [&](auto div) __attribute__((always_inline)) {
+    float t1[8], t2[8];
 #pragma unroll
-  for (int k = 0; k < kNV; ++k) {
-    const uint32_t vec = min(group + k * ngroups, (uint32_t)a.vectors - 1);  // clamped: loads stay in range
-    sh[k].load(static_cast<const E*>(a.X) + (int64_t)vec * D, a.sin_t, a.cos_t, position_of<kPos>(a, vec),
-               a.table_len, j0);
-  }
-#pragma unroll
-  for (int k = 0; k < kNV; ++k) {
-    const uint32_t vec = group + k * ngroups;
-    sh[k].rotate();
-    const float r = sh[k].rms();
-    if (vec >= (uint32_t)a.vectors) continue;  // whole groups (G divides 64), after the group's shuffles
-    E* yv = static_cast<E*>(a.Y) + (int64_t)vec * D;
-    // y = bf(bf(u / r) * 1.2) (fp32: u / r * 1.2); each branch computes and
-    // stores on its own so no array lives across the branch.
-    auto emit = [&](auto div) __attribute__((always_inline)) {
-      float t1[8], t2[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        t1[i] = div(sh[k].x1[i]);
-        t2[i] = div(sh[k].x2[i]);
-        if (kB) bf2(t1[i], t2[i]);
-        t1[i] *= 1.2f;
-        t2[i] *= 1.2f;
-      }
-      Eight<E>::store(yv + j0, t1, false);
-      Eight<E>::store(yv + d + j0, t2, false);
-    };
-    if (sh[k].fast_quotient(r)) {
-      const float y = 1.0f / r;
-      emit([&](float u) __attribute__((always_inline)) { return quotient(u, r, y); });
-    } else {
-      emit([&](float u) __attribute__((always_inline)) { return u / r; });
+    for (int i = 0; i < 8; ++i) {
+      t1[i] = div(sh.x1[i]);
+      t2[i] = div(sh.x2[i]);
+      if (kB) bf2(t1[i], t2[i]);
+      t1[i] *= 1.2f;
+      t2[i] *= 1.2f;
     }
+    Eight<E>::store(yv + j0, t1, false);
+    Eight<E>::store(yv + d + j0, t2, false);
+  };
+  if (sh.fast_quotient(r)) {
+    const float y = 1.0f / r;
+    emit([&](float u) __attribute__((always_inline)) { return quotient(u, r, y); });
+  } else {
+    emit([&](float u) __attribute__((always_inline)) { return u / r; });
   }
 }
 
@@ -297,7 +294,8 @@ __global__ __launch_bounds__(256) void rope_norm_bwd_kernel(RopeNormArgs a) {
 #pragma unroll
   for (int k = 0; k < kNV; ++k) {
     const uint32_t vec = min(group + k * ngroups, (uint32_t)a.vectors - 1);
-    sh[k].load(static_cast<const E*>(a.X) + (int64_t)vec * D, a.sin_t, a.cos_t, position_of<kPos>(a, vec), a.table_len, j0);
+    sh[k].load(static_cast<const E*>(a.X) + (int64_t)vec * D, a.sin_t, a.cos_t, position_of<kPos>(a, vec),
+               a.table_len, j0);
     Eight<E>::load(static_cast<const E*>(a.dY) + (int64_t)vec * D + j0, g1[k]);
     Eight<E>::load(static_cast<const E*>(a.dY) + (int64_t)vec * D + d + j0, g2[k]);
   }
@@ -335,9 +333,12 @@ __global__ __launch_bounds__(256) void rope_norm_bwd_kernel(RopeNormArgs a) {
 template <int D, typename E>
 hipError_t launch_t(const RopeNormArgs& a, bool backward, hipStream_t s) {
   constexpr int G = D / 16;
-  const int nv = backward ? kBwdNV : kFwdNV;
+  const int nv = backward ? kBwdNV : 1;
   const int64_t groups = ((int64_t)a.vectors + nv - 1) / nv;
-  const dim3 grid((unsigned)((groups * G + 255) / 256)), block(256);
+  // (x is bounded by 2^31 threads: 2^30 vectors of one group each reach past a
+  // dimension's 2^32; only the forward can, by memory.)
+  const int64_t blocks = (groups * G + 255) / 256, nx = blocks < (1 << 23) || backward ? blocks : 1 << 23;
+  const dim3 grid((unsigned)nx, (unsigned)((blocks + nx - 1) / nx)), block(256);
   const ProfileMark mk = profile_begin(s);
   if (backward) {
     if (a.pos) hipLaunchKernelGGL((rope_norm_bwd_kernel<D, E, true>), grid, block, 0, s, a);

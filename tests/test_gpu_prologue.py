@@ -14,7 +14,8 @@ import numpy as np
 import pytest
 import torch
 
-from femtochat_amd import AttentionPrologueFunction, attention_prologue, delta_attention_prologue_, rotary_embeddings
+from femtochat_amd import (AttentionPrologueFunction, attention_prologue, attention_prologue_,
+                           delta_attention_prologue_, rotary_embeddings)
 from femtochat_amd import _lib
 from oracle import rope_norm as R
 
@@ -183,3 +184,27 @@ def test_extreme_magnitudes_take_the_exact_division(gpu, dtype):
         u = _ulp_bf16(Y, ref)
         assert np.max(u) <= 2.0
     assert np.all(Y[0, 1, 1] == 0) and np.all(Y[0, 3, 3] == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [16, 128])
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_edges_of_a_workgroup(gpu, dtype, D, over):
+    """Vector counts around a workgroup's 256 * 16 / D (forward) and twice that
+    (backward): the values of the same tokens in a larger call bit for bit, and
+    nothing written past the end (in place too, where a thread without a vector
+    still loads the last one)."""
+    T = 2 * 256 * 16 // D + over
+    X, _, _, _, Xd, tabs, _ = _case(gpu, 1, T + 64, 1, D, dtype, None, seed=5)
+    dYd = torch.randn(X.shape, generator=torch.Generator().manual_seed(6)).to(dtype).to(gpu)
+    whole, dwhole = attention_prologue(Xd, tabs), torch.empty_like(Xd)
+    delta_attention_prologue_(dwhole, dYd, Xd, tabs, accumulate=False)
+    for n in (T, T // 2):
+        Y, dX = torch.full_like(Xd, 7.0), torch.full_like(Xd, 7.0)
+        attention_prologue_(Y[:, :n], Xd[:, :n], tabs)
+        delta_attention_prologue_(dX[:, :n], dYd[:, :n], Xd[:, :n], tabs, accumulate=False)
+        assert torch.equal(Y[:, :n], whole[:, :n]) and torch.equal(dX[:, :n], dwhole[:, :n])
+        assert (Y[:, n:] == 7.0).all() and (dX[:, n:] == 7.0).all()
+        Z = Xd.clone()
+        attention_prologue_(Z[:, :n], Z[:, :n], tabs)
+        assert torch.equal(Z[:, :n], whole[:, :n]) and torch.equal(Z[:, n:], Xd[:, n:])
