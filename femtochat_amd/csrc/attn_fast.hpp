@@ -122,6 +122,12 @@ struct FragOffsets {
       tr_base[e] = Tile::offset(r, u) + 8 * (cc & 1);  // column block 0; block db is ^ 64db
     }
   }
+  // Moves every offset by whole rows (a multiple of what the XORs above flip).
+  __device__ inline void shift(int bytes) {
+    nat_base += bytes;
+    tr_base[0] += bytes;
+    tr_base[1] += bytes;
+  }
   __device__ inline int nat(int c) const { return nat_base ^ (32 * c); }
   __device__ inline int tr(int e, int db) const { return tr_base[e] ^ (64 * db); }
 };

@@ -25,7 +25,8 @@
 // which the row sees a key (O and l are still zero then; its largest P is
 // exactly 1, as with a running maximum) and is never moved, so O is never
 // rescaled: probabilities may grow up to 2^64 against m_ref, which fp32 and
-// bf16 hold with the same relative precision as values near 1.  A
+// bf16 hold with the same relative precision as values near 1 (each part of the
+// key tiles has its own, and the parts meet at the larger one).  A
 // block maximum beyond that flags the wave, which then recomputes its rows
 // after the tile loop with a plain two-pass method (exact maximum first)
 // reading K and V from global memory.  P is rounded to bf16 against m_ref and
@@ -87,8 +88,12 @@ __device__ inline float max16(const f32x16& s) {
   return m;
 }
 
-template <int D>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
+// kParts 2 (grids that leave at most one workgroup on a CU): eight waves, of
+// which waves 4 .. 7 take the odd key tiles of the same 128 queries through
+// stage buffers of their own, so that a wave's chain of tiles is half as long
+// and each SIMD has two waves, as with two workgroups per CU.
+template <int D, int kParts>
+__global__ __launch_bounds__(kThreads * kParts, 2 / kParts) void attn_fwd_fast_kernel(FwdArgs a) {
   using C = FwdFastCfg<D>;
   using M = Mma<bf16>;
   constexpr int BN = C::kBN, KC = C::kKC, DB = C::kDB, NQB = C::kNQB, NKB = C::kNKB;
@@ -96,11 +101,19 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
   constexpr int kSchedVALU = 0x2, kSchedMFMA = 0x8, kSchedDSRead = 0x100;
   // Two stage buffers as distinct objects, so the compiler can tell the LDS
   // loads of one from the DMA writes into the other.
-  __shared__ __attribute__((aligned(1024))) char bufA[C::kStageBytes];
-  __shared__ __attribute__((aligned(1024))) char bufB[C::kStageBytes];
+  constexpr int kOBytes = kThreads * 16 * DB * 4;  // the second part's O (kParts 2)
+  __shared__ __attribute__((aligned(1024))) char
+      bufA[kParts == 2 && kOBytes > 2 * C::kStageBytes ? kOBytes : kParts * C::kStageBytes];
+  __shared__ __attribute__((aligned(1024))) char bufB[kParts * C::kStageBytes];
   __shared__ int s_bounds[2][kWaves];
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lane = threadIdx.x & 63;
+  int wave = (int)threadIdx.x >> 6, part = 0;
+  if (kParts == 2) {  // waves 4 .. 7 are the second part
+    wave = __builtin_amdgcn_readfirstlane(wave);
+    part = wave / kWaves;
+    wave %= kWaves;
+  }
   const int g = lane >> 5, l32 = lane & 31;
   const int T = a.T;
   const int n_qt = (T + C::kBM - 1) / C::kBM;
@@ -166,6 +179,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
 
   FragOffsets<C::kW> fo;
   fo.init(lane);
+  if (kParts > 1) fo.shift(part * C::kStageBytes);
   DmaPlan<D, BN> plan;
   plan.init(wave, lane, kpitch);
 
@@ -212,7 +226,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
     }
   };
   auto issue = [&](int it, char* buf) {
-    nx_at = lds_addr(buf);
+    nx_at = lds_addr(buf) + part * C::kStageBytes;
     if (it < ntiles) {
       const int64_t row0 = (int64_t)(kt0 + it * BN) * kpitch;
       nx_k = tile_words(Kb, krec, row0);
@@ -324,19 +338,62 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
   };
 
   if (ntiles > 0) {
-    issue(0, bufA);
+    issue(part, bufA);
 #pragma unroll
     for (int k = 0; k < NDMA; ++k) dma_part(k);
   }
   dma_wait_barrier();
-  for (int it = 0; it < ntiles; it += 2) {
-    issue(it + 1, bufB);
-    compute(it, bufA);
+  // (A part without a tile in a step sees nothing of the tile past the last.)
+  for (int it = 0; it < ntiles; it += 2 * kParts) {
+    issue(it + part + kParts, bufB);
+    compute(it + part, bufA);
     dma_wait_barrier();
-    if (it + 1 >= ntiles) break;
-    issue(it + 2, bufA);
-    compute(it + 1, bufB);
+    if (it + kParts >= ntiles) break;
+    issue(it + part + 2 * kParts, bufA);
+    compute(it + part + kParts, bufB);
     dma_wait_barrier();
+  }
+
+  if constexpr (kParts == 2) {
+    // The parts meet in LDS: each row's sums go to the larger of the two
+    // references (each part's P, relative to its own, is at most 2^64, so what
+    // a factor loses to underflow is below 2^-62 of the row).
+    float* const so = reinterpret_cast<float*>(bufA);
+    float* const ss = reinterpret_cast<float*>(bufB);
+    const int tid = 64 * wave + __lane_id();
+    if (part == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          *reinterpret_cast<f32x4*>(so + 4 * ((4 * db + j) * kThreads + tid)) =
+              f32x4{o[0][db][4 * j], o[0][db][4 * j + 1], o[0][db][4 * j + 2], o[0][db][4 * j + 3]};
+        }
+      }
+      *reinterpret_cast<f32x4*>(ss + 4 * tid) = f32x4{m_ref[0], m_true[0], l_half[0], flag ? 1.0f : 0.0f};
+    }
+    __syncthreads();
+    if (part == 0) {
+      const f32x4 other = *reinterpret_cast<const f32x4*>(ss + 4 * tid);
+      const float ref = nan_max(m_ref[0], other[0]);
+      const float f0 = m_ref[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_ref[0] - ref);
+      const float f1 = other[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(other[0] - ref);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(so + 4 * ((4 * db + j) * kThreads + tid));
+#pragma unroll
+          for (int t = 0; t < 4; ++t) o[0][db][4 * j + t] = o[0][db][4 * j + t] * f0 + v[t] * f1;
+        }
+      }
+      l_half[0] = l_half[0] * f0 + other[2] * f1;
+      m_ref[0] = ref;
+      m_true[0] = nan_max(m_true[0], other[1]);
+      flag |= other[3] != 0.0f;
+    }
+    __syncthreads();  // O leaves through the same memory
+    if (part == 1) return;
   }
 
   if (__builtin_amdgcn_ballot_w64(flag) != 0) {
@@ -462,9 +519,19 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_fast_kernel(FwdArgs a) {
 template <int D>
 static hipError_t launch_fwd_fast_t(const Problem& p, const FwdArgs& a, hipStream_t s) {
   const int n_qt = (p.T + FwdFastCfg<D>::kBM - 1) / FwdFastCfg<D>::kBM;
-  const dim3 grid(n_qt * p.H * p.B), block(kThreads);
+  const dim3 grid(n_qt * p.H * p.B);
   const ProfileMark mk = profile_begin(s);
-  hipLaunchKernelGGL((attn_fwd_fast_kernel<D>), grid, block, 0, s, a);
+  // Key tiles in two parts when at most one workgroup per CU would run and some
+  // row's workgroup can see more than ten tiles.  8 heads, causal, one part ->
+  // two, us: T 512 (8 tiles) 15.4 -> 15.8 at D128, 12.9 -> 12.3 at D64; T 777
+  // 24.8 -> 21.7, 21.2 -> 18.0; T 2048 39.7 -> 35.4, 31.9 -> 27.0; 4 heads of
+  // 8192 148 -> 118, 107 -> 85.  A window of 512 (ten tiles): 18.0 -> 18.0; of 128
+  // 12.1 -> 13.2.
+  constexpr int kPartTiles = 10;
+  const int64_t span = std::min((int64_t)p.T, (int64_t)a.left + a.right + FwdFastCfg<D>::kBM);
+  const bool parts = (int64_t)grid.x <= a.cus && span > kPartTiles * FwdFastCfg<D>::kBN;
+  if (parts) hipLaunchKernelGGL((attn_fwd_fast_kernel<D, 2>), grid, dim3(2 * kThreads), 0, s, a);
+  else hipLaunchKernelGGL((attn_fwd_fast_kernel<D, 1>), grid, dim3(kThreads), 0, s, a);
   const hipError_t e = hipGetLastError();
   profile_end(mk, "attn_fwd_bf16", s);
   return e;
