@@ -73,10 +73,12 @@ __device__ inline float max_abs8(const float (&x)[8]) {
   for (int e = 1; e < 8; ++e) m = __builtin_elementwise_maximum(m, __builtin_fabsf(x[e]));
   return m;
 }
+// Of the first N elements of an accumulator (8: its rows 0 .. 15).
+template <int N = 16>
 __device__ inline float max_abs16(const f32x16& c) {
   float m = __builtin_fabsf(c[0]);
 #pragma unroll
-  for (int r = 1; r < 16; ++r) m = __builtin_elementwise_maximum(m, __builtin_fabsf(c[r]));
+  for (int r = 1; r < N; ++r) m = __builtin_elementwise_maximum(m, __builtin_fabsf(c[r]));
   return m;
 }
 __device__ inline bool outside_split(float max_abs) {
@@ -109,7 +111,7 @@ __device__ inline void mma_split_pair(const Split8& a0, const Split8& b0, f32x16
 // A tile of 32 token rows x D in LDS: three swizzled bf16 tiles, one per part.
 template <int D>
 struct SplitTile {
-  static constexpr int kW = tile_width(D);  // values past D are never used
+  static constexpr int kW = tile_width(D);  // values past D are never written: rows they reach mean nothing
   using Tile = SwzTile<kW>;
   static constexpr int kPlane = 32 * Tile::kRowBytes;
   static constexpr int kBytes = 3 * kPlane;

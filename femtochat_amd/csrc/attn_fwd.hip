@@ -172,8 +172,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
 
   // Probabilities above 1 may have carried a sum past the float32 range that
   // those against the exact maximum stay in.
+  // (The last block's rows past the head dim come from LDS that nothing wrote.)
 #pragma unroll
-  for (int db = 0; db < DB; ++db) grown |= !(max_abs16(o[db]) < INFINITY);
+  for (int db = 0; db < D / 32; ++db) grown |= !(max_abs16(o[db]) < INFINITY);
+  if (D % 32 != 0) grown |= !(max_abs16<8>(o[DB - 1]) < INFINITY);
   if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
   __syncthreads();
   if (s_outside != 0 || __builtin_amdgcn_ballot_w64(grown) != 0) {

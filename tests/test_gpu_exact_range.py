@@ -16,7 +16,7 @@ import torch
 from femtochat_amd import MFMAExact
 from femtochat_amd import kernels as Kn
 from oracle import attention_ref as R
-from tests.helpers import TOL, rel_err, to_np
+from tests.helpers import TOL, gpu_forward, rel_err, to_np
 
 pytestmark = pytest.mark.gpu
 BOUND = 4e-5
@@ -104,3 +104,20 @@ def test_growing_scores(gpu, D):
     # scores of up to 600 carry a rounding of 600 log2(e) 2^-24 in the exponent
     for x, r in zip((O, dV), (O_ref, g_ref[2])):
         assert rel_err(x, r) <= 3 * TOL["exact"]
+
+
+@pytest.mark.parametrize("D", [16, 48, 80, 112])
+def test_head_dims_between_blocks_ignore_old_lds(gpu, D):
+    """Tiles of these head dims leave LDS columns unwritten (or read past 16 of
+    them): what an earlier launch left there must not send rows to the
+    recomputation.  The same bits after a launch that fills LDS with NaN as after
+    one that fills it with ones."""
+    g = torch.Generator(device=gpu).manual_seed(D)
+    Q, K, V = (torch.randn(2, 200, 4, D, device=gpu, generator=g) for _ in range(3))
+    results = []
+    for fill in (float("nan"), 1.0):
+        X = torch.full((8, 1024, 16, 128), fill, device=gpu)  # enough workgroups for every CU
+        gpu_forward(MFMAExact(), X, X, X, (-1, 0))
+        results.append(gpu_forward(MFMAExact(), Q, K, V, (-1, 0)))
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
