@@ -170,9 +170,8 @@ inline Problem kernel_problem(const Problem& p, bool backward) {
 // What the workspace of head dims 48, 80, 96 and 112 begins with (byte
 // offsets, 256-aligned): room for Q, K, V (input format), O (its format), and
 // in the backward dO (its format) and float32 dQ, dK, dV with rows of Dk
-// values.  The kernels once ran on zero-padded copies held there and no longer
-// touch it, but the sizes fc_attn_workspace_bytes gives, and the forward's
-// refusal to run without a workspace, are what callers were built against.
+// values.  The kernels run on the caller's rows; a tensor off a 16-byte
+// boundary goes through its place here (attn_api.hip, needs_room).
 // The kernels' own workspace follows at `inner`.
 struct PadWorkspace {
   size_t Q, K, V, O, dO, dQ, dK, dV, inner;

@@ -95,8 +95,8 @@ fc_status fc_attn_workspace_bytes(const fc_attn_desc* desc, int32_t pass,
    fc_attn_workspace_bytes(FC_PASS_FORWARD) bytes, 256-byte aligned, lets the
    kernel take the query tiles in order of decreasing work (long documents
    first); the results are the same.  At every other head_dim (48, 80, 96,
-   112) the workspace is required (FC_ERR_WORKSPACE without it; the kernels
-   read and write the caller's rows directly and leave most of it alone). */
+   112) the workspace is required (FC_ERR_WORKSPACE without it): tensors off a
+   16-byte boundary are copied through it; others are used in place. */
 fc_status fc_attn_fwd(const fc_attn_desc* desc, const void* Q, const void* K,
                       const void* V, const int32_t* positions, void* O,
                       float* l, float* m, void* workspace,
