@@ -252,8 +252,6 @@ def _desc(A, Q, K, window, out_dtype, dout_dtype, grad_dtype, overwrite=False) -
         raise TypeError(f"expected MFMAExact() or MFMAFast(), got {A!r}")
     if Q.dim() != 4 or K.dim() != 4:
         raise ValueError("Q, K, V must be 4-d (B, T, H, D) tensors")
-    if Q.dim() != 4 or K.dim() != 4:
-        raise ValueError("Q, K, V must be 4-d (B, T, H, D) tensors")
     B, T, H, D = Q.shape
     return _lib.AttnDesc(D, H, K.shape[2], T, B, int(window[0]), int(window[1]), A.mode, _dtype_code(Q.dtype), out_dtype,
                          dout_dtype, grad_dtype, _lib.FC_FLAG_OVERWRITE if overwrite else 0)
