@@ -11,7 +11,7 @@
 // Frobenius norm (a two-stage float64 reduction), copies it into the iteration
 // buffer (transposed through LDS when m > n, so the Gram matrix is the
 // smaller one) and runs three batched products per step with the elementwise
-// terms folded into their beta: in bf16, for sizes that are multiples of 128,
+// terms folded into their beta: in bf16, for sizes that are multiples of 64,
 // the MFMA kernel below (whose last product writes the result), otherwise
 // strided-batched rocBLAS GEMMs followed by a copy back.
 #include "../../include/femtochat_optim.h"
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256) void copy_scaled_kernel(int R, int C, const S*
 // The epilogue leaves through LDS: each wave writes its fp32 quadrant by
 // column (padded), then eight lanes cover one 128-byte column segment of D,
 // adding beta C (loaded in that layout before the k loop) and rounding once.
-// M, N multiples of 128, K a multiple of 64, every operand under 2^31 bytes
+// M, N, K multiples of 64, every operand under 2^31 bytes
 // (checked by the caller): all tiles are whole and every offset is 32-bit.
 struct PolarGemm {
   const bf16* P;
@@ -362,6 +362,9 @@ __device__ inline void wait_vmcnt() {
 // and each one below it is also written transposed to its place above; D is then
 // its own transpose bit for bit.  A of 8 matrices of 512 x 2048 in a grouped call:
 // 27 -> 18.5 us.
+// M, N and K are multiples of 64: in the last tile of an odd multiple the waves
+// past the edge multiply what they find (values of the matrix or zeros), and
+// their descriptors without records drop what they store.
 template <bool kTr, int kStages, bool kNarrow = false, bool kSym = false>
 __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(PolarGemm a) {
   constexpr int kTN = kNarrow ? 64 : kGemmTile;  // tile width (j)
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
   constexpr int kLds = kStageBytes * kStages > 4 * kQuadBytes ? kStageBytes * kStages : 4 * kQuadBytes;
   __shared__ __attribute__((aligned(1024))) char lds[kLds];
   auto tile = [&](int stage, int which) __attribute__((always_inline)) { return lds + kStageBytes * stage + 16384 * which; };
-  const int tm = a.M / kGemmTile, tiles = kSym ? tm * (tm + 1) / (kNarrow ? 1 : 2) : tm * (a.N / kTN);
+  const int tm = (a.M + kGemmTile - 1) / kGemmTile, tiles = kSym ? tm * (tm + 1) / (kNarrow ? 1 : 2) : tm * ((a.N + kTN - 1) / kTN);
   // XCD-aware order: workgroup w runs on XCD w mod 8, so the eight XCDs take
   // contiguous runs of tiles (whole matrices, sharing operands in their L2)
   int w = blockIdx.x;
@@ -436,7 +439,8 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
   // 8t + l/8 of its quadrant, rows 8 (l mod 8) .. +7 (16 bytes of bf16), so
   // eight lanes write one whole 128-byte column segment.  C is loaded in the
   // same layout before the k loop (its loads complete under the first wait).
-  const int64_t dbytes = (int64_t)a.M * a.N * 2;
+  const bool live = __builtin_amdgcn_readfirstlane((int)(i0 + 64 * wi < a.M && j0 + 32 * kNY * wj < a.N)) != 0;
+  const int64_t dbytes = live ? (int64_t)a.M * a.N * 2 : 0;
   const auto rd = make_rsrc(a.D + b * a.sd, (uint32_t)dbytes);
   const bool has_c = a.beta != 0.0f;  // without C the loads read zero records: no memory access
   const auto rc = make_rsrc(has_c ? a.C + b * a.sd : a.D, has_c ? (uint32_t)dbytes : 0u);
@@ -601,9 +605,13 @@ __global__ __launch_bounds__(256, kStages == 2 ? 2 : 1) void polar_gemm_kernel(P
   }
 }
 
-// True when the Polar Express products of these sizes fit polar_gemm_kernel.
+// True when the Polar Express products of these sizes fit polar_gemm_kernel.  Sizes
+// that are odd multiples of 64 leave half of their last tiles idle and are still
+// faster here than through rocBLAS's batched products (its host time per call
+// included): one Muon step of 12 layers, n_embed 64 / 192 / 320: 843 / 871 / 851 us
+// there, 223 / 242 / 486 here; 1 layer: 857 / 843 / 848 and 231 / 232 / 244.
 bool polar_gemm_fits(int lo, int hi) {
-  return lo % kGemmTile == 0 && hi % kGemmTile == 0 && (int64_t)lo * hi * 4 < ((int64_t)1 << 31);
+  return lo % kGemmK == 0 && hi % kGemmK == 0 && (int64_t)lo * hi * 4 < ((int64_t)1 << 31);
 }
 
 // Compute units of the current device (cached per device).
@@ -623,10 +631,12 @@ int cu_count() {
 // steps: 135 -> 124 us).
 template <bool kSym>
 void polar_launch(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus) {
-  const int64_t tm = a.M / kGemmTile, per = kSym ? tm * (tm + 1) / 2 : tm * (a.N / kGemmTile), grid = per * batch;
-  const bool narrow = grid < (int64_t)cus;
-  const dim3 g((unsigned)(narrow ? 2 * grid : grid)), b(256);
-  const bool deep = narrow ? 2 * grid <= (int64_t)cus : grid < (kSym ? 1 : 2) * (int64_t)cus;
+  const int64_t tm = (a.M + kGemmTile - 1) / kGemmTile;
+  const int64_t wide = (kSym ? tm * (tm + 1) / 2 : tm * ((a.N + kGemmTile - 1) / kGemmTile)) * batch;
+  const bool narrow = wide < (int64_t)cus;
+  const int64_t grid = !narrow ? wide : kSym ? 2 * wide : tm * ((a.N + 63) / 64) * batch;
+  const dim3 g((unsigned)grid), b(256);
+  const bool deep = narrow ? grid <= (int64_t)cus : grid < (kSym ? 1 : 2) * (int64_t)cus;
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, s, a); };
   if (narrow && deep) tr ? go(polar_gemm_kernel<true, 3, true, kSym>) : go(polar_gemm_kernel<false, 3, true, kSym>);
   else if (narrow) tr ? go(polar_gemm_kernel<true, 2, true, kSym>) : go(polar_gemm_kernel<false, 2, true, kSym>);
@@ -640,7 +650,8 @@ void polar_launch(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus
 // 640: 323 -> 232 us; for 32 of 512 x 512 both grids take two rounds and the
 // transposed stores made the call 282 us instead of 268, so they stay whole.
 void polar_gemm(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus, bool symmetric = false) {
-  const int64_t tm = a.M / kGemmTile, full = tm * (a.N / kGemmTile) * batch, lower = tm * (tm + 1) / 2 * batch;
+  const int64_t tm = (a.M + kGemmTile - 1) / kGemmTile, full = tm * ((a.N + kGemmTile - 1) / kGemmTile) * batch;
+  const int64_t lower = tm * (tm + 1) / 2 * batch;
   auto rounds = [&](int64_t grid) { return (grid + cus - 1) / cus; };
   if (symmetric && (full < (int64_t)cus || rounds(lower) < rounds(full))) polar_launch<true>(tr, a, batch, s, cus);
   else polar_launch<false>(tr, a, batch, s, cus);

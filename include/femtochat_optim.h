@@ -79,7 +79,7 @@ fc_status fc_polar_workspace_bytes(const fc_polar_desc* desc, size_t* bytes);
    then per step A = X X^T, B = b A + c A A, X = a X + B X, and G = X (or
    X^T), with b A and a X folded into the products' beta terms (the
    reference's CUBLAS gemmStridedBatchedEx, ext/FemtoChatCUDAExt.jl:121-125).
-   In bf16 with min(m, n) and max(m, n) multiples of 128 the products are the
+   In bf16 with min(m, n) and max(m, n) multiples of 64 the products are the
    library's own MFMA kernels (the last one writes G); otherwise they are
    strided-batched rocBLAS GEMMs, whose handle (one per device, created on
    the first such call) owns rocBLAS's own device workspace.  Everything else

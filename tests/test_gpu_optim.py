@@ -172,7 +172,7 @@ def _torch_polar_bf16(G):
     return torch.stack(out)
 
 
-# sizes that are multiples of 128 run the library's own MFMA GEMM (128 x 64 tiles
+# sizes that are multiples of 64 run the library's own MFMA GEMM (128 x 64 tiles
 # for grids below the CU count), the others rocBLAS
 @pytest.mark.parametrize("m,n,k", [(64, 64, 3), (160, 48, 2), (128, 128, 3), (256, 384, 2), (384, 256, 2),
                                    (512, 512, 4), (512, 2048, 1), (2048, 512, 1),
@@ -263,6 +263,21 @@ def test_polar_bf16_tile_choices(gpu, m, n, k):
     g = torch.Generator().manual_seed(m + n + k)
     G = torch.randn(k, n, m, generator=g)
     out = polar_express(G.to(gpu), compute_type=torch.bfloat16).cpu()
+    for j in sorted({0, k // 2, k - 1}):
+        ref = O.polar_express(G[j].numpy()[None], 5)[0]
+        assert rel_err(out[j].numpy(), ref) <= POLAR_TOL_BF16
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 64, 1), (64, 4096, 70), (192, 192, 2), (192, 192, 150), (192, 768, 3), (768, 192, 3),
+                                   (320, 320, 40), (1280, 320, 12), (448, 64, 150)])
+def test_polar_bf16_odd_multiples_of_64(gpu, m, n, k):
+    """Sizes whose last 128-wide tile is half outside the matrix, in each tile
+    width, with and without lower-tiles-only grids, transposed and not.  (The
+    bound is that of the other bf16 sizes: rounding to bf16 after each product.)"""
+    g = torch.Generator().manual_seed(m + n + k)
+    G = torch.randn(k, n, m, generator=g)
+    out = polar_express(G.to(gpu), compute_type=torch.bfloat16).cpu()
+    assert bool(torch.isfinite(out).all())
     for j in sorted({0, k // 2, k - 1}):
         ref = O.polar_express(G[j].numpy()[None], 5)[0]
         assert rel_err(out[j].numpy(), ref) <= POLAR_TOL_BF16
