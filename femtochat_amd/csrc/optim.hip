@@ -291,7 +291,8 @@ __global__ __launch_bounds__(256) void copy_scaled_kernel(int R, int C, const S*
 // column (padded), then eight lanes cover one 128-byte column segment of D,
 // adding beta C (loaded in that layout before the k loop) and rounding once.
 // M, N, K multiples of 64, every operand under 2^31 bytes
-// (checked by the caller): all tiles are whole and every offset is 32-bit.
+// (checked by the caller): each wave's part of a tile is whole or past the edge,
+// and every offset is 32-bit.
 struct PolarGemm {
   const bf16* P;
   const bf16* Q;
