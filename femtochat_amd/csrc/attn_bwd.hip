@@ -223,17 +223,17 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
 
   bf16x8 kf[KC][2], vf[KC][2];
   const int64_t krow = (int64_t)min(key, T - 1) * kpitch;
-  bool outside;
+  bool outside = false;  // a row's log-sum-exp is below kSplitLse
   {
     Split8 f[KC];
-    outside = split_rows<D>(Kb + krow, key < T, g, f);
+    split_rows<D>(Kb + krow, key < T, g, f);
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       kf[c][0] = f[c].part[0];
       kf[c][1] = f[c].part[1];
       s_low[wave][0][c][lane] = f[c].part[2];
     }
-    outside |= split_rows<D>(Vb + krow, key < T, g, f);
+    split_rows<D>(Vb + krow, key < T, g, f);
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       vf[c][0] = f[c].part[0];
@@ -282,13 +282,15 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
   auto store_rows = [&](int buf) {
     if (tid < BQ) {
       s_lse[buf][tid] = r_lse;
-      s_delta[buf][tid] = r_delta;
+      s_delta[buf][tid] = r_delta * kSplitScale2;
       s_lb[buf][tid] = r_lb;
+      outside |= r_lse < kSplitLse && r_lse != -INFINITY;  // (-inf: a row that sees no key)
     }
   };
 
-  // P of a tile in place of the scores, dS in place of dP.
-  auto softmax = [&](auto need_mask, f32x16& s, f32x16& dp, int q0, int buf) __attribute__((always_inline)) {
+  // P of a tile (times pscale) in place of the scores, dS in place of dP.
+  auto softmax = [&](auto need_mask, f32x16& s, f32x16& dp, int q0, int buf, float c2, float pscale)
+      __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int i0 = 8 * j + 4 * g;
@@ -297,8 +299,9 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int r = 4 * j + t;
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -L[t]));
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c2, -L[t]));
         float ds = p * (dp[r] - Dl[t]);
+        p *= pscale;
         if constexpr (decltype(need_mask)::value) {
           const int lbq = s_lb[buf][i0 + t], ubq = key_ub(q0 + i0 + t, T, a.right);
           const bool vis = (key >= lbq) & (key <= ubq);
@@ -324,11 +327,12 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
     return even + odd;
   };
 
+  const float c2 = a.scale_log2 * kSplitInv2;
   int st = next_step(0), st_next = total_steps;
   if (st < total_steps) {
     load_q(st);
     load_o(st);
-    outside |= qst.store(Qbuf[0], tid);
+    qst.store(Qbuf[0], tid);
     store_rows(0);
     st_next = next_step(st + 1);
   }
@@ -357,18 +361,17 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
     f32x16 s = zero16();
     if (active) {
       s = product(Qs, kf, 0);
-      outside |= ost.store(Os, tid);
+      ost.store(Os, tid);
     } else {
-      outside |= ost.store(Os, tid);
+      ost.store(Os, tid);
     }
     load_q(more ? st_next : st);
     load_o(more ? st_next : st);
     __syncthreads();
     if (active) {
       f32x16 dp = product(Os, vf, 1);
-      if (!(lbmax <= kw0 && kw1 <= ubmin)) softmax(std::true_type{}, s, dp, q0, buf);
-      else softmax(std::false_type{}, s, dp, q0, buf);
-      outside |= !(max_abs16(dp) < kSplitMax);
+      if (!(lbmax <= kw0 && kw1 <= ubmin)) softmax(std::true_type{}, s, dp, q0, buf, c2, kSplitScale);
+      else softmax(std::false_type{}, s, dp, q0, buf, c2, kSplitScale);
       // dV += P^T dO, dK += dS^T Q  (k = query, accumulator order)
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
@@ -378,9 +381,9 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
         for (int db = 0; db < DB; ++db)
           mma_split_pair(pf, split_tr<D>(Os, fo, kc, db), dv[db], sf, split_tr<D>(Qs, fo, kc, db), dk[db]);
       }
-      outside |= qst.store(Qbuf[buf ^ 1], tid);
+      qst.store(Qbuf[buf ^ 1], tid);
     } else {
-      outside |= qst.store(Qbuf[buf ^ 1], tid);
+      qst.store(Qbuf[buf ^ 1], tid);
     }
     store_rows(buf ^ 1);
     st = st_next;
@@ -389,11 +392,17 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
     __syncthreads();
   }
 
+  // (columns past the head dim, d >= D, come from LDS that nothing wrote)
+#pragma unroll
+  for (int db = 0; db < DB; ++db) outside |= (32 * db + l32 < D) & !(all_finite(dk[db]) & all_finite(dv[db]));
+  float kscale = a.scale * kSplitInv3, vscale = kSplitInv2;  // dK holds dS (2^32) times Q, dV holds P (2^16) times dO
   if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
   __syncthreads();
   if (s_outside != 0) {
     // fp32 MFMA from global memory.
     using M = Mma<float>;
+    kscale = a.scale;
+    vscale = 1.0f;
 #pragma unroll
     for (int i = 0; i < DB; ++i) {
       dk[i] = zero16();
@@ -420,7 +429,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
         s = M::mma(M::load8(Qb + qrow + at), key < T ? M::load8(Kb + krow + at) : M::zero(), s);
         dp = M::mma(M::load8(Ob + qrow + at), key < T ? M::load8(Vb + krow + at) : M::zero(), dp);
       }
-      softmax(std::true_type{}, s, dp, q0, 0);
+      softmax(std::true_type{}, s, dp, q0, 0, a.scale_log2, 1.0f);
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
         const f32x8 pf = kc ? M::from_acc<1>(s) : M::from_acc<0>(s);
@@ -447,7 +456,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
         const int kk = kw0 + acc_row(r, g);
         if (kk < T) {
           const int64_t off = ((int64_t)b * T + kk) * kpitch + (int64_t)kvh * D + d;
-          float vk = dk[db][r] * a.scale, vv = dv[db][r];
+          float vk = dk[db][r] * kscale, vv = dv[db][r] * vscale;
           float* pk = static_cast<float*>(a.dK) + off;
           float* pv = static_cast<float*>(a.dV) + off;
           if (a.accumulate) {
@@ -477,7 +486,6 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
   constexpr int kTile = SplitTile<D>::kBytes, kBM = 128;
   __shared__ __attribute__((aligned(1024))) char bufs[2][2 * kTile];  // K, V
   __shared__ int s_bounds[2][kWaves];
-  __shared__ int s_outside;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 5, l32 = lane & 31;
@@ -505,14 +513,15 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
     s_bounds[0][wave] = wlb_min;
     s_bounds[1][wave] = wub_max;
   }
-  if (tid == 0) s_outside = 0;
   const int64_t si = ((int64_t)b * a.H + h) * T + min(q, T - 1);
   const float lse = q < T ? a.lse2[si] : INFINITY;
-  const float dlt = q < T ? a.delta[si] : 0.0f;
+  float dlt = q < T ? a.delta[si] * kSplitScale2 : 0.0f;
+  bool outside = lse < kSplitLse && lse != -INFINITY;  // (-inf: a row that sees no key)
 
   Split8 qf[KC], of[KC];
   const int64_t qrow = (int64_t)min(q, T - 1) * qpitch;
-  bool outside = split_rows<D>(Qb + qrow, q < T, g, qf) | split_rows<D>(Ob + qrow, q < T, g, of);
+  split_rows<D>(Qb + qrow, q < T, g, qf);
+  split_rows<D>(Ob + qrow, q < T, g, of);
   FragOffsets<tile_width(D)> fo;
   fo.init(lane);
   f32x16 dq[DB];
@@ -529,11 +538,13 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
   const int kt0 = __builtin_amdgcn_readfirstlane((kmin / BN) * BN);
   const int ntiles = __builtin_amdgcn_readfirstlane(kmax >= kmin ? (kmax - (kmin / BN) * BN) / BN + 1 : 0);
 
+  float c2 = a.scale_log2 * kSplitInv2, qscale = a.scale * kSplitInv3;  // dQ holds dS (2^32) times K
+
   // dS of a tile into dp.
   auto softmax = [&](auto need_mask, const f32x16& s, f32x16& dp, int kt) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], a.scale_log2, -lse));
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c2, -lse));
       const float ds = p * (dp[r] - dlt);
       if constexpr (decltype(need_mask)::value) {
         const int kk = kt + acc_row(r, g);
@@ -549,7 +560,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
   // between dP and dQ (past the last tile, rows of the slice go to the idle
   // buffer); a mask is a uniform branch of its own, so that one copy of the
   // products serves all tiles.
-  auto body = [&](int kt, int buf, bool more, bool need_mask) __attribute__((always_inline)) {
+  auto body = [&](int kt, int buf, bool need_mask) __attribute__((always_inline)) {
     const char* Ks = bufs[buf];
     const char* Vs = Ks + kTile;
     char* next = bufs[buf ^ 1];
@@ -557,50 +568,50 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
     vst.load(Vb, kpitch, kt + BN, T, tid);
 #pragma unroll
     for (int c = 0; c < KC; ++c) s = mma_split(split_nat<D>(Ks, fo, c), qf[c], s);
-    bool out = kst.store(next, tid);
+    kst.store(next, tid);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int c = 0; c < KC; ++c) dp = mma_split(split_nat<D>(Vs, fo, c), of[c], dp);
-    out |= vst.store(next + kTile, tid);
+    vst.store(next + kTile, tid);
     __builtin_amdgcn_sched_barrier(0);
     if (need_mask) softmax(std::true_type{}, s, dp, kt);
     else softmax(std::false_type{}, s, dp, kt);
-    outside |= !(max_abs16(dp) < kSplitMax);
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
       const Split8 sf = kc ? split_acc<1>(dp) : split_acc<0>(dp);
 #pragma unroll
       for (int db = 0; db < DB; ++db) dq[db] = mma_split(split_tr<D>(Ks, fo, kc, db), sf, dq[db]);
     }
-    outside |= out & more;
   };
   if (ntiles > 0) {
     kst.load(Kb, kpitch, kt0, T, tid);
     vst.load(Vb, kpitch, kt0, T, tid);
-    outside |= kst.store(bufs[0], tid) | vst.store(bufs[0] + kTile, tid);
+    kst.store(bufs[0], tid);
+    vst.store(bufs[0] + kTile, tid);
     kst.load(Kb, kpitch, kt0 + BN, T, tid);
   }
   __syncthreads();
   for (int it = 0; it < ntiles; ++it) {
     const int kt = kt0 + it * BN;
-    const bool more = it + 1 < ntiles;
     if (wlb_min > kt + BN - 1 || wub_max < kt) {
       vst.load(Vb, kpitch, kt + BN, T, tid);
       char* next = bufs[(it + 1) & 1];
-      const bool out = kst.store(next, tid) | vst.store(next + kTile, tid);
-      outside |= out & more;
+      kst.store(next, tid);
+      vst.store(next + kTile, tid);
     } else {
-      body(kt, it & 1, more, !(wlb_max <= kt && kt + BN - 1 <= wub_min));
+      body(kt, it & 1, !(wlb_max <= kt && kt + BN - 1 <= wub_min));
     }
     kst.load(Kb, kpitch, kt + 2 * BN, T, tid);
     __syncthreads();
   }
 
-  if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
-  __syncthreads();
-  if (s_outside != 0) {
+  outside |= !all_finite<D>(dq);
+  if (__builtin_amdgcn_ballot_w64(outside) != 0) {
     // fp32 MFMA from global memory.
     using M = Mma<float>;
+    c2 = a.scale_log2;
+    qscale = a.scale;
+    dlt = q < T ? a.delta[si] : 0.0f;
 #pragma unroll
     for (int i = 0; i < DB; ++i) dq[i] = zero16();
 #pragma unroll 1
@@ -636,7 +647,7 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dq_exact_k
         if (d0 < D) {
           f32x4 v;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] = dq[db][4 * j + t] * a.scale;
+          for (int t = 0; t < 4; ++t) v[t] = dq[db][4 * j + t] * qscale;
           store4(static_cast<float*>(a.dQ) + orow * D + d0, v, a.accumulate);
         }
       }

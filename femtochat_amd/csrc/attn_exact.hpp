@@ -4,18 +4,28 @@
 // significant bits, each the rounded rest of the one before), so a float32
 // product is six bf16 products with exact terms and fp32 accumulation:
 //   x y ~ hh' + hm' + mh' + hl' + mm' + lh',
-// the terms left out being at most 2^-26 of |x y|.  v_mfma_f32_32x32x16_bf16
+// the terms left out (m l' and l m' above all) being at most 2^-24 of |x y|,
+// 2^-27.5 in the root mean square.  v_mfma_f32_32x32x16_bf16
 // does 16 k values in half the time v_mfma_f32_32x32x2_f32 takes for 2, so the
 // six together run at up to 2.7 times the fp32 rate, and round the running sum
 // 48 times per 128 k values instead of 64: the 2-norm error against float64 of
 // an 8 x 2048, H6, D128 causal step is 3.7e-7 (O), 5.2e-7 (dQ), 8.8e-7 (dK) and
 // 8.6e-7 (dV), with fp32 MFMA 3.7-4.4e-7, 6.2e-7, 1.15e-6 and 1.15e-6.
 //
-// The parts need a normal range: an input at or beyond 2^127 (h could round
-// to infinity), an infinity or a NaN (h - x would be NaN) or a run of eight
-// values none of which reaches 2^-96 (parts would be subnormal) raises the
-// workgroup's flag, and flagged workgroups recompute their rows with fp32
-// MFMA straight from global memory.
+// Every operand is multiplied by kSplitScale before it is split (and the
+// results by its inverse powers, both exact): the bf16 spacing at 0 is 2^-133,
+// the float32 spacing 2^-149, so the scaled parts hold every bit of every value
+// down to subnormal ones (the matrix cores take subnormal bf16 as they are: at
+// dS of 2^-120 the unscaled parts gave the error of gradual underflow).
+// At the other end, a scaled value at or beyond 2^127 (an input beyond 2^111,
+// an infinity or a NaN) has parts that are infinite or NaN, and so has any sum
+// of products that leaves the float32 range with the scale on it (S and dP
+// beyond 2^96, dQ, dK beyond 2^80): these reach the accumulators, and rows
+// (in dK/dV a workgroup's) that end with one that is not finite are computed
+// again with fp32 MFMA straight from global memory, unscaled, which makes them
+// take four times as long.  Only a score of -inf would go unseen, as a
+// probability of 0: a row whose scores are all -inf, or whose log-sum-exp is
+// below -2^80, is computed again too.
 #pragma once
 
 #include "attn_fast.hpp"
@@ -25,7 +35,10 @@ namespace fc {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-constexpr float kSplitMax = 0x1p127f, kSplitMin = 0x1p-96f;
+constexpr float kSplitScale = 0x1p16f;         // of every operand
+constexpr float kSplitScale2 = 0x1p32f;        // of a product of two
+constexpr float kSplitInv = 0x1p-16f, kSplitInv2 = 0x1p-32f, kSplitInv3 = 0x1p-48f;
+constexpr float kSplitLse = -0x1p80f;          // a log-sum-exp below it may go with scores of -inf
 
 // Eight consecutive k values of one operand row in three bf16 parts.
 struct Split8 {
@@ -66,23 +79,23 @@ __device__ inline Split8 split_acc(const f32x16& c) {
   return split8(x);
 }
 
-// NaN-propagating maximum of magnitudes.
-__device__ inline float max_abs8(const float (&x)[8]) {
-  float m = __builtin_fabsf(x[0]);
-#pragma unroll
-  for (int e = 1; e < 8; ++e) m = __builtin_elementwise_maximum(m, __builtin_fabsf(x[e]));
-  return m;
-}
-// Of the first N elements of an accumulator (8: its rows 0 .. 15).
+// The first N elements of an accumulator (8: its rows 0 .. 15) are finite.
 template <int N = 16>
-__device__ inline float max_abs16(const f32x16& c) {
+__device__ inline bool all_finite(const f32x16& c) {
   float m = __builtin_fabsf(c[0]);
 #pragma unroll
-  for (int r = 1; r < N; ++r) m = __builtin_elementwise_maximum(m, __builtin_fabsf(c[r]));
-  return m;
+  for (int r = 1; r < N; ++r) m = __builtin_elementwise_maximum(m, __builtin_fabsf(c[r]));  // propagates NaN
+  return m < INFINITY;
 }
-__device__ inline bool outside_split(float max_abs) {
-  return !(max_abs < kSplitMax) | ((max_abs < kSplitMin) & (max_abs != 0.0f));
+// The same of D rows in blocks of 32.  (The last block's rows past the head dim
+// come from LDS that nothing wrote.)
+template <int D>
+__device__ inline bool all_finite(const f32x16 (&c)[(D + 31) / 32]) {
+  bool finite = true;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db) finite &= all_finite(c[db]);
+  if (D % 32 != 0) finite &= all_finite<8>(c[(D + 31) / 32 - 1]);
+  return finite;
 }
 
 // c += a b: the six products, the smallest first.
@@ -136,7 +149,7 @@ __device__ inline Split8 split_tr(const char* tile, const FragOffsets<tile_width
 }
 
 // Loads 32 rows x D of float32 (two 16-byte loads per 8-value unit) and
-// writes them to LDS in parts.  Rows at or beyond T read row T - 1: what they
+// writes them to LDS, scaled, in parts.  Rows at or beyond T read row T - 1: what they
 // give is masked or multiplied by zero.
 template <int D>
 struct SplitStage {
@@ -153,39 +166,34 @@ struct SplitStage {
       v[i][1] = *reinterpret_cast<const f32x4*>(p + 4);
     }
   }
-  // Writes unit i; returns whether it is outside the range the parts need.
-  __device__ inline bool store_unit(char* tile, int tid, int i) const {
+  __device__ inline void store_unit(char* tile, int tid, int i) const {
     const int unit = min(tid + i * kThreads, kUnits - 1);  // past the end: the same values to the same place again
-    const float x[8] = {v[i][0][0], v[i][0][1], v[i][0][2], v[i][0][3], v[i][1][0], v[i][1][1], v[i][1][2], v[i][1][3]};
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = v[i][e / 4][e % 4] * kSplitScale;
     const Split8 s = split8(x);
     const int at = SplitTile<D>::Tile::offset(unit / kUPR, unit % kUPR);
 #pragma unroll
     for (int p = 0; p < 3; ++p) lds_store16(tile + p * SplitTile<D>::kPlane, at, __builtin_bit_cast(uint4, s.part[p]));
-    return outside_split(max_abs8(x));
   }
-  __device__ inline bool store(char* tile, int tid) const {
-    bool outside = false;
+  __device__ inline void store(char* tile, int tid) const {
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) outside |= store_unit(tile, tid, i);
-    return outside;
+    for (int i = 0; i < kPer; ++i) store_unit(tile, tid, i);
   }
 };
 
-// One wave's operand rows (row = lane l32) from global memory in parts.
+// One wave's operand rows (row = lane l32) from global memory, scaled, in parts.
 template <int D>
-__device__ inline bool split_rows(const float* row, bool valid, int g, Split8 (&f)[D / 16]) {
-  bool outside = false;
+__device__ inline void split_rows(const float* row, bool valid, int g, Split8 (&f)[D / 16]) {
 #pragma unroll
   for (int c = 0; c < D / 16; ++c) {
     float x[8];
     const f32x4 lo = valid ? *reinterpret_cast<const f32x4*>(row + 16 * c + 8 * g) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const f32x4 hi = valid ? *reinterpret_cast<const f32x4*>(row + 16 * c + 8 * g + 4) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = lo[e], x[4 + e] = hi[e];
-    outside |= outside_split(max_abs8(x));
+    for (int e = 0; e < 4; ++e) x[e] = lo[e] * kSplitScale, x[4 + e] = hi[e] * kSplitScale;
     f[c] = split8(x);
   }
-  return outside;
 }
 
 // For the recomputation: column d of 16 float32 rows from row0 as a fragment in

@@ -57,7 +57,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
   __shared__ __attribute__((aligned(1024))) char Ks[SplitTile<D>::kBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[SplitTile<D>::kBytes];
   __shared__ int s_bounds[2][kWaves];
-  __shared__ int s_outside;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 5, l32 = lane & 31;
@@ -83,18 +82,17 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
     s_bounds[0][wave] = wlb_min;
     s_bounds[1][wave] = wub_max;
   }
-  if (tid == 0) s_outside = 0;
 
   Split8 qf[KC];
-  bool outside = split_rows<D>(Qb + (int64_t)min(q, T - 1) * qpitch, q < T, g, qf);
+  split_rows<D>(Qb + (int64_t)min(q, T - 1) * qpitch, q < T, g, qf);
   FragOffsets<tile_width(D)> fo;
   fo.init(lane);
 
   f32x16 o[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) o[i] = zero16();
-  float m_ref = -INFINITY, m_true = -INFINITY, l_run = 0.0f;  // unscaled scores
-  const float c2 = a.scale_log2;
+  float m_ref = -INFINITY, m_true = -INFINITY, l_run = 0.0f;  // of scores times kSplitScale2, probabilities times kSplitScale
+  float c2 = a.scale_log2 * kSplitInv2, unscale = kSplitInv;  // of the scores' exponent; of O / l
 
   __syncthreads();
   int kmin = s_bounds[0][0], kmax = s_bounds[1][0];
@@ -111,7 +109,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
   if (ntiles > 0) {
     kst.load(Kb, kpitch, kt0, T, tid);
     vst.load(Vb, kpitch, kt0, T, tid);
-    outside |= kst.store(Ks, tid);
+    kst.store(Ks, tid);
   }
   __syncthreads();
 
@@ -123,9 +121,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
     if (active) {
 #pragma unroll
       for (int c = 0; c < KC; ++c) s = mma_split(split_nat<D>(Ks, fo, c), qf[c], s);
-      outside |= vst.store(Vs, tid);
+      vst.store(Vs, tid);
     } else {
-      outside |= vst.store(Vs, tid);
+      vst.store(Vs, tid);
     }
     if (more) kst.load(Kb, kpitch, kt + BN, T, tid);
     __syncthreads();
@@ -152,7 +150,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         // The difference first: the largest probability is exactly 1.
-        s[r] = __builtin_amdgcn_exp2f((s[r] - ref) * c2);
+        s[r] = __builtin_amdgcn_exp2f((s[r] - ref) * c2) * kSplitScale;
         psum += s[r];
       }
       l_run += psum;
@@ -164,23 +162,20 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
       }
     }
     if (more) {
-      outside |= kst.store(Ks, tid);
+      kst.store(Ks, tid);
       vst.load(Vb, kpitch, kt + BN, T, tid);
     }
     __syncthreads();
   }
 
-  // Probabilities above 1 may have carried a sum past the float32 range that
-  // those against the exact maximum stay in.
-  // (The last block's rows past the head dim come from LDS that nothing wrote.)
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db) grown |= !(max_abs16(o[db]) < INFINITY);
-  if (D % 32 != 0) grown |= !(max_abs16<8>(o[DB - 1]) < INFINITY);
-  if (__builtin_amdgcn_ballot_w64(outside) != 0 && lane == 0) s_outside = 1;
-  __syncthreads();
-  if (s_outside != 0 || __builtin_amdgcn_ballot_w64(grown) != 0) {
+  // Values or sums outside the parts' range (attn_exact.hpp), or probabilities
+  // above 1 that carried a sum past the float32 range.
+  grown |= !all_finite<D>(o) | (m_true == -INFINITY && lb <= ub);
+  if (__builtin_amdgcn_ballot_w64(grown) != 0) {
     // fp32 MFMA from global memory, with the exact maximum first.
     using M = Mma<float>;
+    c2 = a.scale_log2;
+    unscale = 1.0f;
     f32x8 q32[KC];
 #pragma unroll
     for (int c = 0; c < KC; ++c) q32[c] = q < T ? M::load8(Qb + (int64_t)q * qpitch + 16 * c + 8 * g) : M::zero();
@@ -218,7 +213,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
   }
 
   const float lt = l_run + __shfl_xor(l_run, 32);
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = lt > 0.0f ? unscale / lt : 0.0f;
   if (q < T) {
     const int64_t orow = ((int64_t)b * T + q) * a.H + h;
 #pragma unroll
@@ -237,7 +232,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
     if (g == 0) {
       const int64_t si = ((int64_t)b * a.H + h) * T + q;
       const bool any = m_true != -INFINITY;
-      a.l[si] = any ? lt * __builtin_amdgcn_exp2f((m_ref - m_true) * c2) : lt;
+      a.l[si] = any ? lt * unscale * __builtin_amdgcn_exp2f((m_ref - m_true) * c2) : lt * unscale;
       a.m[si] = any ? m_true * c2 * kLn2 : -kFltMax;
     }
   }

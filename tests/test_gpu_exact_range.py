@@ -1,7 +1,7 @@
-"""Exact mode outside the range its bf16 parts hold: the products of three
-bf16 parts stand for float32 products while values are below 2^127 and eight
-of a row are not all below 2^-96; workgroups that meet others (or scores that
-outgrow the first tile's maximum by 2^64) recompute with fp32 products.
+"""Exact mode at the ends of the float32 range: the products of three bf16
+parts stand for float32 products while inputs stay below 2^111 and scores below
+2^96; rows that meet others (or scores that outgrow the first tile's maximum by
+2^64) are computed again with fp32 products.
 
 Scaling by a power of two is exact, so a scaled problem must give the scaled
 results of the plain one (itself compared with the float64 oracle); both
@@ -54,6 +54,54 @@ def test_scaled_inputs(gpu, D, q, k, v, do):
     fs = [float(x) for x in f]
     for x, y, s in zip(scaled, plain, (fs[2], fs[2] * fs[3] / fs[0], fs[2] * fs[3] / fs[1], fs[3])):
         assert np.all(np.isfinite(x)) and _close(x / s, y)
+
+
+@pytest.mark.parametrize("D", [16, 64, 112, 128])
+@pytest.mark.parametrize("v,do", [(-24, -92), (-56, -56), (-60, -60)])
+def test_small_score_gradients(gpu, D, v, do):
+    """V and dO whose product, and with it dS, falls to 2^-112 .. 2^-120 while
+    neither is small for a float32: dS keeps its 24 bits.  What float32 itself
+    loses are sums' terms below 2^-149 (2^-26 of a dS of 2^-123, few of them:
+    6e-8 in all at v + do = -120 in fp32 products); the bound is 1e-6."""
+    Q, K, V, dO = _inputs(D)
+    plain = _run(gpu, Q, K, V, dO)
+    fv, fd = 2.0 ** v, 2.0 ** do
+    scaled = _run(gpu, Q, K, V * np.float32(fv), dO * np.float32(fd))
+    for name, x, y, s in zip(("O", "dQ", "dK", "dV"), scaled, plain, (fv, fv * fd, fv * fd, fd)):
+        e = np.linalg.norm(x / s - y) / np.linalg.norm(y)
+        assert e <= 1e-6, f"{name} {e}"
+
+
+@pytest.mark.parametrize("D", [64, 96])
+@pytest.mark.parametrize("which", ["Q", "K", "V", "dO"])
+def test_tiny_column(gpu, D, which):
+    """One column of 2^-118 times its neighbours: the output column that it alone
+    makes (of dK, dQ, O, dV) has the relative precision of the others, a few
+    1e-7 (float32 sums of 300 terms); the bound is 2e-6."""
+    t = dict(zip(("Q", "K", "V", "dO"), _inputs(D, B=1)))
+    t[which][..., 3] *= np.float32(2.0) ** np.float32(-118)
+    Q, K, V, dO = t.values()
+    out = dict(zip(("O", "dQ", "dK", "dV"), _run(gpu, Q, K, V, dO)))
+    O, l, m = R.forward(Q, K, V, (-1, 0))
+    ref = dict(zip(("O", "dQ", "dK", "dV"), (O, *R.backward(dO, Q, K, V, O, l, m, (-1, 0)))))
+    name = dict(Q="dK", K="dQ", V="O", dO="dV")[which]
+    x, y = out[name][..., 3], ref[name][..., 3]
+    e = np.linalg.norm(x - y) / np.linalg.norm(y)
+    assert e <= 2e-6, f"{name} {e}"
+
+
+@pytest.mark.parametrize("B,T,H,Hkv,D,window", [(2, 333, 4, 2, 128, (-1, 0)), (1, 300, 6, 2, 64, (200, 3)),
+                                                (2, 270, 4, 1, 80, (-1, 0)), (1, 257, 2, 2, 16, (-1, 0))])
+def test_float32_precision(gpu, B, T, H, Hkv, D, window):
+    """O and the gradients within 2e-6 (2-norm) of float64, as float32 products
+    give them; without the products of the third parts the error is above 3e-6
+    (tests/test_exact_split.py)."""
+    Q, K, V, dO = _inputs(D, T=T, B=B, H=H, Hkv=Hkv)
+    O, l, m = R.forward(Q, K, V, window)
+    ref = (O, *R.backward(dO, Q, K, V, O, l, m, window))
+    for name, x, y in zip(("O", "dQ", "dK", "dV"), _run(gpu, Q, K, V, dO, window), ref):
+        e = np.linalg.norm(x - y) / np.linalg.norm(y)
+        assert e <= 2e-6, f"{name} {e}"
 
 
 @pytest.mark.parametrize("D", [32, 128])
