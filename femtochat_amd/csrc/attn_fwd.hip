@@ -15,8 +15,10 @@
 //    split and stored; while the P V products read V, the next K tile is, each
 //    loaded a phase ahead (16 registers per thread in flight);
 //  * the exponent reference of a row is the maximum of the first tile in which
-//    it sees a key and never moves (as in the fast kernel: O is not rescaled),
-//    and a row that outgrows it by 2^64 is recomputed;
+//    it sees a key; a row whose scores outgrow it by 2^8 moves it and rescales
+//    its O and l, in a branch that few tiles take (with a reference that never
+//    moved, rows that outgrew it by 2^64 were computed again: queries times 30, 8 x
+//    2048 tokens, took 1197 us at H6 D128, now 302);
 //  * key tiles outside [min lb, max ub] of the workgroup are never visited,
 //    fully visible tiles skip the mask, and waves with no visible key in a
 //    tile skip its products.
@@ -33,7 +35,7 @@ namespace fc {
 
 constexpr int kExactBM = 128;  // queries per workgroup
 constexpr int kExactBN = 32;   // keys per tile
-constexpr float kExactGrowth = 64.0f;  // log2 units above the reference that send a row to the recomputation
+constexpr float kExactGrowth = 8.0f;  // log2 units that a score may lie above its row's reference
 
 // S^T of 32 keys from k0 in fp32 MFMA, K straight from global memory, masked.
 template <int D>
@@ -105,7 +107,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
   const int ntiles = __builtin_amdgcn_readfirstlane(kmax >= kmin ? (kmax - (kmin / BN) * BN) / BN + 1 : 0);
 
   SplitStage<D> kst, vst;
-  bool grown = false;
   if (ntiles > 0) {
     kst.load(Kb, kpitch, kt0, T, tid);
     vst.load(Vb, kpitch, kt0, T, tid);
@@ -143,8 +144,16 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       m_true = fmaxf(m_true, mx);
-      m_ref = m_ref == -INFINITY ? mx : m_ref;  // a row's first visible key sets the reference
-      grown |= (mx - m_ref) * c2 > kExactGrowth;
+      // A row's first visible key sets the reference (O and l are zero then); one
+      // that outgrows it moves it.
+      const bool grown = (mx - m_ref) * c2 > kExactGrowth;
+      if (__builtin_amdgcn_ballot_w64(grown) != 0) {
+        const float f = grown ? __builtin_amdgcn_exp2f((m_ref - mx) * c2) : 1.0f;
+        m_ref = grown ? mx : m_ref;
+        l_run *= f;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db] *= f;
+      }
       const float ref = m_ref == -INFINITY ? 0.0f : m_ref;
       float psum = 0.0f;
 #pragma unroll
@@ -168,10 +177,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_exact_kernel(FwdArgs a) 
     __syncthreads();
   }
 
-  // Values or sums outside the parts' range (attn_exact.hpp), or probabilities
-  // above 1 that carried a sum past the float32 range.
-  grown |= !all_finite<D>(o) | (m_true == -INFINITY && lb <= ub);
-  if (__builtin_amdgcn_ballot_w64(grown) != 0) {
+  // Values or sums outside the parts' range (attn_exact.hpp).
+  const bool outside = !all_finite<D>(o) | (m_true == -INFINITY && lb <= ub);
+  if (__builtin_amdgcn_ballot_w64(outside) != 0) {
     // fp32 MFMA from global memory, with the exact maximum first.
     using M = Mma<float>;
     c2 = a.scale_log2;

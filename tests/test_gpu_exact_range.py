@@ -1,7 +1,6 @@
 """Exact mode at the ends of the float32 range: the products of three bf16
 parts stand for float32 products while inputs stay below 2^111 and scores below
-2^96; rows that meet others (or scores that outgrow the first tile's maximum by
-2^64) are computed again with fp32 products.
+2^96; rows that meet others are computed again with fp32 products.
 
 Scaling by a power of two is exact, so a scaled problem must give the scaled
 results of the plain one (itself compared with the float64 oracle); both
@@ -128,8 +127,7 @@ def test_infinite_value_and_nan_query(gpu, D):
 @pytest.mark.parametrize("D", [16, 128])
 def test_large_values_behind_growing_scores(gpu, D):
     """Probabilities of up to 2^40 against the first tile's maximum times values
-    of 2^100: the sum leaves the float32 range unless the exact maximum is the
-    reference."""
+    of 2^100: the sum leaves the float32 range unless the reference moves."""
     Q, K, V, dO = _inputs(D, B=1, H=2, Hkv=1)
     Q, K = np.abs(Q) + 0.5, np.abs(K) + 0.5
     K *= np.where(np.arange(K.shape[1]) < 256, 0.1, 1.0).astype(np.float32)[None, :, None, None]
@@ -152,6 +150,25 @@ def test_growing_scores(gpu, D):
     # scores of up to 600 carry a rounding of 600 log2(e) 2^-24 in the exponent
     for x, r in zip((O, dV), (O_ref, g_ref[2])):
         assert rel_err(x, r) <= 3 * TOL["exact"]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_growing_scores_leave_the_other_rows(gpu, D):
+    """A query whose scores grow by far more than 2^64 behind the first tile
+    changes its own row alone: the other rows of its wave keep their bits (they
+    would not, were the wave's products done again another way)."""
+    g = torch.Generator(device=gpu).manual_seed(D)
+    Q, K, V = (torch.randn(1, 500, 2, D, device=gpu, generator=g) for _ in range(3))
+    plain = gpu_forward(MFMAExact(), Q, K, V, (-1, 0))
+    Q2 = Q.clone()
+    Q2[0, 400, 1] = 40.0 * K[0, 200, 1]
+    O, l, m = gpu_forward(MFMAExact(), Q2, K, V, (-1, 0))
+    torch.cuda.synchronize()
+    O_ref, l_ref, m_ref = R.forward(*(to_np(x) for x in (Q2, K, V)), (-1, 0))
+    assert m_ref[0, 1, 400] > 200 and rel_err(to_np(O), O_ref) <= TOL["exact"]
+    for x, y, at in zip((O, l, m), plain, ((0, 400, 1), (0, 1, 400), (0, 1, 400))):
+        x[at] = y[at]
+        assert torch.equal(x, y)
 
 
 @pytest.mark.parametrize("D", [16, 48, 80, 112])
