@@ -162,19 +162,28 @@ def test_autograd_matches_explicit_backward(gpu):
     ("fast", (torch.float16, torch.float16, torch.float16), 64),
     ("exact", (torch.bfloat16, torch.bfloat16, torch.bfloat16), 64),
 ])
-def test_autograd_gradient_dtypes(gpu, mode, dtypes, D):
+def test_autograd_gradient_dtypes(gpu, monkeypatch, mode, dtypes, D):
     """The gradients in each leaf's dtype equal the float32 gradients of an
     explicit backward into zeroed buffers, rounded once, bit for bit; rows and
-    keys that see nothing (a window left of every key) get zeros."""
+    keys that see nothing (a window left of every key) get zeros, also in
+    buffers that come filled with NaN."""
     B, T, H, Hkv, window = 2, 200, 4, 2, (40, -3)
     A = MFMAFast() if mode == "fast" else MFMAExact()
     Q, K, V, dO = _inputs(5 + D, B, T, H, Hkv, D)
     leaves = [torch.from_numpy(x).to(gpu).to(dt).requires_grad_(True) for x, dt in zip((Q, K, V), dtypes)]
-    junk = torch.full((64 << 20,), float("nan"), device=gpu)  # what the freed blocks of the next allocations hold
-    del junk
-    O = Kn.AttentionFunction.apply(*leaves, window, A, None)
-    dOd = torch.from_numpy(dO).to(gpu).to(O.dtype)
-    grads = torch.autograd.grad(O, leaves, dOd)
+    poisoned, empty = [], torch.empty
+
+    def nan_empty(*args, **kwargs):
+        t = empty(*args, **kwargs)
+        poisoned.append(t.shape)
+        return t.fill_(float("nan") if t.is_floating_point() else 255)
+
+    with monkeypatch.context() as patch:
+        patch.setattr(torch, "empty", nan_empty)
+        O = Kn.AttentionFunction.apply(*leaves, window, A, None)
+        dOd = torch.from_numpy(dO).to(gpu).to(O.dtype)
+        grads = torch.autograd.grad(O, leaves, dOd)
+    assert all(x.shape in poisoned for x in grads)
     st = Kn.attention_state(A, *(x.detach() for x in leaves), window)
     ref = [torch.zeros(x.shape, dtype=torch.float32, device=gpu) for x in (st.Q, st.K, st.V)]
     Kn.delta_attention_(A, *ref, dOd, st.Q, st.K, st.V, st.O, st.l, st.m, window)
