@@ -29,7 +29,8 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kFwdBatch = 8;  // 16-byte loads in flight per thread in a forward round (4, 8, 16 within 1%)
-constexpr int kWaveV = 2048; // longest column that the forward gives to one wave
+constexpr int kWaveV = 2048;  // longest column that a wave reads in one round
+constexpr int kWaveN = 1024;  // columns from which on waves take up to three rounds (four waves per CU)
 constexpr int kBwdBatch = 8;  // chunks per backward round (4, 8 measured within 3%)
 
 template <typename I>
@@ -133,15 +134,34 @@ __global__ __launch_bounds__(256) void xent_fwd_kernel(XentArgs a) {
   if (threadIdx.x == 0) store_loss(a, token, col, r);
 }
 
-// Short columns: a wave each, four to a workgroup, no barrier (8192 x 1000: 10
-// us, 28 with a workgroup each; 8192 x 53: 10 and 12).
+// Short columns: a wave each, four to a workgroup, no barrier, with as many loads
+// in flight as the column has for a lane.  us, a workgroup / a wave each:
+// 8192 x 50 19 / 6.0, x 1000 28 / 8.6, x 2048 27.7 / 13.5, x 4096 30.3 / 23.5, x 6001
+// 36.6 / 32.8, x 8192 43.6 / 45.6; 1024 x 2048 6.7 / 4.7, x 4096 6.9 / 6.3, x 6001
+// 7.6 / 7.4, x 8192 7.4 / 8.6; 512 x 3000 5.3 / 6.0; 256 x 2048 4.5 / 4.6 (with four
+// loads in flight 5.3), x 3000 4.6 / 6.0; 8 x 1500 4.4 / 4.3.
 template <int kBatch>
 __global__ __launch_bounds__(256) void xent_fwd_wave_kernel(XentArgs a) {
   const int64_t token = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
   if (token >= a.N) return;
   const int lane = threadIdx.x & 63;
   const float* col = a.logits + token * (int64_t)a.V;
-  Lse r = column_pass<true, 64, kBatch>(col, a.V, lane);
+  Lse r;
+  if constexpr (kBatch == 0) {  // up to 256 values: four per lane, one by one, whatever the column's alignment
+    float x[4], m = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[k] = lane + 64 * k < a.V ? __builtin_nontemporal_load(col + lane + 64 * k) : -INFINITY;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m = fmaxf(m, x[k]);
+    const float ref = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum += exp2f((x[k] - ref) * kLog2e);
+    r = Lse{m, sum};
+  } else {
+    r = column_pass<true, 64, kBatch>(col, a.V, lane);
+  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) r = combine(r, Lse{__shfl_xor(r.m, o), __shfl_xor(r.s, o)});
   if (lane == 0) store_loss(a, token, col, r);
@@ -458,8 +478,9 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(EmbedArgs a) {
 hipError_t launch_xent_fwd(const XentArgs& a, hipStream_t s) {
   const ProfileMark mk = profile_begin(s);
   const dim3 waves((unsigned)((a.N + 3) / 4)), block(256);
-  if (a.V <= kWaveV / 8) hipLaunchKernelGGL(xent_fwd_wave_kernel<1>, waves, block, 0, s, a);
-  else if (a.V <= kWaveV) hipLaunchKernelGGL(xent_fwd_wave_kernel<4>, waves, block, 0, s, a);
+  if (a.V <= kWaveV / 8) hipLaunchKernelGGL(xent_fwd_wave_kernel<0>, waves, block, 0, s, a);
+  else if (a.V <= kWaveV / 2) hipLaunchKernelGGL(xent_fwd_wave_kernel<4>, waves, block, 0, s, a);
+  else if (a.V <= kWaveV || (a.N >= kWaveN && a.V <= 3 * kWaveV)) hipLaunchKernelGGL(xent_fwd_wave_kernel<8>, waves, block, 0, s, a);
   else hipLaunchKernelGGL(xent_fwd_kernel, dim3((unsigned)a.N), block, 0, s, a);
   hipError_t e = hipGetLastError();
   profile_end(mk, "xent_fwd", s);

@@ -369,6 +369,26 @@ def test_gradient_routes_agree(gpu, N, V, reduction):
     assert torch.equal(g[~ign], one[~ign]) and not g[ign].any()
 
 
+@pytest.mark.parametrize("N,V", [(5, 1), (6, 64), (5, 65), (9, 255), (9, 256), (9, 257), (7, 1024), (7, 1025), (6, 2048),
+                                 (6, 2049), (1023, 2049), (1024, 2049), (1025, 4099), (1024, 6144), (1025, 6145)])
+def test_forward_routes(gpu, N, V):
+    """Around the forward's rules (values one by one up to 256, a wave's loads up
+    to 1024, 2048 and, from 1024 columns on, three rounds up to 6144): the
+    log-sum-exp against float64, the sum of V exponentials in float32, and
+    infinities and NaN in their own rows."""
+    x, t, xd, td = _ce_case(gpu, N, V, seed=N + V)
+    x[0, V - 1], x[1, 0], x[2, V // 2], x[3, :] = float("inf"), float("nan"), -float("inf"), -float("inf")
+    losses, lse = torch.empty(N, device=gpu), torch.empty(N, device=gpu)
+    cross_entropy_(losses, x.to(gpu), td, -1, "none", lse=lse)
+    ref, got = torch.logsumexp(x.double(), 1), lse.cpu().double()
+    assert not torch.isfinite(got[0]) and torch.isnan(got[1]) and got[3] == -float("inf")
+    rows = [i for i in range(N) if i not in (0, 1, 3) and torch.isfinite(ref[i])]
+    assert float((got[rows] - ref[rows]).abs().max()) <= 1e-5
+    keep = [i for i in rows if t[i] != -1 and torch.isfinite(x[i, t[i]])]
+    one_hot = x.double()[keep, t[keep].long()]
+    assert float((losses.cpu().double()[keep] - (ref[keep] - one_hot)).abs().max()) <= 1e-5
+
+
 def test_masked_logits(gpu):
     """Vocabulary entries at -inf add nothing to the sum, wherever they stand
     in the column (a whole first round of loads, the head and the tail)."""
