@@ -715,7 +715,7 @@ fc_status fc_embedding_bwd_full(const fc_embed_desc* desc, float* dweights, cons
   if (st != FC_OK) return st;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
-  if (fc::embed_grad_full_supported(a)) {
+  if (fc::embed_grad_full_pays(a)) {
     e = fc::launch_embed_grad_full(a, desc->y_dtype == FC_BF16, s);
   } else {
     st = fc_fill_zero(dweights, (size_t)a.vocab * a.D * sizeof(float), stream);

@@ -163,8 +163,9 @@ struct EmbedArgs {
 };
 hipError_t launch_embed(const EmbedArgs& a, bool backward, bool bf16_y, hipStream_t s);
 
-// The gradient into a fresh table (embed_grad.hip).
-bool embed_grad_full_supported(const EmbedArgs& a);
+// The gradient into a fresh table in one kernel (embed_grad.hip), where that is
+// the faster way.
+bool embed_grad_full_pays(const EmbedArgs& a);
 hipError_t launch_embed_grad_full(const EmbedArgs& a, bool bf16_dy, hipStream_t s);
 
 // Workspace of the sorted (deterministic) embedding gradient: keys and token

@@ -19,6 +19,7 @@
 // 8192 x 256: 9.4 us (11.3).
 #include "attn_launch.hpp"
 #include "attn_device.hpp"
+#include "embed_rule.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -31,9 +32,7 @@ constexpr int kEgThreads = 512, kEgWaves = kEgThreads / 64;
 constexpr int kEgPer = 8;                        // tokens a thread looks at per scan step
 constexpr int kEgStep = kEgThreads * kEgPer;     // tokens per scan step
 constexpr int kEgCap = kEgStep + 2048;           // list entries: a full step beyond 2048 kept ones
-constexpr int kEgSlots = 128;                    // table columns per workgroup at most
 constexpr int kEgSegs = kEgThreads / kEgSlots;   // list segments counted side by side
-constexpr int kEgCols = 256;                     // values of a column per workgroup, four per lane
 constexpr int kEgRows = 8;                       // rows in flight per wave
 
 // A lane's four values of a row as loaded (lanes past the row's end read its
@@ -263,22 +262,14 @@ __global__ __launch_bounds__(kEgThreads) void embed_grad_kernel(EmbedArgs a, int
 
 }  // namespace
 
-// At least 256 groups (one per CU and value block), at most kEgSlots columns each.
-static int embed_groups(int vocab) {
-  return vocab < 256 ? vocab : vocab <= 256 * kEgSlots ? 256 : (vocab + kEgSlots - 1) / kEgSlots;
-}
-
-// Every group scans every token, so a table of many more columns than this
-// would spend longer scanning (groups x value blocks x 8 bytes per token, some
-// 12 TB/s from L2) than the atomics on a cleared table take (D values per
-// token, 50 per ns); the token count is limited by the 32-bit list entries.
-bool embed_grad_full_supported(const EmbedArgs& a) {
-  return a.vocab <= (1 << 19) && a.N <= UINT32_MAX &&
+// Token indices are 32-bit list entries.
+bool embed_grad_full_pays(const EmbedArgs& a) {
+  return embed_one_kernel_pays(a.N, a.vocab, a.D) && a.N <= UINT32_MAX &&
          (int64_t)embed_groups(a.vocab) * ((a.D + kEgCols - 1) / kEgCols) <= INT32_MAX / kEgThreads;
 }
 
 hipError_t launch_embed_grad_full(const EmbedArgs& a, bool bf16_dy, hipStream_t s) {
-  if (!embed_grad_full_supported(a)) return hipErrorInvalidValue;
+  if (!embed_grad_full_pays(a)) return hipErrorInvalidValue;
   const int groups = embed_groups(a.vocab);
   const int64_t blocks = (int64_t)groups * ((a.D + kEgCols - 1) / kEgCols);
   const uintptr_t dy = reinterpret_cast<uintptr_t>(a.dy);

@@ -107,9 +107,10 @@ fc_status fc_embedding_bwd(const fc_embed_desc* desc, float* dweights, const voi
                            void* stream);
 
 /* The same gradient written over the whole of dweights (sums of the tokens'
-   dy columns, zeros elsewhere), so dweights needs no clearing; one kernel, no
-   workspace, and the same bits on every call (a table of more than 2^19
-   columns is cleared and added into with atomics instead). */
+   dy columns, zeros elsewhere), so dweights needs no clearing.  Without a
+   workspace; one kernel that sums in token order (the same bits on every
+   call), or, where that takes longer (large tables of short columns, few
+   tokens for a wide table), a cleared table and fc_embedding_bwd's atomics. */
 fc_status fc_embedding_bwd_full(const fc_embed_desc* desc, float* dweights, const void* dy, const void* tokens,
                                 void* stream);
 

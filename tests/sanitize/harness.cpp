@@ -6,6 +6,7 @@
 // softmax attention.
 #include "../../femtochat_amd/csrc/attn_index.hpp"
 #include "../../femtochat_amd/csrc/attn_problem.hpp"
+#include "../../femtochat_amd/csrc/embed_rule.hpp"
 
 #include <cmath>
 #include <cstdio>
@@ -268,8 +269,39 @@ static void paired_grids() {
   }
 }
 
+// The embedding gradient's two ways: where each was measured the faster one by a
+// fifth or more (word frequencies), and more tokens never turn the choice away
+// from the one kernel while its workgroups all run at once.
+static void embedding_ways() {
+  const struct {
+    int64_t N;
+    int vocab, D;
+    bool one;
+  } at[] = {{8192, 32768, 512, true},   {8192, 32768, 32, true},   {8192, 50257, 768, true},  {65536, 32768, 32, true},
+            {8192, 131072, 512, true},  {8192, 131072, 128, true}, {1024, 32768, 512, true},  {8192, 1000, 1280, true},
+            {8192, 262144, 32, false},  {8192, 524288, 32, false}, {8192, 524288, 64, false}, {8192, 524288, 128, false},
+            {65536, 524288, 32, false}, {1024, 131072, 32, false}, {64, 131072, 32, false},   {64, 524288, 128, false},
+            {64, 1000, 1280, false},    {64, 8192, 1280, false}};
+  for (const auto& c : at) {
+    const bool got = fc::embed_one_kernel_pays(c.N, c.vocab, c.D);
+    if (got != c.one) std::fprintf(stderr, "embedding N=%lld V=%d D=%d\n", (long long)c.N, c.vocab, c.D);
+    CHECK(got == c.one);
+  }
+  for (int V : {1, 50, 1000, 32768, 65536})
+    for (int D : {1, 16, 64, 256, 512}) {
+      if ((int64_t)fc::embed_groups(V) * ((D + fc::kEgCols - 1) / fc::kEgCols) > 512) continue;
+      bool before = false;
+      for (int64_t N = 1; N <= (int64_t)1 << 33; N *= 2) {
+        const bool one = fc::embed_one_kernel_pays(N, V, D);
+        CHECK(one || !before);
+        before = one;
+      }
+    }
+}
+
 int main() {
   validation();
+  embedding_ways();
   grid_orders();
   paired_grids();
   restatement(16, 2, 1, 37, 2, -1, 0, 1, false);

@@ -454,3 +454,22 @@ def test_embedding_gradient_full(gpu, N, vocab, D, dy_dtype, ids):
     assert not outs[0][terms[:, 0] == 0].any()
     if vocab <= 1 << 19:
         assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("N,vocab,D", [(64, 1000, 1280), (500, 262144, 32), (9, 524288, 100)])
+def test_embedding_gradient_full_by_atomics(gpu, N, vocab, D):
+    """Where the one kernel would take longer, the table is cleared and added
+    into: the same sums over a table of NaN, in any order (the rounding of an
+    fp32 sum of that many terms)."""
+    g = torch.Generator().manual_seed(N + D)
+    tok = (vocab * torch.rand(N, generator=g) ** 6).long().clamp(max=vocab - 1)
+    dy = torch.randn(N, D, generator=g)
+    dw = torch.full((vocab, D), float("nan"), device=gpu)
+    d = _lib.EmbedDesc(D, vocab, N, 0, _lib.FC_INDEX_I64, _lib.FC_F32, 0)
+    dyd, td = dy.to(gpu), tok.to(gpu)
+    _lib.check(_lib.lib().fc_embedding_bwd_full(ctypes.byref(d), dw.data_ptr(), dyd.data_ptr(), td.data_ptr(),
+                                                torch.cuda.current_stream().cuda_stream))
+    ref = torch.zeros(vocab, D, dtype=torch.float64).index_add_(0, tok, dy.double())
+    size = torch.zeros(vocab, D, dtype=torch.float64).index_add_(0, tok, dy.double().abs())
+    terms = torch.bincount(tok, minlength=vocab).double()[:, None]
+    assert bool(((dw.cpu().double() - ref).abs() <= terms * 2.0 ** -24 * size).all())
