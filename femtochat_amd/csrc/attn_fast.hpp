@@ -132,44 +132,6 @@ struct FragOffsets {
   __device__ inline int tr(int e, int db) const { return tr_base[e] ^ (64 * db); }
 };
 
-// Stages a tile of R rows x D bf16 (16-byte units) from global memory into a
-// swizzled LDS tile.  StagePlan holds each thread's unit offsets (global,
-// relative to the tile's first row, and LDS), shared by every tile of the
-// same shape; StageRegs holds one tile's data in flight.
-template <int D, int R, int NT>
-struct StagePlan {
-  using Tile = SwzTile<D>;
-  static constexpr int kUnits = R * Tile::kUPR;
-  static constexpr int kPer = (kUnits + NT - 1) / NT;
-  int goff[kPer];
-  int loff[kPer];
-
-  __device__ inline void init(int tid, int pitch_bytes) {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      int unit = tid + i * NT;
-      if (unit >= kUnits) unit = kUnits - 1;  // duplicates a valid unit (same data, same slot)
-      const int row = unit / Tile::kUPR, u = unit % Tile::kUPR;
-      goff[i] = row * pitch_bytes + 16 * u;
-      loff[i] = Tile::offset(row, u);
-    }
-  }
-};
-
-template <int D, int R, int NT>
-struct StageRegs {
-  using Plan = StagePlan<D, R, NT>;
-  uint4 v[Plan::kPer];
-  __device__ inline void load(const Plan& pl, __amdgpu_buffer_rsrc_t r) {
-#pragma unroll
-    for (int i = 0; i < Plan::kPer; ++i) v[i] = buf_load16(r, pl.goff[i], 0);
-  }
-  __device__ inline void store(const Plan& pl, char* lds) const {
-#pragma unroll
-    for (int i = 0; i < Plan::kPer; ++i) lds_store16(lds, pl.loff[i], v[i]);
-  }
-};
-
 // Direct global -> LDS staging (buffer_load_dwordx4 ... lds, gfx950): one
 // wave instruction writes 64 lanes x 16 bytes to a contiguous 1 KB block of
 // LDS (lane l at M0 + 16 l) from per-lane global offsets, so the swizzle is

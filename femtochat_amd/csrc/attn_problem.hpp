@@ -156,17 +156,6 @@ struct FwdWorkspace {
   size_t chunk_lb, qorder, total;
 };
 
-// A problem with float32 gradients that are overwritten, the widest case of a
-// backward workspace with PadWorkspace.
-inline Problem kernel_problem(const Problem& p, bool backward) {
-  Problem k = p;
-  if (padded(p) && backward) {
-    k.grad_bf16 = false;
-    k.accumulate = false;
-  }
-  return k;
-}
-
 // What the workspace of head dims 48, 80, 96 and 112 begins with (byte
 // offsets, 256-aligned): room for Q, K, V (input format), O (its format), and
 // in the backward dO (its format) and float32 dQ, dK, dV with rows of Dk

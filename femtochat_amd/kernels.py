@@ -68,7 +68,8 @@ _GEOMETRY_KEYWORDS = {"warps", "query_tile", "head_span", "order", "query_subtil
 
 
 class MFMAExact:
-    """fp32 inputs, fp32 MFMA, fp32 outputs: the analogue of the reference's
+    """fp32 inputs and outputs, float32 precision (products on three bf16 parts
+    of each value, fp32 accumulation): the analogue of the reference's
     ``SIMTInstruction`` (ext/FemtoChatCUDAExt.jl:210, kernels :243-1002)."""
 
     mode = _lib.FC_MODE_EXACT

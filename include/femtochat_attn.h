@@ -55,8 +55,9 @@ typedef enum {
 typedef enum { FC_F32 = 0, FC_BF16 = 1 } fc_dtype;
 
 typedef enum {
-  /* fp32 in, fp32 MFMA, fp32 out (analogue of SIMTInstruction,
-     reference ext/FemtoChatCUDAExt.jl:243-1002) */
+  /* fp32 in and out; products in bf16 MFMA on three bf16 parts of each float32
+     value (24 bits), fp32 accumulation and statistics: float32 precision
+     (analogue of SIMTInstruction, reference ext/FemtoChatCUDAExt.jl:243-1002) */
   FC_MODE_EXACT = 0,
   /* bf16 Q/K/V/dO, bf16 MFMA with fp32 accumulation and statistics; P and dS
      rounded to bf16 before their second product (analogue of

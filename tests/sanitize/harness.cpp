@@ -71,9 +71,9 @@ static void validation() {
     CHECK(std::strlen(small) < sizeof small);
   }
   CHECK(fc::make_problem(nullptr, &p, msg, sizeof msg) == FC_ERR_INVALID_ARGUMENT);
-  // Every multiple of 16 up to 128 is accepted; the kernels run the next
-  // compiled width, and the padded copies lead both workspaces without
-  // overlapping each other or the kernels' own regions.
+  // Every multiple of 16 up to 128 is accepted; where the tiles are wider than
+  // the head dim, the room for copies of unaligned tensors leads both workspaces
+  // without overlapping itself or the kernels' own regions.
   for (int D = 16; D <= 128; D += 16) {
     for (int mode : {FC_MODE_FAST, FC_MODE_EXACT}) {
       fc_attn_desc e = desc(D, 4, 2, 333, 3, mode);
@@ -94,8 +94,8 @@ static void validation() {
       CHECK(fc::fwd_workspace(p).total == pf.inner);
       const fc::BwdWorkspace bw = fc::bwd_workspace(p);
       CHECK(bw.delta == pb.inner && bw.total > pb.inner);
-      const fc::Problem k = fc::kernel_problem(p, true);
-      CHECK(!k.grad_bf16 && !k.accumulate && k.D == D && k.Dk == p.Dk && fc::bwd_workspace(k).total == bw.total);
+      // (a float32 gradient of the caller's width fits its place)
+      CHECK(pb.dK - pb.dQ >= 3ull * 333 * 4 * D * 4 && pb.dV - pb.dK >= 3ull * 333 * 2 * D * 4);
     }
   }
   fc_attn_desc x = desc(64, 4, 2, 100, 3, FC_MODE_EXACT);

@@ -55,11 +55,11 @@ def test_abi_version_and_head_dims():
 
 @pytest.mark.parametrize("D,Dk", [(48, 64), (80, 128), (96, 128), (112, 128)])
 @pytest.mark.parametrize("mode", [L.FC_MODE_FAST, L.FC_MODE_EXACT])
-def test_padded_head_dims_need_their_copies_in_the_workspace(D, Dk, mode):
-    """Head dims between the compiled widths run on zero-padded copies: the
-    forward's workspace grows by Q, K, V and O of width Dk (and becomes
-    required), the backward's by those plus dO and float32 dQ, dK, dV; a
-    compiled width asks for none of it."""
+def test_padded_head_dims_need_their_room_in_the_workspace(D, Dk, mode):
+    """Head dims whose tiles are wider ask for room for copies (which tensors off
+    a 16-byte boundary go through): the forward's workspace grows by Q, K, V and
+    O of width Dk (and becomes required), the backward's by those plus dO and
+    float32 dQ, dK, dV; the other widths ask for none of it."""
     t = L.FC_BF16 if mode == L.FC_MODE_FAST else L.FC_F32
     B, T, H, Hkv = 2, 64, 4, 2
     e = 2 if t == L.FC_BF16 else 4

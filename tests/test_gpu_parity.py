@@ -125,16 +125,15 @@ PADDED_CASES = [
 @pytest.mark.parametrize("case", PADDED_CASES, ids=lambda c: "-".join(map(str, c)))
 def test_padded_head_dims(gpu, case):
     """D in {48, 80, 96, 112} (the reference's tensor-core path takes any
-    D % 16 == 0 up to 128, ext/FemtoChatCUDAExt.jl:214-223): the library runs
-    them zero-padded to 64 or 128 with the scale of the real D."""
+    D % 16 == 0 up to 128, ext/FemtoChatCUDAExt.jl:214-223): LDS tiles of 64 or
+    128 columns, of which the caller's rows fill D."""
     mode, B, T, H, Hkv, D, window = case
     _check_case(gpu, mode, B, T, H, Hkv, D, window, seed=zlib.crc32(repr(case).encode()) % 1000)
 
 
 def test_padded_head_dims_storage_positions_accumulate(gpu):
-    """The padded path with fp32 O/dO/gradients in fast mode, with a document
-    mask, and adding into existing bf16 gradients (the padded kernels write
-    float32 gradients that are added to the caller's values and rounded once)."""
+    """These widths with fp32 O/dO/gradients in fast mode, with a document mask,
+    and adding into existing bf16 gradients (float32 sums, rounded once)."""
     pos = W.document_positions(180, 2, seed=96, mean=40, sigma=1.0, cap=120)
     _check_case(gpu, "fast", 2, 180, 4, 2, 96, (-1, 0), positions=pos, out_dtype=torch.float32,
                 grad_dtype=torch.float32, dout_dtype=torch.float32, seed=96)

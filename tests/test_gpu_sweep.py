@@ -5,8 +5,7 @@ of src/kernels.jl:30-96,131-379).
 The hand-picked cases in test_gpu_parity.py name each code path; this sweep
 draws the parameters instead, so combinations nobody picked also run: T on
 and around the tile edges (32, 64, 128 queries or keys) and in between, every
-head dim the library takes (D % 16 == 0 up to 128, the non-compiled widths
-through zero-padded copies), GQA ratios 1-4, causal, sliding, two-sided and
+head dim the library takes (D % 16 == 0 up to 128), GQA ratios 1-4, causal, sliding, two-sided and
 right-of-query windows (some leaving rows empty), packed documents, and fp32
 O/dO/gradients in fast mode.  The list is drawn once from a fixed seed, so
 every run checks the same cases and a failure names its parameters.
