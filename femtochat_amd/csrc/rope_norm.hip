@@ -23,13 +23,14 @@
 // eight rotation pairs (elements j..j+7 and j+d..j+d+7, one 16-byte bf16
 // load per half), so the rotation needs no cross-lane exchange and the sum
 // of squares is a butterfly over D/16 lanes.  Memory-bound: a vector is read
-// and written once; the tables stay in L2.  Results are stored non-temporally:
-// the kernel never reads them and the stores leave the inputs in the caches.
-// 16 x 2048 tokens, D128, H10, bf16, packed positions: forward 67 -> 61 us of
-// Q and K together, backward 74 -> 65 (5.8 TB/s of its bytes); with H = Hkv =
-// 12 the backward 115 -> 102; 777 tokens, forward 18 -> 13.  Non-temporal loads
-// as well measured slower (the gradient at D64 32 -> 39: its inputs fit the
-// last-level cache).
+// and written once; the tables stay in L2.  16 x 2048 tokens, H10 D128, bf16,
+// inputs from memory: forward 39 us, backward 50 (4.3 and 5.0 TB/s).  Results are
+// stored plainly, as attention or a matrix product reads them next: with
+// non-temporal stores the calls alone took 37 and 47 us, but with a copy of the
+// result after them 72 and 82 (65 and 83 plain), at D64 39 and 46 (36 and 42), and
+// for 16 x 2048, H20 D16 in float32 30 and 45 alone (24 and 29), 49 and 64 with the
+// copy (38 and 43): a row's 64 bytes leave in separate writes.  Non-temporal loads
+// measured slower too (the gradient at D64 32 -> 39).
 #include <type_traits>
 
 #include "attn_launch.hpp"
@@ -105,8 +106,8 @@ struct Eight<float> {
       a += *reinterpret_cast<const f32x4*>(p);
       b += *reinterpret_cast<const f32x4*>(p + 4);
     }
-    __builtin_nontemporal_store(a, reinterpret_cast<f32x4*>(p));
-    __builtin_nontemporal_store(b, reinterpret_cast<f32x4*>(p + 4));
+    *reinterpret_cast<f32x4*>(p) = a;
+    *reinterpret_cast<f32x4*>(p + 4) = b;
   }
 };
 
@@ -132,7 +133,7 @@ struct Eight<bf16> {
 #pragma unroll
       for (int i = 0; i < 8; ++i) w[i] += static_cast<float>(o[i]);
     }
-    __builtin_nontemporal_store(__builtin_convertvector(w, bf16x8), reinterpret_cast<bf16x8*>(p));
+    *reinterpret_cast<bf16x8*>(p) = __builtin_convertvector(w, bf16x8);
   }
 };
 
