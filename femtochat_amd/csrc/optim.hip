@@ -645,16 +645,28 @@ void polar_launch(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus
   else tr ? go(polar_gemm_kernel<true, 2, false, kSym>) : go(polar_gemm_kernel<false, 2, false, kSym>);
 }
 
+// 128 x 128 tiles of one stack's symmetric products.
+int64_t polar_tiles(int lo, int batch) {
+  const int64_t tm = (lo + kGemmTile - 1) / kGemmTile;
+  return tm * tm * batch;
+}
+
 // A symmetric result (M = N) takes the lower tiles only where that saves a
-// round of workgroups, or where the full grid would leave CUs idle (what the
-// rest leaves free, the other stacks of a grouped call use).  16 matrices of 640 x
-// 640: 323 -> 232 us; for 32 of 512 x 512 both grids take two rounds and the
-// transposed stores made the call 282 us instead of 268, so they stay whole.
-void polar_gemm(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus, bool symmetric = false) {
-  const int64_t tm = (a.M + kGemmTile - 1) / kGemmTile, full = tm * ((a.N + kGemmTile - 1) / kGemmTile) * batch;
+// round of workgroups, or where the full grid would leave CUs idle while the
+// stacks of a grouped call have more than two tiles per CU between them (tiles),
+// which take what the rest leaves free.  16 matrices of 640 x 640: 323 -> 232 us; for
+// 32 of 512 x 512 both grids take two rounds and the transposed stores made the
+// call 282 us instead of 268, so they stay whole.  Grouped, 4 k matrices of n x n
+// and k of n x 4n and 4n x n, whole / lower, us: n 640 k 8 865 / 802, n 512 k 8 541 /
+// 517, n 640 k 4 545 / 529, n 320 k 12 420 / 410 (648 to 2400 tiles); n 512 k 4
+// 370 / 375 (384), n 320 k 8 264 / 285, n 384 k 1 196 / 239, n 128 k 4 152 / 177; one
+// stack of 4 x 256 x 256 80 / 86.
+void polar_gemm(bool tr, const PolarGemm& a, int batch, hipStream_t s, int cus, int64_t tiles = 0) {
+  const int64_t full = polar_tiles(a.M, batch), tm = (a.M + kGemmTile - 1) / kGemmTile;
   const int64_t lower = tm * (tm + 1) / 2 * batch;
   auto rounds = [&](int64_t grid) { return (grid + cus - 1) / cus; };
-  if (symmetric && (full < (int64_t)cus || rounds(lower) < rounds(full))) polar_launch<true>(tr, a, batch, s, cus);
+  const bool symmetric = tiles > 0 && (rounds(lower) < rounds(full) || (full < (int64_t)cus && tiles > 2 * (int64_t)cus));
+  if (symmetric) polar_launch<true>(tr, a, batch, s, cus);
   else polar_launch<false>(tr, a, batch, s, cus);
 }
 
@@ -921,9 +933,9 @@ static fc_status polar_args(const fc_polar_desc* d, const float* G, const void* 
 }
 
 // Polar Express of one stack on stream s with the rocBLAS handle h (held by
-// the caller under g_blas_mutex).
+// the caller under g_blas_mutex); tiles: polar_tiles of all stacks of the call.
 static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, size_t workspace_bytes, hipStream_t s,
-                           rocblas_handle h) {
+                           rocblas_handle h, int64_t tiles) {
   fc_status st = polar_args(d, G, workspace, workspace_bytes);
   if (st != FC_OK) return st;
   const PolarLayout L = polar_layout(*d);
@@ -942,7 +954,7 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
   hipLaunchKernelGGL(norm_partial_kernel, dim3(kNormParts, k), dim3(256), 0, s, (int64_t)m * n, G, partial);
   if ((st = launched("polar norm")) != FC_OK) return st;
   // X (lo x hi) = G / scale, or G^T / scale, rounded to the compute type
-  const dim3 tiles((lo + 31) / 32, (hi + 31) / 32, k), back((hi + 31) / 32, (lo + 31) / 32, k);
+  const dim3 in((lo + 31) / 32, (hi + 31) / 32, k), back((hi + 31) / 32, (lo + 31) / 32, k);
   const int64_t msize = (int64_t)m * n;
   const bool flat = !transposed && msize % 4 == 0 && aligned16(G) && aligned16(X);
   const dim3 flat_grid((unsigned)std::min<int64_t>((msize / 4 + 255) / 256, std::max<int64_t>(1, 2048 / k)), k);
@@ -953,11 +965,11 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
   } else if (half && transposed && lo % 64 == 0 && hi % 64 == 0 && aligned16(G) && aligned16(X)) {
     hipLaunchKernelGGL(copy_in_transposed_kernel, dim3(lo / 64, hi / 64, k), dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
   } else if (half) {
-    if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, bf16>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
-    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, bf16>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
+    if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, bf16>), in, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
+    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, bf16>), in, dim3(256), 0, s, lo, hi, G, reinterpret_cast<bf16*>(X), partial, scale);
   } else {
-    if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, float>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<float*>(X), partial, scale);
-    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, float>), tiles, dim3(256), 0, s, lo, hi, G, reinterpret_cast<float*>(X), partial, scale);
+    if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, float>), in, dim3(256), 0, s, lo, hi, G, reinterpret_cast<float*>(X), partial, scale);
+    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, float>), in, dim3(256), 0, s, lo, hi, G, reinterpret_cast<float*>(X), partial, scale);
   }
   if ((st = launched("polar copy in")) != FC_OK) return st;
 
@@ -971,10 +983,10 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
       bf16* a = reinterpret_cast<bf16*>(A);
       bf16* b = reinterpret_cast<bf16*>(B);
       // A = X X^T: P(i, p) = X(i, p), Q(p, j) = X(j, p), both contiguous in i, j
-      polar_gemm(true, PolarGemm{x, x, none, a, sx, sx, sa, lo, lo, lo, lo, hi, 1.0f, 0.0f}, k, s, cus, true);
+      polar_gemm(true, PolarGemm{x, x, none, a, sx, sx, sa, lo, lo, lo, lo, hi, 1.0f, 0.0f}, k, s, cus, tiles);
       // B = c A A + b A: Q(q, j) = A(q, j), contiguous in q; A is symmetric
       // (X X^T), so P(i, q) is read as A(q, i), also contiguous in q
-      polar_gemm(false, PolarGemm{a, a, a, b, sa, sa, sa, lo, lo, lo, lo, lo, c[2], c[1]}, k, s, cus, true);
+      polar_gemm(false, PolarGemm{a, a, a, b, sa, sa, sa, lo, lo, lo, lo, lo, c[2], c[1]}, k, s, cus, tiles);
       // Y = B X + a X: Q(q, p) = X(q, p), contiguous in q; P(i, q) read as
       // B(q, i) (B = c A A + b A is symmetric)
       // (the last step writes G itself: the bf16 iterate widened to fp32, as
@@ -1006,10 +1018,10 @@ static fc_status polar_run(const fc_polar_desc* d, float* G, void* workspace, si
   // G = X, or X^T (widened to fp32)
   if (half) {
     if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, bf16, float>), back, dim3(256), 0, s, hi, lo, reinterpret_cast<const bf16*>(X), G, nullptr, nullptr);
-    else hipLaunchKernelGGL((copy_scaled_kernel<false, bf16, float>), tiles, dim3(256), 0, s, lo, hi, reinterpret_cast<const bf16*>(X), G, nullptr, nullptr);
+    else hipLaunchKernelGGL((copy_scaled_kernel<false, bf16, float>), in, dim3(256), 0, s, lo, hi, reinterpret_cast<const bf16*>(X), G, nullptr, nullptr);
   } else {
     if (transposed) hipLaunchKernelGGL((copy_scaled_kernel<true, float, float>), back, dim3(256), 0, s, hi, lo, reinterpret_cast<const float*>(X), G, nullptr, nullptr);
-    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, float>), tiles, dim3(256), 0, s, lo, hi, reinterpret_cast<const float*>(X), G, nullptr, nullptr);
+    else hipLaunchKernelGGL((copy_scaled_kernel<false, float, float>), in, dim3(256), 0, s, lo, hi, reinterpret_cast<const float*>(X), G, nullptr, nullptr);
   }
   return launched("polar copy out");
 }
@@ -1020,7 +1032,9 @@ fc_status fc_polar_express(const fc_polar_desc* d, float* G, void* workspace, si
   std::lock_guard<std::mutex> lock(g_blas_mutex);
   rocblas_handle h = blas_handle(dev);
   if (h == nullptr) return failf(FC_ERR_HIP, "polar express: rocblas_create_handle failed");
-  return polar_run(d, G, workspace, workspace_bytes, static_cast<hipStream_t>(stream), h);
+  fc_status st = polar_args(d, G, workspace, workspace_bytes);
+  if (st != FC_OK) return st;
+  return polar_run(d, G, workspace, workspace_bytes, static_cast<hipStream_t>(stream), h, polar_tiles(std::min(d->m, d->n), d->count));
 }
 
 fc_status fc_polar_express_grouped(int32_t count, const fc_polar_desc* descs, float* const* G, void* const* workspaces,
@@ -1029,9 +1043,11 @@ fc_status fc_polar_express_grouped(int32_t count, const fc_polar_desc* descs, fl
     return failf(FC_ERR_INVALID_ARGUMENT, "polar express grouped: count must be positive and the arrays non-null");
   // Every stack is checked before anything is launched, so a rejected call
   // leaves no work behind on the helper streams.
+  int64_t tiles = 0;
   for (int i = 0; i < count; ++i) {
     const fc_status st = polar_args(&descs[i], G[i], workspaces[i], workspace_bytes[i]);
     if (st != FC_OK) return st;
+    tiles += polar_tiles(std::min(descs[i].m, descs[i].n), descs[i].count);
   }
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return failf(FC_ERR_HIP, "polar express grouped: hipGetDevice failed");
@@ -1047,7 +1063,7 @@ fc_status fc_polar_express_grouped(int32_t count, const fc_polar_desc* descs, fl
   fc_status first = FC_OK;
   for (int i = 0; i < count && first == FC_OK; ++i) {
     const int j = i % kHelpers;
-    first = polar_run(&descs[i], G[i], workspaces[i], workspace_bytes[i], f->stream[j], f->blas[j]);
+    first = polar_run(&descs[i], G[i], workspaces[i], workspace_bytes[i], f->stream[j], f->blas[j], tiles);
   }
   // join, also after a failed launch: the caller's stream waits for every
   // helper stream, so nothing enqueued there outlives the caller's view

@@ -239,6 +239,21 @@ def test_grouped_bf16_many_stacks_equals_separate_calls(gpu):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n,layers", [(512, 8), (320, 12), (192, 60)])
+def test_grouped_bf16_lower_tiles_equal_separate_calls(gpu, n, layers):
+    """A model's matrix groups with more than two tiles per CU between them: stacks
+    that would leave CUs idle take their symmetric products by the lower tiles,
+    which alone they take whole; the bits are the same."""
+    g = torch.Generator(device=gpu).manual_seed(n)
+    stacks = [torch.randn(k, a, b, generator=g, device=gpu) for k, a, b in
+              ((4 * layers, n, n), (layers, 4 * n, n), (layers, n, 4 * n))]
+    separate = [polar_express(G, compute_type=torch.bfloat16) for G in stacks]
+    polar_express_grouped_(stacks, compute_type=torch.bfloat16)
+    torch.cuda.synchronize()
+    for a, b in zip(separate, stacks):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("compute_type", [torch.float32, torch.bfloat16])
 def test_grouped_equals_separate_calls(gpu, compute_type):
     # the stacks run concurrently on helper streams, each with the same GEMMs as
