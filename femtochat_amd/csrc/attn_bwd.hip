@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kOrderThreads) void attn_order_kernel(OrderArgs a) 
 // the keys, whose Q and dO are split once per workgroup into swizzled LDS.
 // At one wave per SIMD (D = 128) the LDS reads bound it next to the products:
 // a wave reads 112 KB of parts per tile for 192 products.  8 x 2048 tokens,
-// causal, H6 D128: 676 us (fp32 MFMA 1142-1183), H12 D64: 535 (1278).
+// causal, H6 D128: 677 us (fp32 MFMA 1103), H12 D64: 558 (1190).
 constexpr int kExactBK = 128;  // keys per workgroup
 constexpr int kExactBT = 32;   // rows per staged tile (queries here, keys in dQ)
 
@@ -476,8 +476,8 @@ __global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void attn_bwd_dkdv_exact
 // with Q and dO resident in parts; S^T and dP^T are recomputed with the query
 // as the lane index, so dS^T is directly the B operand of dQ^T += K^T dS^T.
 // K and V tiles of 32 keys are split once per workgroup into double-buffered
-// LDS, a tile ahead.  8 x 2048 tokens, causal, H6 D128: 500 us (fp32 MFMA
-// 782-798), H12 D64: 394 (769).  Loading a further tile ahead, alternating
+// LDS, a tile ahead.  8 x 2048 tokens, causal, H6 D128: 497 us (fp32 MFMA
+// 782), H12 D64: 398 (756).  Loading a further tile ahead, alternating
 // products of two sums and fixed orders of reads and products measured within
 // 3% (slower at D = 64, where they spill).
 template <int D>

@@ -24,8 +24,10 @@
 //    tile skip its products.
 //
 // Bound by the matrix cores and, next to them, by LDS (48 KB of parts read per
-// wave and tile for 96 products): 8 x 2048 tokens, causal, H6 D128 in 303 us
-// (1.02 PFLOP/s of bf16 products; 475 us with fp32 MFMA), H12 D64 in 296 (523).
+// wave and tile for 96 products): 8 x 2048 tokens, causal, H6 D128 in 315 us
+// (0.98 PFLOP/s of bf16 products; 474 us with fp32 MFMA), H12 D64 in 304 (525).
+// At D = 112 and 128 the kernel spills 79 and 28 registers (five to seven scratch
+// accesses per tile; D = 112 240 us for 4 x 2048, H6, 227 with 13 spilled).
 #include "attn_exact.hpp"
 #include "attn_launch.hpp"
 
