@@ -25,12 +25,14 @@
 // of squares is a butterfly over D/16 lanes.  Memory-bound: a vector is read
 // and written once; the tables stay in L2.  16 x 2048 tokens, H10 D128, bf16,
 // inputs from memory: forward 39 us, backward 50 (4.3 and 5.0 TB/s).  Results are
-// stored plainly, as attention or a matrix product reads them next: with
-// non-temporal stores the calls alone took 37 and 47 us, but with a copy of the
-// result after them 72 and 82 (65 and 83 plain), at D64 39 and 46 (36 and 42), and
-// for 16 x 2048, H20 D16 in float32 30 and 45 alone (24 and 29), 49 and 64 with the
-// copy (38 and 43): a row's 64 bytes leave in separate writes.  Non-temporal loads
-// measured slower too (the gradient at D64 32 -> 39).
+// stored plainly, as attention or a matrix product reads them next.  Non-temporal
+// stores make the bf16 calls alone faster (37 and 47 us) and what follows slower:
+// attention's backward, the prologue's and the projections' products took 451 us
+// for 16 x 2048, H8 D64 (437 plain), 138 for 1 x 2048, H8 D128 (133), 53.1 for 512
+// tokens (50.0), and at H10, Hkv5, D128 as long (825 and 821); in float32 the calls
+// alone were slower too (16 x 2048, H20 D16 30 and 45 us, 24 and 29 plain: a row's 64
+// bytes leave in separate writes).  Non-temporal loads measured slower as well
+// (the gradient at D64 32 -> 39).
 #include <type_traits>
 
 #include "attn_launch.hpp"
